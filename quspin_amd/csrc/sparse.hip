@@ -78,11 +78,88 @@ static void launch_csr_g(const CsrArgs& A, int G, hipStream_t st) {
   }
 }
 
+// Lanes per row of k_csr_mm for rows of n column runs: the width that leaves
+// the fewest idle lanes over the row's column tiles, a further tile counted
+// as four lanes, the widest of equals, at least 8 lanes unless the row is
+// shorter.  Narrower tiles read segments below 64 bytes and lose (XXZ L = 22,
+// 16 float64 vectors one column per lane: 4 lanes 285 us, 8 lanes 170, 16
+// lanes 165; 12 complex128 vectors: 4 lanes 254 us, 8 lanes 223, 16 lanes 187).
+static int mm_group(int64_t n) {
+  int best = 64;
+  int64_t cost = INT64_MAX;
+  for (int g = 64; g >= 8; g >>= 1) {
+    const int64_t c = (n + g - 1) / g * (g + 4);
+    if (c < cost) { cost = c; best = g; }
+  }
+  while (best > 2 && best / 2 >= n) best >>= 1;
+  return best;
+}
+
+// Rows per lane group: two with 16 lanes or more (one round of staged entries
+// then serves up to 32 rows: 16 float64 vectors at L = 22 184 -> 167 us), one
+// below, where a block covers 32 rows or more already (8 lanes: 89 against
+// 83 us, but 53 against 57 with 4).
+constexpr int mm_rpg(int G) { return G >= 16 ? 2 : 1; }
+
+static int64_t mm_blocks(int64_t Ns, int G) {
+  const int64_t nb = qsx_grid(Ns, 256 / G * mm_rpg(G));
+  return nb < 1 ? 1 : nb > EPI_MAX_BLOCKS ? EPI_MAX_BLOCKS : nb;
+}
+
+template <typename MT, typename VT, int CW, bool EPI>
+static int64_t launch_mm_g(const CsrArgs& A, hipStream_t st) {
+  const int G = mm_group(A.nvec / CW);
+  const int64_t nb = mm_blocks(A.Ns, G);
+  const dim3 grid((unsigned)nb), blk(256);
+  switch (G) {
+    case 2: hipLaunchKernelGGL((k_csr_mm<MT, VT, 2, mm_rpg(2), CW, EPI>), grid, blk, 0, st, A); break;
+    case 4: hipLaunchKernelGGL((k_csr_mm<MT, VT, 4, mm_rpg(4), CW, EPI>), grid, blk, 0, st, A); break;
+    case 8: hipLaunchKernelGGL((k_csr_mm<MT, VT, 8, mm_rpg(8), CW, EPI>), grid, blk, 0, st, A); break;
+    case 16: hipLaunchKernelGGL((k_csr_mm<MT, VT, 16, mm_rpg(16), CW, EPI>), grid, blk, 0, st, A); break;
+    case 32: hipLaunchKernelGGL((k_csr_mm<MT, VT, 32, mm_rpg(32), CW, EPI>), grid, blk, 0, st, A); break;
+    default: hipLaunchKernelGGL((k_csr_mm<MT, VT, 64, mm_rpg(64), CW, EPI>), grid, blk, 0, st, A); break;
+  }
+  return nb;
+}
+
+// Two columns per lane where that makes a 16-byte element run of every row
+// (8-byte elements, an even number of vectors, x on a 16-byte boundary): half
+// the lanes and gathers (XXZ L = 22, 16 float64 vectors 165 -> 122 us, 8
+// vectors 89 -> 67 us; 2 vectors 43 -> 46 us).
+template <typename MT, typename VT, bool EPI>
+static int64_t launch_mm_w(const CsrArgs& A, hipStream_t st) {
+  if constexpr (sizeof(VT) == 8) {
+    if (A.nvec % 2 == 0 && (uintptr_t)A.x % 16 == 0) return launch_mm_g<MT, VT, 2, EPI>(A, st);
+  }
+  return launch_mm_g<MT, VT, 1, EPI>(A, st);
+}
+
+// Several vectors go to k_csr_mm (one dtype for terms and accumulator, columns
+// below 2^31); 0: the caller takes k_csr_spmv, else the blocks launched.
+template <bool EPI>
+static int64_t launch_mm(const CsrArgs& A, int mdt, int vdt, int fdt, hipStream_t st) {
+  if (A.nvec < 2 || fdt != vdt || A.Ns >= INT32_MAX) return 0;
+  if (vdt == QSX_F32 && mdt == QSX_F32) return launch_mm_w<float, float, EPI>(A, st);
+  if (vdt == QSX_F64 && mdt == QSX_F64) return launch_mm_w<double, double, EPI>(A, st);
+  if (vdt == QSX_C64 && mdt == QSX_F32) return launch_mm_w<float, float2, EPI>(A, st);
+  if (vdt == QSX_C64 && mdt == QSX_C64) return launch_mm_w<float2, float2, EPI>(A, st);
+  if (vdt == QSX_C128 && mdt == QSX_F64) return launch_mm_w<double, double2, EPI>(A, st);
+  if (vdt == QSX_C128 && mdt == QSX_C128) return launch_mm_w<double2, double2, EPI>(A, st);
+  return 0;
+}
+
 // fdt: dtype of the expm accumulator F (-1: the vector dtype); FP64 F with
 // FP32 vectors is the mixed-precision form.
 template <bool EPI>
 static int launch_csr(const CsrArgs& A, int mdt, int vdt, int G, hipStream_t st, int fdt = -1) {
   if (fdt < 0) fdt = vdt;
+  int64_t blocks = launch_mm<EPI>(A, mdt, vdt, fdt, st);
+  if (blocks > 0) {
+    QSX_LAUNCH_CHECK();
+    if constexpr (EPI) return qsx_part_reduce_launch(A, blocks, st);
+    return QSX_OK;
+  }
+  blocks = csr_blocks(A.Ns, G, EPI);
   // matrix dtype must be the vector dtype or its real counterpart
   if (fdt == vdt) {
     if (vdt == QSX_F32 && mdt == QSX_F32) launch_csr_g<float, float, EPI>(A, G, st);
@@ -102,7 +179,7 @@ static int launch_csr(const CsrArgs& A, int mdt, int vdt, int G, hipStream_t st,
     return QSX_ERR_ARG;
   }
   QSX_LAUNCH_CHECK();
-  if constexpr (EPI) return qsx_part_reduce_launch(A, csr_blocks(A.Ns, G, true), st);
+  if constexpr (EPI) return qsx_part_reduce_launch(A, blocks, st);
   return QSX_OK;
 }
 

@@ -252,3 +252,114 @@ __global__ void __launch_bounds__(256) k_csr_spmv(CsrArgs A) {
   }
   if constexpr (EPI) block_norm_partials(A, rowB, rowF);
 }
+
+// Several vectors, (Ns, nvec) row-major: G lanes per row, lane l of a row
+// takes the columns l, l + G, ... of its output row, so a gathered vector row
+// is read in segments of G consecutive elements.  The block's 256 / G rows
+// are consecutive and so are their matrix entries: these are staged in LDS
+// with coalesced loads, CSR_MM_CAP at a time, and read back from there as
+// broadcasts; a lane keeps U gathers in flight.  FP64 accumulation.
+//
+// Bound by the gathers: every entry reads one vector row (nvec elements)
+// through L2, and by their latency where nvec is small.  k_csr_spmv, which
+// several vectors used before, walks the whole row once per vector, each lane
+// of a gather on a line of its own and the matrix re-read per vector: a Taylor
+// term of 12 complex128 vectors on the XXZ L = 18 matrix (48,620 rows) takes
+// 80 us there and 15 us here.
+constexpr int CSR_MM_CAP = 1024;  // staged entries
+
+template <typename VT, int CW>
+struct alignas(CW * sizeof(VT)) VecRun {
+  VT a[CW];
+};
+
+template <typename MT, typename VT, int G, int RPG, int CW, bool EPI>
+__global__ void __launch_bounds__(256) k_csr_mm(CsrArgs A) {
+  __shared__ int32_t s_col[CSR_MM_CAP];
+  __shared__ MT s_val[CSR_MM_CAP];
+  double2 a_t = A.a, mu_t = A.mu, xs = A.xdscale;
+  if constexpr (EPI) {
+    if (!expm_term_prologue(A, a_t, mu_t, xs)) return;
+  }
+  constexpr int RB = 256 / G;                        // rows side by side
+  constexpr int RT = RB * RPG;                       // rows per tile
+  constexpr int U = CW * sizeof(VT) >= 16 ? 4 : 8;
+  const int lane = threadIdx.x % G, rg = threadIdx.x / G;
+  const MT* __restrict__ val = (const MT*)A.data;
+  const VT* __restrict__ x = (const VT*)A.x;
+  const int64_t nv = A.nvec;
+  const int64_t ntile = (A.Ns + RT - 1) / RT;
+  const int64_t bxi = xcd_chunked(blockIdx.x, gridDim.x, gridDim.x >= 16384 ? 256 : 64);
+  double rowB = 0.0, rowF = 0.0;
+  for (int64_t tile = bxi; tile < ntile; tile += gridDim.x) {
+    const int64_t t0 = tile * RT, t1 = t0 + RT < A.Ns ? t0 + RT : A.Ns;
+    const int64_t b0 = ld_idx(A.indptr, A.idx64, t0), b1 = ld_idx(A.indptr, A.idx64, t1);
+    const bool one = b1 - b0 <= CSR_MM_CAP;          // the tile's entries fit one round
+    for (int i = 0; i < RPG && t0 + i * RB < A.Ns; ++i) {
+      const int64_t r0 = t0 + i * RB, row = r0 + rg;
+      const bool live = row < A.Ns;
+      const int64_t s0 = one ? b0 : ld_idx(A.indptr, A.idx64, r0);
+      const int64_t s1 = one ? b1 : ld_idx(A.indptr, A.idx64, r0 + RB < A.Ns ? r0 + RB : A.Ns);
+      const int64_t k0 = live ? ld_idx(A.indptr, A.idx64, row) : s1;
+      const int64_t k1 = live ? ld_idx(A.indptr, A.idx64, row + 1) : s1;
+      double curB = 0.0, curF = 0.0;
+      for (int64_t j0 = 0; j0 < nv; j0 += G * CW) {
+        const bool ok = live && j0 + lane * CW < nv;
+        const int64_t j = ok ? j0 + lane * CW : 0;
+        double sr[CW], si[CW];
+#pragma unroll
+        for (int q = 0; q < CW; ++q) sr[q] = si[q] = 0.0;
+        for (int64_t c0 = s0; c0 < s1; c0 += CSR_MM_CAP) {
+          const int n = (int)(s1 - c0 < CSR_MM_CAP ? s1 - c0 : CSR_MM_CAP);
+          if (one ? (i == 0 && j0 == 0) : (j0 == 0 || s1 - s0 > CSR_MM_CAP)) {
+            __syncthreads();  // every reader of the previous round is done
+            for (int q = threadIdx.x; q < n; q += 256) {
+              s_col[q] = (int32_t)ld_idx(A.indices, A.idx64, c0 + q);
+              s_val[q] = val[c0 + q];
+            }
+            __syncthreads();
+          }
+          const int e0 = (int)(k0 > c0 ? k0 - c0 : 0);
+          const int e1 = k1 - c0 < n ? (int)(k1 - c0) : n;  // may be <= e0: no entries of this row here
+          for (int e = e0; e < e1; e += U) {
+            VecRun<VT, CW> v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+              const int ee = e + u < e1 ? e + u : e;  // past the row's end: this step's first entry again
+              v[u] = *(const VecRun<VT, CW>*)(x + (int64_t)s_col[ee] * nv + j);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+              if (e + u < e1) {
+                const double2 m = MTr<MT>::ld(s_val + e + u);
+#pragma unroll
+                for (int q = 0; q < CW; ++q) {
+                  const double2 w = VTr<VT>::ld(&v[u].a[q]);
+                  if constexpr (VTr<VT>::cplx) {
+                    if constexpr (MTr<MT>::cplx) { sr[q] += m.x * w.x - m.y * w.y; si[q] += m.x * w.y + m.y * w.x; }
+                    else { sr[q] += m.x * w.x; si[q] += m.x * w.y; }
+                  } else {
+                    sr[q] += m.x * w.x;
+                  }
+                }
+              }
+            }
+          }
+        }
+        if (ok) {
+          const int64_t o = row * nv + j;
+#pragma unroll
+          for (int q = 0; q < CW; ++q)
+            spmv_out<VT, EPI, VT>(A, o + q, row, make_double2(sr[q], si[q]), VTr<VT>::ld(x + o + q), a_t, mu_t, xs,
+                                  curB, curF);
+        }
+      }
+      if constexpr (EPI) {
+        // the row's sums of |B| and |F| over its G lanes
+        rowB = fmax(rowB, grp_sum<G>(curB));
+        rowF = fmax(rowF, grp_sum<G>(curF));
+      }
+    }
+  }
+  if constexpr (EPI) block_norm_partials(A, rowB, rowF);
+}

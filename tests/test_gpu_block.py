@@ -1,0 +1,109 @@
+"""Products with several vectors at once: the assembled matrix and the
+matrix-free operator against the same product in 64-bit host arithmetic."""
+
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+pytestmark = pytest.mark.gpu
+
+EPS = {np.dtype(np.float32): 2.0 ** -24, np.dtype(np.complex64): 2.0 ** -24,
+       np.dtype(np.float64): 2.0 ** -53, np.dtype(np.complex128): 2.0 ** -53}
+
+
+def _random_csr(rng, n, lengths, cplx):
+    rows = np.repeat(np.arange(n), lengths)
+    cols = np.concatenate([rng.choice(n, size=m, replace=False) for m in lengths]) if rows.size else rows
+    vals = rng.normal(size=rows.size)
+    if cplx:
+        vals = vals + 1j * rng.normal(size=rows.size)
+    return sp.csr_matrix((vals, (rows, cols)), shape=(n, n))
+
+
+def _vectors(rng, n, nv, dtype):
+    x = rng.normal(size=(n, nv))
+    if np.dtype(dtype).kind == "c":
+        x = x + 1j * rng.normal(size=(n, nv))
+    return x.astype(dtype)
+
+
+def _bound(A, x, dtype):
+    """|computed - exact| <= (entries + 4) eps_64 |A| |x| from the FP64 sums,
+    plus one rounding of the stored result."""
+    m = int(np.diff(A.indptr).max()) if A.nnz else 0
+    mag = abs(A) @ np.abs(x.astype(np.complex128))
+    return 4 * (m + 4) * 2.0 ** -53 * mag + 2 * EPS[np.dtype(dtype)] * mag
+
+
+@pytest.mark.parametrize("mdt,vdt", [(np.float32, np.float32), (np.float64, np.float64), (np.float32, np.complex64),
+                                     (np.complex64, np.complex64), (np.float64, np.complex128),
+                                     (np.complex128, np.complex128)])
+@pytest.mark.parametrize("n,nv", [(1, 2), (31, 3), (129, 2), (257, 8), (300, 12), (64, 33), (70, 64), (65, 130)])
+def test_csr_block_product(mdt, vdt, n, nv):
+    from quspin_amd import _lib as L
+    from quspin_amd.operators._devop import DeviceCSR
+    rng = np.random.default_rng(n * 1000 + nv)
+    # empty rows, short rows and one full row
+    lengths = rng.integers(0, min(n, 20) + 1, size=n)
+    lengths[rng.integers(n)] = n
+    A = _random_csr(rng, n, lengths, np.dtype(mdt).kind == "c").astype(mdt)
+    A.sort_indices()
+    D = DeviceCSR.from_scipy(A, mdt)
+    x = _vectors(rng, n, nv, vdt)
+    y0 = _vectors(rng, n, nv, vdt)
+    a = 0.75 - (0.5j if np.dtype(vdt).kind == "c" else 0)
+    exact = a * (A.astype(np.complex128) @ x.astype(np.complex128))
+    bound = abs(a) * 4 * _bound(A, x, vdt) + 2 * EPS[np.dtype(vdt)] * np.abs(y0)
+    xd, yd = L.to_device(x), L.empty((n, nv), vdt)
+    D.apply(xd, yd, a=a)
+    assert np.all(np.abs(L.to_host(yd) - exact) <= bound)
+    yd = L.to_device(y0)
+    D.apply(xd, yd, a=a, beta=1)
+    assert np.all(np.abs(L.to_host(yd) - exact - y0) <= bound)
+
+
+def test_csr_block_long_rows_and_unaligned_vectors():
+    """Rows longer than one staged round, and vectors off the 16-byte boundary."""
+    from quspin_amd import _lib as L
+    from quspin_amd.operators._devop import DeviceCSR
+    rng = np.random.default_rng(5)
+    n, nv = 2600, 6
+    lengths = rng.integers(0, 4, size=n)
+    lengths[[3, 4, 1000, n - 1]] = [1024, 1025, 2600, 2049]
+    A = _random_csr(rng, n, lengths, False)
+    A.sort_indices()
+    D = DeviceCSR.from_scipy(A, np.float64)
+    x = _vectors(rng, n, nv, np.float64)
+    buf = L.empty(n * nv + 1, np.float64)
+    for off in (0, 1):
+        xd = buf[off:off + n * nv].view(n, nv)
+        xd.copy_(L.to_device(x))
+        yd = L.empty((n, nv), np.float64)
+        D.apply(xd, yd)
+        assert np.all(np.abs(L.to_host(yd) - A @ x) <= _bound(A, x, np.float64))
+
+
+@pytest.mark.parametrize("nv", [2, 5, 16])
+@pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
+def test_expm_block_equals_single_columns(nv, dtype):
+    """The Taylor loop on a block equals the loop on each column to rounding
+    (the block's truncation test takes row sums, so it may run longer)."""
+    from models import xxz_static
+    from quspin_amd import _lib as L
+    from quspin_amd.basis import spin_basis_general
+    from quspin_amd.operators import hamiltonian
+    from quspin_amd.tools.evolution import expm_multiply_parallel
+    size = 9
+    rng = np.random.default_rng(nv)
+    B = spin_basis_general(size, Nup=4, pauli=0)
+    real = np.float32 if np.dtype(dtype) == np.complex64 else np.float64
+    H = hamiltonian(xxz_static(size, h=rng.uniform(-1, 1, size)), [], basis=B, dtype=real, check_symm=False,
+                    check_herm=False, check_pcon=False)
+    E = expm_multiply_parallel(H, a=-0.7j, dtype=dtype)
+    X = _vectors(rng, B.Ns, nv, dtype)
+    got = L.to_host(E.dot(L.to_device(X)))
+    import scipy.linalg
+    exact = scipy.linalg.expm(-0.7j * H.toarray().astype(np.float64)) @ X.astype(np.complex128)
+    # the loop's truncation tolerance and one rounding per term, with a margin
+    tol = 40 * EPS[np.dtype(dtype)] * 2
+    assert np.abs(got - exact).max() <= tol * np.abs(X).max() * 4
