@@ -1186,12 +1186,16 @@ int qsx_hv_ctx_export(const qsx_hv_ctx* X, HvArgs* A, int* dtype, int* N, int* l
   return QSX_OK;
 }
 
-int qsx_hv_expm_term(void* ctx, const void* x, void* y, double2 coef, double2 shift, const int* skip,
-                     hipStream_t st) {
+static void expm_term_args(HvArgs& A, const HvTerm& T) {
+  A.v_in = T.x; A.v_out = T.y;
+  A.alpha_off = T.coef; A.alpha_diag = T.coef; A.shift = T.shift; A.beta = 0;
+  A.skip = T.skip;
+}
+
+int qsx_hv_expm_term(void* ctx, const HvTerm& T, hipStream_t st) {
   qsx_hv_ctx* X = (qsx_hv_ctx*)ctx;
   HvArgs A = X->A;
-  A.v_in = x; A.v_out = y;
-  A.alpha_off = coef; A.alpha_diag = coef; A.shift = shift; A.skip = skip; A.beta = 0;
+  expm_term_args(A, T);
   return hv_launch(X->c, X->L, A, X->transposed, X->conjugated, X->dtype, st);
 }
 
@@ -1199,13 +1203,13 @@ int qsx_hv_expm_term(void* ctx, const void* x, void* y, double2 coef, double2 sh
 // the term and of F into nB, nF) fused into the product.  Only the two-pass
 // split schedule fuses it; otherwise QSX_ERR_UNSUPPORTED is returned before
 // anything is launched, and the caller runs the separate epilogue.
-int qsx_hv_expm_term_epi(void* ctx, const void* x, void* y, double2 coef, double2 shift, const int* skip, void* F,
-                         double* nB, double* nF, hipStream_t st) {
+int qsx_hv_expm_term_epi(void* ctx, const HvTerm& T, void* F, double* nB, double* nF, hipStream_t st) {
   qsx_hv_ctx* X = (qsx_hv_ctx*)ctx;
   if (!X->split_z || X->A.sched != 11 || X->A.nvec != 1) return QSX_ERR_UNSUPPORTED;
   HvArgs A = X->A;
-  A.v_in = x; A.v_out = y;
-  A.alpha_off = coef; A.alpha_diag = coef; A.shift = shift; A.skip = skip; A.beta = 0;
+  expm_term_args(A, T);
+  A.done = T.skip;
+  A.chk_c1 = T.chk_c1; A.chk_c2 = T.chk_c2; A.chk_F = T.chk_F; A.tol = T.tol;
   A.epi_F = F; A.epi_nB = nB; A.epi_nF = nF;
   return hv_launch(X->c, X->L, A, X->transposed, X->conjugated, X->dtype, st);
 }

@@ -169,6 +169,14 @@ struct HvArgs {
   void* epi_F;
   double* epi_nB;
   double* epi_nF;
+  // truncation test of the previous term (c1 + c2 <= tol F; null: none), made
+  // by the row pass, which sets *done (the skip flag) for itself and the
+  // strip pass
+  int* done;
+  const double* chk_c1;
+  const double* chk_c2;
+  const double* chk_F;
+  double tol;
 };
 
 // Split-chain layout of one hard-core-boson particle sector of N <= 32 bits
@@ -1591,6 +1599,10 @@ __global__ void __launch_bounds__(NT) k_split2_rows(HvArgs A) {
   __shared__ int64_t sbk[SPLIT_MAX_K * 33];  // C(n, k) for n < K (the ranks of d)
   __shared__ double2 lut[SPLIT_MAX_LUT];
   if (A.skip && *A.skip) return;
+  if (A.chk_c1 && *A.chk_c1 + *A.chk_c2 <= A.tol * *A.chk_F) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *A.done = 1;
+    return;
+  }
   const SplitDev S = *A.split;
   const int u1 = S.rpair[2 * blockIdx.x], u2 = R > 1 ? S.rpair[2 * blockIdx.x + 1] : -1;
   const int nb = u2 >= 0 ? 2 : 1;

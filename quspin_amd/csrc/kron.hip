@@ -650,12 +650,15 @@ int qsx_evolve_steps_with(int64_t Ns, int64_t nvec, const double* xdiag, int nst
                           int (*term)(const CsrArgs&, const void*, int, int, hipStream_t), const void* term_ctx,
                           const StepOpKey& key, int use_graph, hipStream_t st);
 int qsx_part_reduce_launch(const CsrArgs& A, int64_t nblocks, hipStream_t st);
+bool qsx_norms_direct(int64_t nblocks);
 
 static int kron_term(const CsrArgs& A, const void* ctx, int vdt, int fdt, hipStream_t st) {
   const qsx_kron* K = (const qsx_kron*)ctx;
-  const int rc = launch_kron<true>(A, K, vdt, fdt, st);
+  CsrArgs B = A;
+  if (qsx_norms_direct(kron_blocks(K, vt_size(vdt)))) B.part = nullptr;
+  const int rc = launch_kron<true>(B, K, vdt, fdt, st);
   if (rc) return rc;
-  return qsx_part_reduce_launch(A, kron_blocks(K, vt_size(vdt)), st);
+  return qsx_part_reduce_launch(B, kron_blocks(K, vt_size(vdt)), st);
 }
 
 extern "C" int qsx_evolve_kron_steps(const qsx_kron* K, const double* xdiag, int nsteps, const void* es, int s_max,

@@ -45,6 +45,23 @@ int qsx_compile_term(const qsx_core* c, const char* opstr, const int32_t* indx, 
 struct qsx_hv_ctx;
 uint64_t qsx_hv_ctx_owner(const qsx_hv_ctx* X);
 
+
+// One Taylor term of a matrix-free expm: y = coef (Op + diagonal) x + shift x,
+// unless *skip is set or the previous term's truncation test passes (chk_c1
+// null: no test).
+struct HvTerm {
+  const void* x;
+  void* y;
+  double2 coef, shift;
+  int* skip;
+  const double* chk_c1;
+  const double* chk_c2;
+  const double* chk_F;
+  double tol;
+};
+int qsx_hv_expm_term(void* hv_ctx, const HvTerm& T, hipStream_t st);
+int qsx_hv_expm_term_epi(void* hv_ctx, const HvTerm& T, void* F, double* nB, double* nF, hipStream_t st);
+
 #define QSX_CHECK_HIP(expr)                                               \
   do {                                                                    \
     hipError_t _e = (expr);                                               \

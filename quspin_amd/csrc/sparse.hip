@@ -44,9 +44,20 @@ __global__ void __launch_bounds__(256) k_part_reduce(const double* __restrict__ 
   }
 }
 
+// Whether an expm launch of nblocks blocks puts its norms straight into the
+// slots (one atomic per block and norm) instead of a partials buffer that a
+// second launch reduces.  Small grids save the launch (XXZ L = 12 step, 4
+// blocks per term: 795 -> 601 us); grids of many rounds spread their atomics
+// over the launch (driven Hubbard L = 14, 11,610 blocks: 59.3 -> 58.3 ms).
+// In between the blocks end together and their atomics queue up behind one
+// address (12 vectors at L = 18, 1,520 blocks: 1.92 -> 2.08 ms), so those keep
+// partials.
+bool qsx_norms_direct(int64_t nblocks) { return nblocks <= 256 || nblocks >= 8192; }
+
 // Fold the per-block norm partials of one expm launch (nblocks blocks) into
 // its norm slots; used by every expm term kernel.
 int qsx_part_reduce_launch(const CsrArgs& A, int64_t nblocks, hipStream_t st) {
+  if (!A.part) return QSX_OK;
   hipLaunchKernelGGL(k_part_reduce, dim3(64), dim3(256), 0, st, A.part, nblocks, &A.ctl->done, A.normB, A.normF,
                      A.nsp);
   QSX_LAUNCH_CHECK();
@@ -107,9 +118,10 @@ static int64_t mm_blocks(int64_t Ns, int G) {
 }
 
 template <typename MT, typename VT, int CW, bool EPI>
-static int64_t launch_mm_g(const CsrArgs& A, hipStream_t st) {
+static int64_t launch_mm_g(CsrArgs& A, hipStream_t st) {
   const int G = mm_group(A.nvec / CW);
   const int64_t nb = mm_blocks(A.Ns, G);
+  if (qsx_norms_direct(nb)) A.part = nullptr;
   const dim3 grid((unsigned)nb), blk(256);
   switch (G) {
     case 2: hipLaunchKernelGGL((k_csr_mm<MT, VT, 2, mm_rpg(2), CW, EPI>), grid, blk, 0, st, A); break;
@@ -127,7 +139,7 @@ static int64_t launch_mm_g(const CsrArgs& A, hipStream_t st) {
 // the lanes and gathers (XXZ L = 22, 16 float64 vectors 165 -> 122 us, 8
 // vectors 89 -> 67 us; 2 vectors 43 -> 46 us).
 template <typename MT, typename VT, bool EPI>
-static int64_t launch_mm_w(const CsrArgs& A, hipStream_t st) {
+static int64_t launch_mm_w(CsrArgs& A, hipStream_t st) {
   if constexpr (sizeof(VT) == 8) {
     if (A.nvec % 2 == 0 && (uintptr_t)A.x % 16 == 0) return launch_mm_g<MT, VT, 2, EPI>(A, st);
   }
@@ -137,7 +149,7 @@ static int64_t launch_mm_w(const CsrArgs& A, hipStream_t st) {
 // Several vectors go to k_csr_mm (one dtype for terms and accumulator, columns
 // below 2^31); 0: the caller takes k_csr_spmv, else the blocks launched.
 template <bool EPI>
-static int64_t launch_mm(const CsrArgs& A, int mdt, int vdt, int fdt, hipStream_t st) {
+static int64_t launch_mm(CsrArgs& A, int mdt, int vdt, int fdt, hipStream_t st) {
   if (A.nvec < 2 || fdt != vdt || A.Ns >= INT32_MAX) return 0;
   if (vdt == QSX_F32 && mdt == QSX_F32) return launch_mm_w<float, float, EPI>(A, st);
   if (vdt == QSX_F64 && mdt == QSX_F64) return launch_mm_w<double, double, EPI>(A, st);
@@ -151,7 +163,7 @@ static int64_t launch_mm(const CsrArgs& A, int mdt, int vdt, int fdt, hipStream_
 // fdt: dtype of the expm accumulator F (-1: the vector dtype); FP64 F with
 // FP32 vectors is the mixed-precision form.
 template <bool EPI>
-static int launch_csr(const CsrArgs& A, int mdt, int vdt, int G, hipStream_t st, int fdt = -1) {
+static int launch_csr(CsrArgs A, int mdt, int vdt, int G, hipStream_t st, int fdt = -1) {
   if (fdt < 0) fdt = vdt;
   int64_t blocks = launch_mm<EPI>(A, mdt, vdt, fdt, st);
   if (blocks > 0) {
@@ -160,6 +172,7 @@ static int launch_csr(const CsrArgs& A, int mdt, int vdt, int G, hipStream_t st,
     return QSX_OK;
   }
   blocks = csr_blocks(A.Ns, G, EPI);
+  if (qsx_norms_direct(blocks)) A.part = nullptr;
   // matrix dtype must be the vector dtype or its real counterpart
   if (fdt == vdt) {
     if (vdt == QSX_F32 && mdt == QSX_F32) launch_csr_g<float, float, EPI>(A, G, st);
@@ -1116,11 +1129,6 @@ extern "C" int qsx_expm_multiply_csr_noalloc(const void* indptr, const void* ind
 }
 
 // Matrix-free Taylor loop: same recurrence with H.v from the fused kernel.
-int qsx_hv_expm_term(void* hv_ctx, const void* x, void* y, double2 coef, double2 shift, const int* skip,
-                     hipStream_t st);
-int qsx_hv_expm_term_epi(void* hv_ctx, const void* x, void* y, double2 coef, double2 shift, const int* skip,
-                         void* F, double* nB, double* nF, hipStream_t st);
-
 extern "C" int qsx_expm_multiply_mf(void* hv_ctx, int64_t Ns, int s, int m_star, double tol, double mu_re,
                                     double mu_im, double a_re, double a_im, void* v, void* work, int vec_dtype,
                                     int64_t nvec, void* stream) {
@@ -1147,24 +1155,32 @@ extern "C" int qsx_expm_multiply_mf(void* hv_ctx, int64_t Ns, int s, int m_star,
   QSX_LAUNCH_CHECK();
   for (int i = 0; i < s; ++i) {
     for (int j = 0; j < m_star; ++j) {
-      if (j >= 1) {
-        hipLaunchKernelGGL(k_expm_check, dim3(1), dim3(1), 0, st, ctl, normB + i * stride + j - 1,
-                           normB + i * stride + j, normF + i * stride + j);
-      }
+      HvTerm T;
+      T.x = Bb[j & 1];
+      T.y = Bb[(j + 1) & 1];
       const double cf = 1.0 / ((double)s * (double)(j + 1));
-      const double2 coef = make_double2(a_re * cf, a_im * cf);
+      T.coef = make_double2(a_re * cf, a_im * cf);
       // shift = -coef * mu
-      const double2 shift = make_double2(-(coef.x * mu_re - coef.y * mu_im), -(coef.x * mu_im + coef.y * mu_re));
+      T.shift = make_double2(-(T.coef.x * mu_re - T.coef.y * mu_im), -(T.coef.x * mu_im + T.coef.y * mu_re));
+      T.skip = &ctl->done;
+      T.tol = tol;
+      T.chk_c1 = j >= 1 ? normB + i * stride + j - 1 : nullptr;
+      T.chk_c2 = normB + i * stride + j;
+      T.chk_F = normF + i * stride + j;
       if (fuse) {
-        // the two-pass split product writes the term and updates F and the
-        // norms in its strip pass (no separate epilogue pass)
-        rc = qsx_hv_expm_term_epi(hv_ctx, Bb[j & 1], Bb[(j + 1) & 1], coef, shift, &ctl->done, v,
-                                  normB + i * stride + j + 1, normF + i * stride + j + 1, st);
+        // the two-pass split product makes the truncation test in its row
+        // pass, and writes the term and updates F and the norms in its strip
+        // pass (no separate launches for either)
+        rc = qsx_hv_expm_term_epi(hv_ctx, T, v, normB + i * stride + j + 1, normF + i * stride + j + 1, st);
         if (rc == QSX_OK) continue;
         if (rc != QSX_ERR_UNSUPPORTED) return rc;
         fuse = false;
       }
-      rc = qsx_hv_expm_term(hv_ctx, Bb[j & 1], Bb[(j + 1) & 1], coef, shift, &ctl->done, st);
+      if (j >= 1) {
+        hipLaunchKernelGGL(k_expm_check, dim3(1), dim3(1), 0, st, ctl, T.chk_c1, T.chk_c2, T.chk_F);
+        QSX_LAUNCH_CHECK();
+      }
+      rc = qsx_hv_expm_term(hv_ctx, T, st);
       if (rc) return rc;
       QSX_VT_SWITCH(vec_dtype, hipLaunchKernelGGL(k_expm_epi<VT>, dim3(rg), dim3(256), 0, st, (const VT*)Bb[(j + 1) & 1],
                                                   (VT*)v, Ns, nvec, ctl, normB + i * stride + j + 1,

@@ -44,14 +44,14 @@ __device__ __forceinline__ void atomic_max_nonneg(double* addr, double v) {
 __device__ __forceinline__ double cabs2(double2 z) { return sqrt(z.x * z.x + z.y * z.y); }
 
 // A norm slot is a group of nsp doubles: writers take the atomic max into
-// entry blockIdx % nsp (spreading the same-address atomics of large grids),
+// entry blockIdx mod nsp (a power of two; it spreads same-address atomics),
 // readers take the max over the group.
 __device__ __forceinline__ double slot_max(const double* p, int nsp) {
   double m = p[0];
   for (int i = 1; i < nsp; ++i) m = fmax(m, p[i]);
   return m;
 }
-__device__ __forceinline__ void slot_put(double* p, int nsp, double v) { atomic_max_nonneg(p + (blockIdx.x % nsp), v); }
+__device__ __forceinline__ void slot_put(double* p, int nsp, double v) { atomic_max_nonneg(p + (blockIdx.x & (nsp - 1)), v); }
 
 // Taylor-loop control block (one per expm call).
 struct ExpmCtl {
@@ -111,7 +111,7 @@ struct CsrArgs {
   const double* chk_c2;
   const double* chk_F;
   int nsp;              // doubles per norm slot (>= 1)
-  double* part;         // expm: per-block (max |B| row sum, max |F| row sum), reduced by k_part_reduce
+  double* part;         // expm: per-block (max |B| row sum, max |F| row sum), reduced by k_part_reduce (null: slots)
   // optional extra diagonal: A + xdscale * diag(xdiag) (xdscale from rec when set)
   const double* xdiag;
   double2 xdscale;
@@ -190,8 +190,9 @@ __device__ __forceinline__ void spmv_out(const CsrArgs& A, int64_t o, int64_t ro
   }
 }
 
-// Block max of the per-thread row-sum maxima into part[blockIdx] (two
-// doubles); k_part_reduce folds the partials of a launch into the slots.
+// Block max of the per-thread row-sum maxima: into part[blockIdx] (two
+// doubles; k_part_reduce folds a launch's partials into the slots), or
+// straight into the slots when there is no partials buffer (small grids).
 __device__ __forceinline__ void block_norm_partials(const CsrArgs& A, double mb, double mf) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
@@ -204,8 +205,13 @@ __device__ __forceinline__ void block_norm_partials(const CsrArgs& A, double mb,
   __syncthreads();
   if (threadIdx.x == 0) {
     for (int i = 1; i < (int)(blockDim.x >> 6); ++i) { mb = fmax(mb, sw[0][i]); mf = fmax(mf, sw[1][i]); }
-    A.part[2 * (int64_t)blockIdx.x] = mb;
-    A.part[2 * (int64_t)blockIdx.x + 1] = mf;
+    if (A.part) {
+      A.part[2 * (int64_t)blockIdx.x] = mb;
+      A.part[2 * (int64_t)blockIdx.x + 1] = mf;
+    } else {
+      slot_put(A.normB, A.nsp, mb);
+      slot_put(A.normF, A.nsp, mf);
+    }
   }
 }
 
