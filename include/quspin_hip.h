@@ -141,7 +141,8 @@ int qsx_hv(qsx_core* core, qsx_oplist* l, const void* basis, const void* n, int 
  * split-chain blocks, 8/9 = direct-rank chunks of 4/8 terms with predicated
  * gathers, 10 = batches of 14 terms with the table, 11 = split-chain layout
  * in two passes through a buffer the context allocates, 12 = as 10 with the
- * workgroups of each XCD on one contiguous run of rows), apply. */
+ * workgroups of each XCD on one contiguous run of rows, 13 = packed rows,
+ * after qsx_hv_ctx_set_packed), apply. */
 int qsx_hv_ctx_create(qsx_core* core, qsx_oplist* l, const void* basis, const void* n, int n_bytes, int64_t Ns,
                       const int64_t* begin, const int64_t* end, int N_p, int dtype, int64_t nvec, int transposed,
                       int conjugated, int diag_conj, const void* diag_arr, int diag_arr_cplx, qsx_hv_ctx** out);
@@ -154,6 +155,23 @@ void qsx_hv_ctx_destroy(qsx_hv_ctx* ctx);
 int qsx_hv_ctx_set_table(qsx_hv_ctx* ctx, const void* table, int entry_bytes, int idx_bits, const void* lut,
                          int lut_len);
 int qsx_hv_ctx_set_schedule(qsx_hv_ctx* ctx, int sched);
+/* Packed rows: the off-diagonal elements of the context's operator evaluated
+ * once, four bytes each (column and coefficient id) in slices of 64 rows.
+ * qsx_hv_pack_count (work: device, qsx_hv_pack_work_bytes(Ns) bytes) fills the
+ * slice offsets off (device int64[(Ns + 63) / 64 + 1]) and gives the number
+ * of entries, of coefficients and the column bits; qsx_hv_pack_fill, with the
+ * same off and work, writes the entries (device uint32) and the coefficients
+ * (device complex128).  Both synchronise the stream.  QSX_ERR_UNSUPPORTED:
+ * the operator has no such form (no off-diagonal terms, a list that does not
+ * commute with the group, or too many distinct coefficients).  The buffers
+ * serve every context of the same basis, list and flags; the caller keeps
+ * them alive while they are bound (ent NULL unbinds). */
+int64_t qsx_hv_pack_work_bytes(int64_t Ns);
+int qsx_hv_pack_count(const qsx_hv_ctx* ctx, int64_t* off, void* work, int64_t work_bytes, int64_t* entries,
+                      int* n_lut, int* idx_bits, void* stream);
+int qsx_hv_pack_fill(const qsx_hv_ctx* ctx, int64_t* off, void* work, void* ent, void* lut, void* stream);
+int qsx_hv_ctx_set_packed(qsx_hv_ctx* ctx, const int64_t* off, const void* ent, const void* lut, int n_lut,
+                          int idx_bits);
 /* Replace the context's diagonal (diagonal terms and extra diagonal) by a
  * precomputed per-row array (Ns doubles, or Ns (re, im) pairs when
  * diag_arr_cplx), as quantum_LinearOperator keeps `_diagonal`

@@ -373,6 +373,20 @@ class basis_general:
         self._dev["table"] = (tab, eb.value, ib.value, lut)
         return self._dev["table"]
 
+    def has_lookup_table(self):
+        """Whether ``lookup_table`` has been built (and is held)."""
+        return self._dev.get("table") is not None
+
+    def lookup_table_bytes(self):
+        """Size of ``lookup_table`` without building it; 0 when there is none."""
+        if not self._made_basis or not len(self._pers):
+            return 0
+        ent, eb, ib, nl = L._i64(), L._i32(), L._i32(), L._i64()
+        d = self._dev
+        rc = L.load().qsx_table_info(self._core.h, self._Ns, ptr(d["n"]), d["n_bytes"], L.C.byref(ent), L.C.byref(eb),
+                                     L.C.byref(ib), L.C.byref(nl))
+        return int(ent.value) * int(eb.value) if rc == 0 else 0
+
     def _dev_args(self):
         """Positional basis arguments of the C-ABI calls."""
         d = self._dev

@@ -238,6 +238,8 @@ static int dispatch_hv(const HvArgs& A, int dtype, int N, int nmaps, bool fm, in
   }
 }
 
+int qsx_packed_launch(const HvArgs& A, int dtype, hipStream_t st);  // packed.hip
+
 // Launch v_out = beta v_out + (a_diag D + shift) v_in + a_off Op v_in.  A
 // carries everything except the off-diagonal terms.  Symmetric lists (and
 // every transposed product) use the one-launch gather; otherwise the diagonal
@@ -248,6 +250,7 @@ static int hv_launch(const qsx_core* c, const qsx_oplist_full* L, HvArgs A, int 
   const int N = c->h.N, nm = c->h.nmaps;
   const bool fm = c->h.fermion != 0;
   const bool scatter = nm > 0 && !L->symmetric && !transposed && L->base.n_off > 0;
+  if (A.sched == 13 && A.pk_ent && A.n_diag == 0) return qsx_packed_launch(A, dtype, st);
   // binomial rows 0..N, rounded up to an even count (16-byte aligned LDS after them)
   A.n_sb = ((std::min(65, c->rank_h.N + 1) * 33) + 1) & ~1;
   if (!scatter) {
@@ -1018,9 +1021,14 @@ extern "C" int qsx_hv_ctx_set_table(qsx_hv_ctx* X, const void* table, int entry_
 // 11: the split-chain layout in two passes, a row pass over the lower-half
 // terms into a buffer of Ns elements owned by the context, then a
 // column-strip pass over the upper-half and crossing terms (sectors as 7).
-// Single vector; several vectors always use one lane per row.
+// Single vector; several vectors use one lane per row with all of these.
+// 13: packed rows, for one vector or several, after qsx_hv_ctx_set_packed.
 extern "C" int qsx_hv_ctx_set_schedule(qsx_hv_ctx* X, int sched) {
-  if (!X || sched < 0 || sched > 12) { qsx_set_error("qsx_hv_ctx_set_schedule: bad arguments"); return QSX_ERR_ARG; }
+  if (X && sched == 13 && (!X->A.pk_ent || X->A.n_diag > 0)) {
+    qsx_set_error("packed schedule: needs qsx_hv_ctx_set_packed and a folded diagonal");
+    return QSX_ERR_UNSUPPORTED;
+  }
+  if (!X || sched < 0 || sched > 13) { qsx_set_error("qsx_hv_ctx_set_schedule: bad arguments"); return QSX_ERR_ARG; }
   if ((sched == 7 && !X->split_d) || (sched == 11 && !X->split_z)) {
     const int rc = split_build(X, sched == 11);
     if (rc) return rc;
@@ -1081,6 +1089,45 @@ extern "C" int qsx_hv_ctx_set_diag(qsx_hv_ctx* X, const void* diag_arr, int diag
   X->A.diag_conj = 0;
   X->A.diag_arr = diag_arr;
   X->A.diag_arr_cplx = diag_arr_cplx ? 1 : 0;
+  ctx_changed(X);
+  return QSX_OK;
+}
+
+// Arguments of the element evaluation that qsx_hv_pack_count / _fill run.
+int qsx_hv_ctx_pack_args(const qsx_hv_ctx* X, HvArgs* A, int* N, int* nmaps, int* fermion, int* lookup) {
+  const qsx_core* c = X->c;
+  const qsx_oplist_full* L = X->L;
+  const bool scatter = c->h.nmaps > 0 && !L->symmetric && !X->transposed;
+  if (X->A.Ns < 1 || X->A.Ns >= INT32_MAX || L->base.n_off == 0 || scatter) {
+    qsx_set_error("packed rows: needs off-diagonal terms in the gather form");
+    return QSX_ERR_UNSUPPORTED;
+  }
+  *A = X->A;
+  A->off = X->transposed ? L->base.off : L->off_hc;
+  A->n_off = L->base.n_off;
+  A->off_conj = (X->transposed == X->conjugated) ? 1 : 0;
+  *N = c->h.N;
+  *nmaps = c->h.nmaps;
+  *fermion = c->h.fermion != 0;
+  *lookup = A->table ? LOOKUP_TABLE : pick_lookup(c, A->Ns);
+  return QSX_OK;
+}
+
+// Bind the packed rows of this operator (same basis, list and flags; any
+// dtype and number of vectors), which the caller keeps alive.  Null pointers
+// unbind them.
+extern "C" int qsx_hv_ctx_set_packed(qsx_hv_ctx* X, const int64_t* off, const void* ent, const void* lut, int n_lut,
+                                     int idx_bits) {
+  if (!X || (ent && (!off || !lut || n_lut < 1 || n_lut > 1024 || idx_bits < 1 || idx_bits > 31))) {
+    qsx_set_error("qsx_hv_ctx_set_packed: bad arguments");
+    return QSX_ERR_ARG;
+  }
+  if (!ent && X->A.sched == 13) X->A.sched = 0;
+  X->A.pk_off = ent ? off : nullptr;
+  X->A.pk_ent = (const uint32_t*)ent;
+  X->A.pk_lut = ent ? (const double2*)lut : nullptr;
+  X->A.pk_nlut = ent ? n_lut : 0;
+  X->A.pk_bits = ent ? idx_bits : 0;
   ctx_changed(X);
   return QSX_OK;
 }
@@ -1200,12 +1247,14 @@ int qsx_hv_expm_term(void* ctx, const HvTerm& T, hipStream_t st) {
 }
 
 // The same term with the Taylor epilogue (F += the stored term, the norms of
-// the term and of F into nB, nF) fused into the product.  Only the two-pass
-// split schedule fuses it; otherwise QSX_ERR_UNSUPPORTED is returned before
-// anything is launched, and the caller runs the separate epilogue.
+// the term and of F into nB, nF) fused into the product.  The two-pass split
+// schedule and the packed rows fuse it; otherwise QSX_ERR_UNSUPPORTED is
+// returned before anything is launched, and the caller runs the separate
+// epilogue.
 int qsx_hv_expm_term_epi(void* ctx, const HvTerm& T, void* F, double* nB, double* nF, hipStream_t st) {
   qsx_hv_ctx* X = (qsx_hv_ctx*)ctx;
-  if (!X->split_z || X->A.sched != 11 || X->A.nvec != 1) return QSX_ERR_UNSUPPORTED;
+  const bool split2 = X->split_z && X->A.sched == 11 && X->A.nvec == 1;
+  if (!split2 && !(X->A.sched == 13 && X->A.pk_ent && X->A.n_diag == 0)) return QSX_ERR_UNSUPPORTED;
   HvArgs A = X->A;
   expm_term_args(A, T);
   A.done = T.skip;

@@ -170,13 +170,19 @@ struct HvArgs {
   double* epi_nB;
   double* epi_nF;
   // truncation test of the previous term (c1 + c2 <= tol F; null: none), made
-  // by the row pass, which sets *done (the skip flag) for itself and the
-  // strip pass
+  // by the term's first launch (the row pass, or the packed product), which
+  // sets *done (the skip flag) for itself and what follows
   int* done;
   const double* chk_c1;
   const double* chk_c2;
   const double* chk_F;
   double tol;
+  // packed rows (schedule 13, packed_impl.h)
+  const uint32_t* pk_ent;
+  const int64_t* pk_off;
+  const double2* pk_lut;
+  int pk_nlut;
+  int pk_bits;
 };
 
 // Split-chain layout of one hard-core-boson particle sector of N <= 32 bits

@@ -1,0 +1,286 @@
+// Packed rows: the off-diagonal elements of a matrix-free operator in the
+// gather form, four bytes each, evaluated once and read back by every product.
+//
+// Slices of 64 rows (one wavefront); entry e of row r at
+//   off[r / 64] + 64 e + r % 64 :  column | id << idx_bits,
+// id pointing into a table of the operator's distinct coefficients (id 0 = 0,
+// the padding of rows shorter than their slice, which carries the row's own
+// index as its column).  A symmetry-reduced operator has few distinct
+// coefficients (couplings x characters x ratios of stabiliser sizes), so the
+// table sits in LDS and an element costs four streamed bytes and its gather.
+//
+// The sector table (one word per state of the particle sector) needs |G|
+// words per basis state and a divergent read per element; packed rows need
+// one word per element and stream it.  Heisenberg L = 28, k = 0, p = z = +1:
+// 24 MB against 160 MB.
+#pragma once
+#include "sparse_impl.h"
+
+constexpr int PK_SLOTS = 4096;   // hash slots of the coefficient dictionary
+constexpr int PK_LUT_MAX = 1024; // distinct coefficients (16 KB of LDS)
+
+// dictionary scratch of a build, in device memory
+struct PackDict {
+  unsigned long long key[PK_SLOTS];  // hash of the value, 0 = free
+  double2 val[PK_SLOTS];
+  int32_t id[PK_SLOTS];
+  int32_t n_lut;      // entries with id 0
+  int32_t bad;        // dictionary full, or two values with one hash
+  int64_t total;      // entries of all slices
+};
+
+__device__ __forceinline__ unsigned long long pk_hash(double2 v) {
+  unsigned long long a = (unsigned long long)__double_as_longlong(v.x);
+  unsigned long long b = (unsigned long long)__double_as_longlong(v.y);
+  unsigned long long h = a * 0x9E3779B97F4A7C15ull + (b ^ (b >> 29)) * 0xC2B2AE3D27D4EB4Full;
+  h ^= h >> 31;
+  h *= 0xD6E8FEB86659FD93ull;
+  h ^= h >> 32;
+  return h | 1ull;
+}
+
+// Slot of value v, entered when it is new; -1 when every slot is taken.
+__device__ __forceinline__ int pk_slot(PackDict* D, double2 v) {
+  const unsigned long long h = pk_hash(v);
+  int s = (int)(h >> 1) & (PK_SLOTS - 1);
+  for (int p = 0; p < PK_SLOTS; ++p) {
+    unsigned long long k = __hip_atomic_load(&D->key[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (k == 0) {
+      k = atomicCAS(&D->key[s], 0ull, h);
+      if (k == 0) { D->val[s] = v; return s; }
+    }
+    if (k == h) return s;
+    s = (s + 1) & (PK_SLOTS - 1);
+  }
+  return -1;
+}
+
+// A lane's four-byte entries with U gathers in flight.  Rows of the wave's
+// slice are consecutive lanes, so entry loads are 256-byte segments.
+//
+// Bound by the gathers of x (an L2 line per lane and element where the
+// columns of neighbouring rows differ) and the stream of entries.  EPI: the
+// launch is a Taylor term: truncation test of the previous term, F += the
+// stored term, norms into the slots.
+template <typename VT, bool EPI>
+__global__ void __launch_bounds__(256) k_packed_rows(HvArgs A) {
+  constexpr bool CPLX = VTr<VT>::cplx;
+  using LT = typename std::conditional<CPLX, double2, double>::type;
+  constexpr int U = 8;
+  __shared__ LT lut[PK_LUT_MAX];
+  if (A.skip && *A.skip) return;
+  if constexpr (EPI) {
+    if (A.chk_c1 && *A.chk_c1 + *A.chk_c2 <= A.tol * *A.chk_F) {
+      if (blockIdx.x == 0 && threadIdx.x == 0) *A.done = 1;
+      return;
+    }
+  }
+  for (int i = threadIdx.x; i < A.pk_nlut; i += 256) {
+    if constexpr (CPLX) lut[i] = A.pk_lut[i];
+    else lut[i] = A.pk_lut[i].x;
+  }
+  __syncthreads();
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  const int64_t nsl = (A.Ns + 63) >> 6;
+  const VT* __restrict__ vin = (const VT*)A.v_in;
+  VT* __restrict__ vout = (VT*)A.v_out;
+  const int bits = A.pk_bits;
+  const uint32_t cmask = (bits < 32 ? 1u << bits : 0u) - 1u;
+  double maxB = 0.0, maxF = 0.0;
+  const int64_t bi = xcd_chunked(blockIdx.x, gridDim.x, gridDim.x >= 16384 ? 256 : 64);
+  for (int64_t sl = bi * 4 + w; sl < nsl; sl += (int64_t)gridDim.x * 4) {
+    const int64_t r = sl * 64 + lane;
+    const int64_t rc = r < A.Ns ? r : A.Ns - 1;  // lanes past the last row read in bounds, store nothing
+    const int64_t o0 = A.pk_off[sl];
+    const int wid = (int)((A.pk_off[sl + 1] - o0) >> 6);
+    const uint32_t* __restrict__ en = A.pk_ent + o0 + lane;
+    double2 dg = make_double2(0.0, 0.0);
+    if (A.diag_arr) {
+      if (A.diag_arr_cplx) dg = ld_stream<double2>((const double2*)A.diag_arr + rc);
+      else dg = ld_stream<double>((const double*)A.diag_arr + rc);
+    }
+    const double2 xr = VTr<VT>::ld(vin + rc);
+    double2 acc = make_double2(0.0, 0.0);
+    for (int e0 = 0; e0 < wid; e0 += U) {
+      uint32_t ev[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        ev[u] = e0 + u < wid ? en[(int64_t)(e0 + u) * 64] : (uint32_t)rc;
+      VT xv[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) xv[u] = vin[ev[u] & cmask];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const double2 x = VTr<VT>::ld(&xv[u]);
+        const LT c = lut[ev[u] >> bits];
+        if constexpr (CPLX) acc = cadd(acc, cmul(c, x));
+        else acc.x += c * x.x;
+      }
+    }
+    if (r < A.Ns) {
+      const double2 dsum = cadd(cmul(dg, A.alpha_diag), A.shift);
+      double2 res;
+      if constexpr (CPLX) res = cadd(cmul(A.alpha_off, acc), cmul(dsum, xr));
+      else res = make_double2(A.alpha_off.x * acc.x + dsum.x * xr.x, 0.0);
+      if (A.beta) res = cadd(res, VTr<VT>::ld(vout + r));
+      VTr<VT>::st(vout + r, res);
+      if constexpr (EPI) {
+        VT* __restrict__ F = (VT*)A.epi_F;
+        const double2 rs = VTr<VT>::rnd(res);  // the stored (rounded) term enters F
+        const double2 f = VTr<VT>::rnd(cadd(VTr<VT>::ld(F + r), rs));
+        VTr<VT>::st(F + r, f);
+        maxB = fmax(maxB, CPLX ? cabs2(rs) : fabs(rs.x));
+        maxF = fmax(maxF, CPLX ? cabs2(f) : fabs(f.x));
+      }
+    }
+  }
+  if constexpr (EPI) epi_norms_out(A, maxB, maxF);
+}
+
+// Several vectors, (Ns, nvec) row-major: a block takes one slice, its entries
+// staged in LDS, 256 / G rows at a time with G lanes per row and CW columns
+// per lane (as k_csr_mm); gridDim.y splits a slice's rows over blocks when
+// there are few slices.
+constexpr int PK_STAGE = 32;  // entries per row staged; wider slices read from memory
+
+template <typename VT, int G, int CW, bool EPI>
+__global__ void __launch_bounds__(256) k_packed_mm(HvArgs A) {
+  constexpr bool CPLX = VTr<VT>::cplx;
+  using LT = typename std::conditional<CPLX, double2, double>::type;
+  constexpr int U = CW * sizeof(VT) >= 16 ? 4 : 8;
+  constexpr int RB = 256 / G;
+  __shared__ LT lut[PK_LUT_MAX];
+  __shared__ uint32_t s_ent[PK_STAGE * 64];
+  if (A.skip && *A.skip) return;
+  if constexpr (EPI) {
+    if (A.chk_c1 && *A.chk_c1 + *A.chk_c2 <= A.tol * *A.chk_F) {
+      if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *A.done = 1;
+      return;
+    }
+  }
+  const int64_t sl = xcd_chunked(blockIdx.x, gridDim.x, gridDim.x >= 16384 ? 256 : 64);
+  const int64_t o0 = A.pk_off[sl];
+  const int wid = (int)((A.pk_off[sl + 1] - o0) >> 6);
+  const uint32_t* __restrict__ ent = A.pk_ent + o0;
+  const bool staged = wid <= PK_STAGE;
+  if (staged)
+    for (int i = threadIdx.x; i < wid * 64; i += 256) s_ent[i] = ent[i];
+  for (int i = threadIdx.x; i < A.pk_nlut; i += 256) {
+    if constexpr (CPLX) lut[i] = A.pk_lut[i];
+    else lut[i] = A.pk_lut[i].x;
+  }
+  __syncthreads();
+  const VT* __restrict__ vin = (const VT*)A.v_in;
+  VT* __restrict__ vout = (VT*)A.v_out;
+  const int bits = A.pk_bits;
+  const uint32_t cmask = (bits < 32 ? 1u << bits : 0u) - 1u;
+  const int64_t nv = A.nvec;
+  const int lane = threadIdx.x % G;
+  double maxB = 0.0, maxF = 0.0;
+  for (int q0 = (int)blockIdx.y * RB; q0 < 64; q0 += (int)gridDim.y * RB) {
+    const int q = q0 + (int)(threadIdx.x / G);  // row of the slice
+    const int64_t r = sl * 64 + q;
+    const bool live = q < 64 && r < A.Ns;
+    const int qc = live ? q : 0;
+    const int64_t rc = sl * 64 + qc;
+    double2 dg = make_double2(0.0, 0.0);
+    if (A.diag_arr) {
+      if (A.diag_arr_cplx) dg = ((const double2*)A.diag_arr)[rc];
+      else dg.x = ((const double*)A.diag_arr)[rc];
+    }
+    const double2 dsum = cadd(cmul(dg, A.alpha_diag), A.shift);
+    double curB = 0.0, curF = 0.0;
+    for (int64_t j0 = 0; j0 < nv; j0 += G * CW) {
+      const bool ok = live && j0 + lane * CW < nv;
+      const int64_t j = ok ? j0 + lane * CW : 0;
+      double2 acc[CW];
+#pragma unroll
+      for (int c = 0; c < CW; ++c) acc[c] = make_double2(0.0, 0.0);
+      for (int e0 = 0; e0 < wid; e0 += U) {
+        uint32_t ev[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          ev[u] = e0 + u < wid ? (staged ? s_ent[(e0 + u) * 64 + qc] : ent[(int64_t)(e0 + u) * 64 + qc]) : (uint32_t)rc;
+        VecRun<VT, CW> xv[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) xv[u] = *(const VecRun<VT, CW>*)(vin + (int64_t)(ev[u] & cmask) * nv + j);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const LT m = lut[ev[u] >> bits];
+#pragma unroll
+          for (int c = 0; c < CW; ++c) {
+            const double2 x = VTr<VT>::ld(&xv[u].a[c]);
+            if constexpr (CPLX) acc[c] = cadd(acc[c], cmul(m, x));
+            else acc[c].x += m * x.x;
+          }
+        }
+      }
+      if (ok) {
+#pragma unroll
+        for (int c = 0; c < CW; ++c) {
+          const int64_t o = r * nv + j + c;
+          const double2 xr = VTr<VT>::ld(vin + o);
+          double2 res;
+          if constexpr (CPLX) res = cadd(cmul(A.alpha_off, acc[c]), cmul(dsum, xr));
+          else res = make_double2(A.alpha_off.x * acc[c].x + dsum.x * xr.x, 0.0);
+          if (A.beta) res = cadd(res, VTr<VT>::ld(vout + o));
+          VTr<VT>::st(vout + o, res);
+          if constexpr (EPI) {
+            VT* __restrict__ F = (VT*)A.epi_F;
+            const double2 rs = VTr<VT>::rnd(res);
+            const double2 f = VTr<VT>::rnd(cadd(VTr<VT>::ld(F + o), rs));
+            VTr<VT>::st(F + o, f);
+            curB += CPLX ? cabs2(rs) : fabs(rs.x);
+            curF += CPLX ? cabs2(f) : fabs(f.x);
+          }
+        }
+      }
+    }
+    if constexpr (EPI) {
+      maxB = fmax(maxB, grp_sum<G>(curB));
+      maxF = fmax(maxF, grp_sum<G>(curF));
+    }
+  }
+  if constexpr (EPI) epi_norms_out(A, maxB, maxF);
+}
+
+// Lanes per row: as k_csr_mm's rule, four at least (64 rows fill a block).
+inline int pk_group(int64_t n) {
+  int best = 64;
+  int64_t cost = INT64_MAX;
+  for (int g = 64; g >= 8; g >>= 1) {
+    const int64_t c = (n + g - 1) / g * (g + 4);
+    if (c < cost) { cost = c; best = g; }
+  }
+  return best == 8 && n <= 4 ? 4 : best;
+}
+
+template <typename VT, int CW, bool EPI>
+void launch_packed_mm(const HvArgs& A, hipStream_t st) {
+  const int G = pk_group(A.nvec / CW);
+  const int64_t nsl = (A.Ns + 63) / 64;
+  // a slice's row rounds over several blocks until about four blocks per CU
+  const int rounds = 64 * G / 256;
+  int64_t gy = nsl > 0 ? (1024 + nsl - 1) / nsl : 1;
+  if (gy > rounds) gy = rounds;
+  const dim3 grid((unsigned)nsl, (unsigned)(gy < 1 ? 1 : gy)), blk(256);
+  switch (G) {
+    case 4: hipLaunchKernelGGL((k_packed_mm<VT, 4, CW, EPI>), grid, blk, 0, st, A); break;
+    case 8: hipLaunchKernelGGL((k_packed_mm<VT, 8, CW, EPI>), grid, blk, 0, st, A); break;
+    case 16: hipLaunchKernelGGL((k_packed_mm<VT, 16, CW, EPI>), grid, blk, 0, st, A); break;
+    case 32: hipLaunchKernelGGL((k_packed_mm<VT, 32, CW, EPI>), grid, blk, 0, st, A); break;
+    default: hipLaunchKernelGGL((k_packed_mm<VT, 64, CW, EPI>), grid, blk, 0, st, A); break;
+  }
+}
+
+template <typename VT, bool EPI>
+void launch_packed_t(const HvArgs& A, hipStream_t st) {
+  if (A.nvec == 1) {
+    hipLaunchKernelGGL((k_packed_rows<VT, EPI>), dim3((unsigned)qsx_grid(A.Ns, 256)), dim3(256), 0, st, A);
+    return;
+  }
+  if constexpr (sizeof(VT) == 8) {
+    if (A.nvec % 2 == 0 && (uintptr_t)A.v_in % 16 == 0) { launch_packed_mm<VT, 2, EPI>(A, st); return; }
+  }
+  launch_packed_mm<VT, 1, EPI>(A, st);
+}

@@ -1149,7 +1149,7 @@ extern "C" int qsx_expm_multiply_mf(void* hv_ctx, int64_t Ns, int s, int m_star,
   const double er = a_re * mu_re - a_im * mu_im, ei = a_re * mu_im + a_im * mu_re;
   const double mag = std::exp(er / s);
   const double2 eta = make_double2(mag * std::cos(ei / s), mag * std::sin(ei / s));
-  bool fuse = nvec == 1;
+  bool fuse = true;
   QSX_VT_SWITCH(vec_dtype, hipLaunchKernelGGL(k_expm_start<VT>, dim3(rg), dim3(256), 0, st, (const VT*)v, (VT*)Bb[0], Ns,
                                               nvec, normB, 1));
   QSX_LAUNCH_CHECK();
@@ -1168,9 +1168,9 @@ extern "C" int qsx_expm_multiply_mf(void* hv_ctx, int64_t Ns, int s, int m_star,
       T.chk_c2 = normB + i * stride + j;
       T.chk_F = normF + i * stride + j;
       if (fuse) {
-        // the two-pass split product makes the truncation test in its row
-        // pass, and writes the term and updates F and the norms in its strip
-        // pass (no separate launches for either)
+        // the two-pass split product and the packed product make the
+        // truncation test, write the term and update F and the norms
+        // themselves (no separate launches for either)
         rc = qsx_hv_expm_term_epi(hv_ctx, T, v, normB + i * stride + j + 1, normF + i * stride + j + 1, st);
         if (rc == QSX_OK) continue;
         if (rc != QSX_ERR_UNSUPPORTED) return rc;

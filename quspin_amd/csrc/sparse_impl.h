@@ -215,6 +215,24 @@ __device__ __forceinline__ void block_norm_partials(const CsrArgs& A, double mb,
   }
 }
 
+// Block max of the row norms of a matrix-free Taylor term into its slots.
+__device__ __forceinline__ void epi_norms_out(const HvArgs& A, double mb, double mf) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    mb = fmax(mb, __shfl_xor(mb, o, 64));
+    mf = fmax(mf, __shfl_xor(mf, o, 64));
+  }
+  __shared__ double sw[2][4];
+  const int w = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) { sw[0][w] = mb; sw[1][w] = mf; }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int i = 1; i < (int)(blockDim.x >> 6); ++i) { mb = fmax(mb, sw[0][i]); mf = fmax(mf, sw[1][i]); }
+    atomic_max_nonneg(A.epi_nB, mb);
+    atomic_max_nonneg(A.epi_nF, mf);
+  }
+}
+
 template <typename MT, typename VT, int G, bool EPI, typename FT = VT>
 __global__ void __launch_bounds__(256) k_csr_spmv(CsrArgs A) {
   double2 a_t = A.a, mu_t = A.mu, xs = A.xdscale;

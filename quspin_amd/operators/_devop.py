@@ -196,9 +196,38 @@ class MatrixFreeOp:
         if key not in self._ctx:
             ctx = self._new_ctx(vdt, nvec)
             cfg = tuning.choose(self, ctx, vdt, nvec)
-            ctx.configure(cfg, self.basis)
+            self._configure(ctx, cfg)
             self._ctx[key] = ctx
         return self._ctx[key]
+
+    def _configure(self, ctx, cfg):
+        ctx.configure(cfg, self.basis, self._packed(ctx) if cfg.get("schedule") == "packed" else None)
+
+    def _packed(self, ctx):
+        """The operator's packed rows (offsets, entries, coefficients, column
+        bits), evaluated once through ``ctx`` (``qsx_hv_pack_*``) and shared
+        by its contexts; None when it has none or they would take more than
+        ``tuning.packed_limit`` bytes."""
+        if not hasattr(self, "_pk"):
+            self._pk = None
+            limit = tuning.packed_limit(self)
+            lib = L.load()
+            nwork = lib.qsx_hv_pack_work_bytes(self.Ns)
+            if nwork > 0 and 4 * self.Ns <= limit:
+                off = L.empty((self.Ns + 63) // 64 + 1, np.int64)
+                work = L.empty((nwork + 7) // 8, np.int64)
+                ent, nl, bits = L._i64(), L._i32(), L._i32()
+                rc = lib.qsx_hv_pack_count(ctx.h, ptr(off), ptr(work), nwork, C.byref(ent), C.byref(nl),
+                                           C.byref(bits), stream_handle())
+                if rc == L.QSX_OK and 4 * ent.value <= limit:
+                    entries = L.empty(max(ent.value, 1), np.int32)
+                    lut = L.empty(nl.value, np.complex128)
+                    rc = lib.qsx_hv_pack_fill(ctx.h, ptr(off), ptr(work), ptr(entries), ptr(lut), stream_handle())
+                    if rc == L.QSX_OK:
+                        self._pk = (off, entries, lut, bits.value)
+                if rc != L.QSX_ERR_UNSUPPORTED:
+                    L.check(rc, "qsx_hv_pack")
+        return self._pk
 
     @property
     def config(self):
@@ -408,7 +437,7 @@ class _Ctx:
         self.h = h
         self.cfg = {"lookup": "search", "schedule": "rows"}
 
-    def configure(self, cfg, basis):
+    def configure(self, cfg, basis, packed=None):
         lib = L.load()
         self.cfg = dict(cfg)
         if cfg.get("lookup") == "table":
@@ -424,6 +453,15 @@ class _Ctx:
         else:
             L.check(lib.qsx_hv_ctx_set_table(self.h, None, 0, 0, None, 0), "qsx_hv_ctx_set_table")
         code = tuning.SCHEDULES.get(cfg.get("schedule"), 0)
+        if cfg.get("schedule") == "packed":
+            self._pk = packed  # kept alive with the context
+            if packed is None:
+                self.cfg["schedule"] = "rows"
+                code = 0
+            else:
+                off, ent, lut, bits = packed
+                L.check(lib.qsx_hv_ctx_set_packed(self.h, ptr(off), ptr(ent), ptr(lut), int(lut.numel()), bits),
+                        "qsx_hv_ctx_set_packed")
         rc = lib.qsx_hv_ctx_set_schedule(self.h, code)
         if rc == L.QSX_ERR_UNSUPPORTED and code == tuning.SCHEDULES["split"]:
             # the split-chain layout needs one hcb sector without symmetry

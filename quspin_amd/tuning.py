@@ -11,7 +11,10 @@ run of rows; "split": blocks of the split-chain layout of one hard-core-boson
 sector without symmetry maps; "split2": the same layout in two passes, lower
 half-chain terms per block, then upper-half and crossing terms over column
 strips; "chunk4/8": direct-rank rows with the terms in chunks and predicated
-gathers; all but "rows" for one vector only).  Candidates are timed on the operator's own
+gathers; all but "rows" for one vector only; "packed": the elements evaluated
+once, four bytes each, and streamed, for one vector or several).  A
+symmetry-reduced operator takes its packed rows where they are no larger than
+its sector table would be (``packed_limit``); the others' candidates are timed on the operator's own
 basis with HIP events (a few launches each) and the winner is cached per
 (basis signature, dtype, nvec) in memory and in a JSON file
 (``QSX_TUNE_CACHE``, default ``~/.cache/quspin_amd/tune.json``).
@@ -30,7 +33,19 @@ _mem = {}
 
 # schedule name -> launch code of qsx_hv_ctx_set_schedule
 SCHEDULES = {"rows": 0, "queue": 1, "rows2": 2, "rows4": 3, "rows8": 4, "batch4": 5, "batch8": 6, "split": 7,
-             "chunk4": 8, "chunk8": 9, "batch14": 10, "split2": 11, "batch14x": 12}
+             "chunk4": 8, "chunk8": 9, "batch14": 10, "split2": 11, "batch14x": 12, "packed": 13}
+
+# packed rows of sectors without symmetry maps, and of small sectors
+PACKED_BYTES = 64 << 20
+
+
+def packed_limit(op):
+    """Bytes the packed rows of ``op`` may take: what the sector table they
+    stand in for takes, 64 MiB where that is less or there is none."""
+    b = op.basis
+    if not len(b._pers) or 4 * op.oplist.n_off * b.Ns <= PACKED_BYTES:
+        return PACKED_BYTES
+    return max(PACKED_BYTES, b.lookup_table_bytes())
 
 
 def _cache_path():
@@ -58,7 +73,9 @@ def _save_file(d):
 
 def signature(op, vdt, nvec):
     b = op.basis
-    return "N{}_Ns{}_G{}_maps{}_q{}_off{}_diag{}_{}_nv{}_T{}C{}".format(
+    # (the number of schedules: a file written with fewer is timed again)
+    return "S{}_N{}_Ns{}_G{}_maps{}_q{}_off{}_diag{}_{}_nv{}_T{}C{}".format(
+        len(SCHEDULES),
         b.N, b.Ns, int(np.prod(b._pers)) if len(b._pers) else 1, len(b._pers), tuple(int(q) for q in b._qs),
         op.oplist.n_off, op.oplist.n_diag, np.dtype(vdt).name, nvec, int(op.transposed), int(op.conjugated))
 
@@ -87,7 +104,7 @@ def candidates(op, vdt, nvec):
     lookups = ["search"]
     if len(b._pers):
         lookups.append("table")
-    out = []
+    out = [] if len(b._pers) else [{"lookup": "search", "schedule": "packed"}]
     for lk in lookups:
         if nvec != 1:
             out.append({"lookup": lk, "schedule": "rows"})
@@ -131,7 +148,16 @@ def choose(op, ctx, vdt, nvec):
         if forced_s:
             cfg["schedule"] = forced_s
         return cfg
-    if os.environ.get("QSX_TUNE", "on") == "off" or op.basis.Ns < 4096:
+    if os.environ.get("QSX_TUNE", "on") == "off":
+        return static_rule(op, vdt, nvec)
+    if len(op.basis._pers) or op.basis.Ns < 4096:
+        # through the sector table where the basis holds it already
+        lookup = "table" if op.basis.has_lookup_table() else "search"
+        if lookup == "table":
+            ctx.configure({"lookup": lookup, "schedule": "rows"}, op.basis)
+        if op._packed(ctx) is not None:
+            return {"lookup": lookup, "schedule": "packed"}
+    if op.basis.Ns < 4096:
         return static_rule(op, vdt, nvec)
     key = signature(op, vdt, nvec)
     if key in _mem:
@@ -156,7 +182,7 @@ def time_candidates(op, ctx, vdt, nvec, reps=5):
     st = t.cuda.current_stream()
 
     def timed(cfg, n):
-        ctx.configure(cfg, op.basis)
+        op._configure(ctx, cfg)
         if ctx.cfg["lookup"] != cfg["lookup"] or ctx.cfg["schedule"] != cfg["schedule"]:
             return None
         for _ in range(2):

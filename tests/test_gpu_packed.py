@@ -1,0 +1,201 @@
+"""Packed rows of the matrix-free operator (one vector and blocks) against the
+assembled matrix of the same operator in 64-bit host arithmetic, over the
+bases, operator strings, flags and scales the product takes."""
+
+import numpy as np
+import pytest
+
+from models import chain_maps, hubbard_static, ladder_maps, xxz_static
+
+pytestmark = pytest.mark.gpu
+
+KW = dict(check_symm=False, check_herm=False, check_pcon=False)
+EPS = {np.dtype(np.float32): 2.0 ** -24, np.dtype(np.complex64): 2.0 ** -24,
+       np.dtype(np.float64): 2.0 ** -53, np.dtype(np.complex128): 2.0 ** -53}
+
+
+def _all_to_all(L):
+    pairs = [[0.1 * (i + 1), i, j] for i in range(L) for j in range(i + 1, L)]
+    half = [[0.5 * J, i, j] for J, i, j in pairs]
+    return [["+-", half], ["-+", half], ["zz", pairs]]
+
+
+def _case(name):
+    """(basis, static list, real elements)"""
+    from quspin_amd.basis import (spin_basis_general, spinful_fermion_basis_general, spinless_fermion_basis_general)
+    m = chain_maps(12)
+    if name == "kpz":
+        return spin_basis_general(12, Nup=6, pauli=0, kblock=(m["T"], 0), pblock=(m["P"], 0),
+                                  zblock=(m["Z"], 0)), xxz_static(12), True
+    if name == "momentum":
+        return spin_basis_general(12, Nup=5, pauli=0, kblock=(m["T"], 5)), xxz_static(12, Delta=0.7), False
+    if name == "no_nup":
+        return spin_basis_general(9, pauli=0, kblock=(chain_maps(9)["T"], 2)), [
+            ["xx", [[0.3, i, (i + 1) % 9] for i in range(9)]], ["xy", [[0.2, i, (i + 1) % 9] for i in range(9)]],
+            ["z", [[0.4, i] for i in range(9)]]], False
+    if name == "ladder":
+        lm = ladder_maps(4, 2)
+        bonds = [[0.5, i, (i + 1) % 4 + 4 * (i // 4)] for i in range(8)] + [[0.5, i, i + 4] for i in range(4)]
+        return spin_basis_general(8, Nup=4, pauli=0, kxblock=(lm["tx"], 1), zblock=(lm["z"], 1)), [
+            ["+-", bonds], ["-+", bonds], ["zz", bonds]], False
+    if name == "free":
+        return spin_basis_general(11, Nup=4, pauli=0), xxz_static(11, h=np.linspace(-1, 1, 11)), True
+    if name == "wide_rows":  # up to 49 elements per row
+        return spin_basis_general(14, Nup=7, pauli=0), _all_to_all(14), True
+    if name == "words64":
+        return spin_basis_general(34, Nup=3, pauli=0, kblock=(chain_maps(34)["T"], 0)), xxz_static(34), True
+    if name == "spinless":
+        i = np.arange(9)
+        bonds = [[-1.0, j, (j + 1) % 9] for j in range(9)]
+        return spinless_fermion_basis_general(9, Nf=4, kblock=((i + 1) % 9, 3)), [
+            ["+-", bonds], ["-+", [[1.0, a, b] for _, a, b in bonds]], ["nn", [[1.5, a, b] for _, a, b in bonds]]], False
+    i = np.arange(6)
+    return spinful_fermion_basis_general(6, Nf=(3, 2), kblock=((i + 1) % 6, 1)), hubbard_static(6, U=2.0), False
+
+
+def _vec(rng, n, nv, dtype):
+    shape = (n,) if nv == 1 else (n, nv)
+    x = rng.normal(size=shape)
+    if np.dtype(dtype).kind == "c":
+        x = x + 1j * rng.normal(size=shape)
+    return x.astype(dtype)
+
+
+def _check(y, A, x, a, diag, dtype, y0=None):
+    """FP64 sums of at most m elements and one rounding of the result; the
+    elements themselves are equal up to the rounding of their factors."""
+    xx = x.astype(np.complex128)
+    exact = a * (A @ xx)
+    mag = abs(a) * (abs(A) @ np.abs(xx))
+    if diag is not None:
+        d = diag if x.ndim == 1 else diag[:, None]
+        exact = exact + d * xx
+        mag = mag + np.abs(d * xx)
+    if y0 is not None:
+        exact, mag = exact + y0, mag + np.abs(y0)
+    m = int(np.diff(A.indptr).max())
+    bound = (16 * (m + 4) * 2.0 ** -53 + 2 * EPS[np.dtype(dtype)]) * mag + 1e-300
+    assert np.all(np.abs(y - exact) <= bound)
+
+
+@pytest.mark.parametrize("nv", [1, 2, 3, 8, 17, 64, 70])
+@pytest.mark.parametrize("name", ["kpz", "momentum", "no_nup", "ladder", "free", "wide_rows", "words64", "spinless",
+                                  "spinful"])
+def test_packed_product(name, nv):
+    from quspin_amd import _lib as L
+    from quspin_amd.operators import quantum_LinearOperator
+    basis, static, real = _case(name)
+    rng = np.random.default_rng(nv)
+    off = [t for t in static if set(t[0]) & set("+-xy")]
+    for dtype in ((np.float64, np.float32, np.complex128, np.complex64) if real else (np.complex128, np.complex64)):
+        Q = quantum_LinearOperator(static, basis=basis, dtype=dtype, **KW)
+        op = Q._qsx_operator()
+        A = quantum_LinearOperator(off, basis=basis, dtype=np.complex128, **KW)._qsx_operator().to_csr().to_scipy()
+        diag = L.to_host(op.diagonal(np.complex128))
+        x = _vec(rng, basis.Ns, nv, dtype)
+        a = 0.6 - (0.8j if np.dtype(dtype).kind == "c" else 0)
+        y = L.empty(x.shape, dtype)
+        op.apply(L.to_device(x), y, a=a, a_diag=0.5)
+        assert op.config[(np.dtype(dtype), nv)]["schedule"] == "packed"
+        _check(L.to_host(y), A, x, a, 0.5 * diag, dtype)
+        y0 = _vec(rng, basis.Ns, nv, dtype)
+        y = L.to_device(y0)
+        op.apply(L.to_device(x), y, a=a, beta=1, a_diag=0.0)
+        _check(L.to_host(y), A, x, a, None, dtype, y0)
+
+
+@pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("conjugated", [False, True])
+@pytest.mark.parametrize("name", ["momentum", "spinful", "no_nup"])
+def test_packed_flags(name, transposed, conjugated):
+    """Transposed and conjugated operators have rows of their own."""
+    from quspin_amd import _lib as L
+    from quspin_amd.operators._devop import MatrixFreeOp
+    basis, static, _ = _case(name)
+    static = [[op, [[b[0] * (1 + 0.3j)] + list(b[1:]) for b in bonds]] for op, bonds in static
+              if set(op) & set("+-xy")]
+    rng = np.random.default_rng(3)
+    from quspin_amd.operators._make_hamiltonian import _consolidate_static
+    ol = basis._compile_oplist(_consolidate_static(static))
+    A = MatrixFreeOp(basis, ol, np.complex128).to_csr().to_scipy()
+    if transposed:
+        A = A.T.tocsr()
+    if conjugated:
+        A = A.conj()
+    op = MatrixFreeOp(basis, ol, np.complex128, transposed=transposed, conjugated=conjugated)
+    for nv in (1, 5):
+        x = _vec(rng, basis.Ns, nv, np.complex128)
+        y = L.empty(x.shape, np.complex128)
+        op.apply(L.to_device(x), y)
+        assert op.config[(np.dtype(np.complex128), nv)]["schedule"] == "packed"
+        _check(L.to_host(y), A, x, 1.0, None, np.complex128)
+
+
+def test_packed_dictionary_overflow_takes_the_general_kernels():
+    """More distinct coefficients than the dictionary holds: refused, and the
+    product runs as it did."""
+    from itertools import combinations
+    from quspin_amd import _lib as L
+    from quspin_amd.basis import spin_basis_general
+    from quspin_amd.operators import quantum_LinearOperator
+    basis = spin_basis_general(10, pauli=0)
+    J = 1.0
+    static = []
+    for opstr in ("xxxx", "xxxz", "xxzz", "zxxx", "xzzx", "zxzx"):
+        bonds = []
+        for sites in combinations(range(10), 4):
+            J += 0.001
+            bonds.append([J] + list(sites))
+        static.append([opstr, bonds])
+    Q = quantum_LinearOperator(static, basis=basis, dtype=np.float64, **KW)
+    op = Q._qsx_operator()
+    x = _vec(np.random.default_rng(0), basis.Ns, 1, np.float64)
+    y = L.empty(x.shape, np.float64)
+    op.apply(L.to_device(x), y)
+    assert op.config[(np.dtype(np.float64), 1)]["schedule"] != "packed" and op._pk is None
+    _check(L.to_host(y), op.to_csr().to_scipy(), x, 1.0, None, np.float64)
+
+
+def test_packed_limit_and_replaced_diagonal(monkeypatch):
+    """Rows above the byte limit are not kept; a replaced diagonal and a later
+    operator on the same basis give their own products."""
+    from quspin_amd import _lib as L, tuning
+    from quspin_amd.operators import quantum_LinearOperator
+    basis, static, _ = _case("kpz")
+    x = _vec(np.random.default_rng(1), basis.Ns, 1, np.float64)
+    xd = L.to_device(x)
+    off = [t for t in static if set(t[0]) & set("+-")]
+    A = quantum_LinearOperator(off, basis=basis, dtype=np.complex128, **KW)._qsx_operator().to_csr().to_scipy()
+    Q = quantum_LinearOperator(static, basis=basis, dtype=np.float64, **KW)
+    before = L.to_host(Q._qsx_operator().diagonal(np.complex128))
+    _check(L.to_host(Q.dot(xd)), A, x, 1.0, before, np.float64)
+    d = np.linspace(0, 1, basis.Ns)
+    Q.set_diagonal(d)
+    _check(L.to_host(Q.dot(xd)), A, x, 1.0, d, np.float64)
+    Q2 = quantum_LinearOperator([[op, [[3 * b[0]] + b[1:] for b in bonds]] for op, bonds in static], basis=basis,
+                                dtype=np.float64, **KW)
+    _check(L.to_host(Q2.dot(xd)), A, x, 3.0, 3 * before, np.float64)
+    monkeypatch.setattr(tuning, "packed_limit", lambda op: 4 * op.Ns)
+    Q3 = quantum_LinearOperator(static, basis=basis, dtype=np.float64, **KW)
+    _check(L.to_host(Q3.dot(xd)), A, x, 1.0, before, np.float64)
+    assert Q3._qsx_operator()._pk is None
+
+
+@pytest.mark.parametrize("nv", [1, 4, 9])
+@pytest.mark.parametrize("name", ["momentum", "spinful", "free"])
+def test_packed_taylor_terms(name, nv):
+    """The Taylor loop whose terms run in the packed product."""
+    import scipy.linalg
+    from quspin_amd import _lib as L
+    from quspin_amd.operators import quantum_LinearOperator
+    from quspin_amd.tools.evolution import expm_multiply_parallel
+    basis, static, _ = _case(name)
+    Q = quantum_LinearOperator(static, basis=basis, dtype=np.complex128, **KW)
+    E = expm_multiply_parallel(Q, a=-0.9j)
+    x = _vec(np.random.default_rng(nv), basis.Ns, nv, np.complex128)
+    got = L.to_host(E.dot(L.to_device(x)))
+    assert Q._qsx_operator().config[(np.dtype(np.complex128), nv)]["schedule"] == "packed"
+    A = Q._qsx_operator().to_csr().to_scipy().toarray()
+    exact = scipy.linalg.expm(-0.9j * A) @ x
+    # unitary, about 30 terms, each rounded once; the largest partial sums are e^|a||A - mu| / 2
+    assert np.abs(got - exact).max() <= 1e-12 * np.abs(x).max()
