@@ -170,8 +170,8 @@ int64_t qsx_hv_pack_work_bytes(int64_t Ns);
 int qsx_hv_pack_count(const qsx_hv_ctx* ctx, int64_t* off, void* work, int64_t work_bytes, int64_t* entries,
                       int* n_lut, int* idx_bits, void* stream);
 int qsx_hv_pack_fill(const qsx_hv_ctx* ctx, int64_t* off, void* work, void* ent, void* lut, void* stream);
-int qsx_hv_ctx_set_packed(qsx_hv_ctx* ctx, const int64_t* off, const void* ent, const void* lut, int n_lut,
-                          int idx_bits);
+int qsx_hv_ctx_set_packed(qsx_hv_ctx* ctx, const int64_t* off, const void* ent, int64_t entries, const void* lut,
+                          int n_lut, int idx_bits);
 /* Replace the context's diagonal (diagonal terms and extra diagonal) by a
  * precomputed per-row array (Ns doubles, or Ns (re, im) pairs when
  * diag_arr_cplx), as quantum_LinearOperator keeps `_diagonal`
@@ -362,6 +362,15 @@ int qsx_lanczos_div(int dtype, const void* r, const double* b, void* q, int64_t 
 int qsx_lanczos_run(int op_kind, void* hv_ctx, const void* indptr, const void* indices, const void* data, int idx64,
                     int mat_dtype, int64_t nnz, int group, int dtype, int64_t n, int m, void* Q, int store_Q, void* r,
                     double* ab, int use_graph, void* stream);
+/* The recurrence of qsx_lanczos_run for a small operator in one launch, from
+ * v0 (divided by its norm when that is off 1 by more than eps): a_i and b_i
+ * into ab as there, q_0 .. q_{m-1} into Q (m, n) unless Q is NULL.
+ * QSX_ERR_UNSUPPORTED, nothing launched: an assembled matrix of more than
+ * 2,048 rows or 24,576 entries, a context of more than 4,096 rows or 49,152
+ * packed elements or not bound to packed rows. */
+int qsx_lanczos_small(int op_kind, const void* hv_ctx, const void* indptr, const void* indices, const void* data,
+                      int idx64, int mat_dtype, int64_t nnz, int dtype, int64_t n, int m, const void* v0, double eps,
+                      void* Q, double* ab, void* stream);
 int qsx_vdot(int dtype, const void* x, const void* y, int64_t n, double* out, void* stream);
 int qsx_nrm2(int dtype, const void* x, int64_t n, double* out, void* stream);
 int qsx_axpy(int dtype, const void* x, void* y, int64_t n, double a_re, double a_im, const double* sdev, double sgn,

@@ -719,6 +719,7 @@ struct qsx_hv_ctx {
   SplitDev* split_d = nullptr;
   bool split_z = false;
   int split_nxt = 0;  // up + crossing terms of the plan
+  int64_t pk_entries = 0;  // bound packed rows
 };
 
 static void split_free(qsx_hv_ctx* X) {
@@ -1113,12 +1114,21 @@ int qsx_hv_ctx_pack_args(const qsx_hv_ctx* X, HvArgs* A, int* N, int* nmaps, int
   return QSX_OK;
 }
 
+bool qsx_hv_ctx_packed(const void* hv_ctx, HvArgs* A, int* dtype, int64_t* entries) {
+  const qsx_hv_ctx* X = (const qsx_hv_ctx*)hv_ctx;
+  if (!X || X->A.sched != 13 || !X->A.pk_ent || X->A.n_diag > 0) return false;
+  *A = X->A;
+  *dtype = X->dtype;
+  *entries = X->pk_entries;
+  return true;
+}
+
 // Bind the packed rows of this operator (same basis, list and flags; any
 // dtype and number of vectors), which the caller keeps alive.  Null pointers
 // unbind them.
-extern "C" int qsx_hv_ctx_set_packed(qsx_hv_ctx* X, const int64_t* off, const void* ent, const void* lut, int n_lut,
-                                     int idx_bits) {
-  if (!X || (ent && (!off || !lut || n_lut < 1 || n_lut > 1024 || idx_bits < 1 || idx_bits > 31))) {
+extern "C" int qsx_hv_ctx_set_packed(qsx_hv_ctx* X, const int64_t* off, const void* ent, int64_t entries,
+                                     const void* lut, int n_lut, int idx_bits) {
+  if (!X || (ent && (!off || entries < 0 || !lut || n_lut < 1 || n_lut > 1024 || idx_bits < 1 || idx_bits > 31))) {
     qsx_set_error("qsx_hv_ctx_set_packed: bad arguments");
     return QSX_ERR_ARG;
   }
@@ -1128,6 +1138,7 @@ extern "C" int qsx_hv_ctx_set_packed(qsx_hv_ctx* X, const int64_t* off, const vo
   X->A.pk_lut = ent ? (const double2*)lut : nullptr;
   X->A.pk_nlut = ent ? n_lut : 0;
   X->A.pk_bits = ent ? idx_bits : 0;
+  X->pk_entries = ent ? entries : 0;
   ctx_changed(X);
   return QSX_OK;
 }

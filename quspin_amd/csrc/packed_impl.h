@@ -55,6 +55,10 @@ __device__ __forceinline__ int pk_slot(PackDict* D, double2 v) {
   return -1;
 }
 
+// The packed rows an H.v context is bound to and their number of entries
+// (hv.hip); false when its product takes another form.
+bool qsx_hv_ctx_packed(const void* hv_ctx, HvArgs* A, int* dtype, int64_t* entries);
+
 // A lane's four-byte entries with U gathers in flight.  Rows of the wave's
 // slice are consecutive lanes, so entry loads are 256-byte segments.
 //

@@ -62,6 +62,18 @@ struct HvTerm {
 int qsx_hv_expm_term(void* hv_ctx, const HvTerm& T, hipStream_t st);
 int qsx_hv_expm_term_epi(void* hv_ctx, const HvTerm& T, void* F, double* nB, double* nF, hipStream_t st);
 
+// A whole Taylor loop in one workgroup (small.hip): v <- e^{a A} v with the
+// partition (s, m).  False, nothing launched: not a small operator.
+struct SmallTaylor {
+  void* v;
+  int s, m;
+  double tol;
+  double2 a, mu;
+};
+bool qsx_small_expm_csr(const void* indptr, const void* indices, const void* data, int idx64, int mat_dtype, int64_t n,
+                        int64_t nnz, int vec_dtype, int64_t nvec, const SmallTaylor& T, hipStream_t st);
+bool qsx_small_expm_mf(const void* hv_ctx, int vec_dtype, int64_t nvec, const SmallTaylor& T, hipStream_t st);
+
 #define QSX_CHECK_HIP(expr)                                               \
   do {                                                                    \
     hipError_t _e = (expr);                                               \

@@ -1063,6 +1063,11 @@ extern "C" int qsx_expm_multiply_csr(const void* indptr, const void* indices, co
   if (Ns <= 0) return QSX_OK;
   int rc = expm_csr_check(Ns, s, m_star, vec_dtype, a_im, mu_im, "qsx_expm_multiply_csr");
   if (rc) return rc;
+  const SmallTaylor T{v, s, m_star, tol, make_double2(a_re, a_im), make_double2(mu_re, mu_im)};
+  if (qsx_small_expm_csr(indptr, indices, data, idx64, mat_dtype, Ns, nnz, vec_dtype, nvec, T, st)) {
+    QSX_LAUNCH_CHECK();
+    return QSX_OK;
+  }
   ExpmPlan P{s, m_star, tol, make_double2(a_re, a_im), make_double2(mu_re, mu_im), Ns, nvec, vec_dtype};
   ExpmCtl* ctl = nullptr;
   QSX_CHECK_HIP(hipMallocAsync((void**)&ctl, (size_t)expm_csr_ctl_bytes(s, m_star), st));
@@ -1121,6 +1126,11 @@ extern "C" int qsx_expm_multiply_csr_noalloc(const void* indptr, const void* ind
                   std::to_string(QSX_NOALLOC_SCRATCH_BYTES) + "-byte scratch");
     return QSX_ERR_ARG;
   }
+  const SmallTaylor T{v, s, m_star, tol, make_double2(a_re, a_im), make_double2(mu_re, mu_im)};
+  if (qsx_small_expm_csr(indptr, indices, data, idx64, mat_dtype, Ns, nnz, vec_dtype, nvec, T, st)) {
+    QSX_LAUNCH_CHECK();
+    return QSX_OK;
+  }
   void* p = nullptr;
   rc = noalloc_scratch(&p);
   if (rc) return rc;
@@ -1135,6 +1145,11 @@ extern "C" int qsx_expm_multiply_mf(void* hv_ctx, int64_t Ns, int s, int m_star,
   hipStream_t st = (hipStream_t)stream;
   if (Ns <= 0) return QSX_OK;
   if (s < 1 || m_star < 0) { qsx_set_error("qsx_expm_multiply_mf: bad partition"); return QSX_ERR_ARG; }
+  const SmallTaylor ST{v, s, m_star, tol, make_double2(a_re, a_im), make_double2(mu_re, mu_im)};
+  if (qsx_small_expm_mf(hv_ctx, vec_dtype, nvec, ST, st)) {
+    QSX_LAUNCH_CHECK();
+    return QSX_OK;
+  }
   ExpmPlan P{s, m_star, tol, make_double2(a_re, a_im), make_double2(mu_re, mu_im), Ns, nvec, vec_dtype};
   ExpmCtl* ctl = nullptr;
   double* slots = nullptr;

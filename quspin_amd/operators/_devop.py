@@ -460,8 +460,8 @@ class _Ctx:
                 code = 0
             else:
                 off, ent, lut, bits = packed
-                L.check(lib.qsx_hv_ctx_set_packed(self.h, ptr(off), ptr(ent), ptr(lut), int(lut.numel()), bits),
-                        "qsx_hv_ctx_set_packed")
+                L.check(lib.qsx_hv_ctx_set_packed(self.h, ptr(off), ptr(ent), int(ent.numel()), ptr(lut),
+                                                  int(lut.numel()), bits), "qsx_hv_ctx_set_packed")
         rc = lib.qsx_hv_ctx_set_schedule(self.h, code)
         if rc == L.QSX_ERR_UNSUPPORTED and code == tuning.SCHEDULES["split"]:
             # the split-chain layout needs one hcb sector without symmetry

@@ -4,7 +4,7 @@ _expm.py:7-52) with the recurrence on the device.
 For operators the library can run (``hamiltonian``, ``quantum_LinearOperator``,
 scipy matrices, device CSR) each step is one H.v launch plus two fused
 update kernels (r -= b v, a = Re<q,r>; r -= a q, b = ||r||) with FP64
-accumulation; a and b stay in device memory until the loop ends, and the
+accumulation (small operators run the whole recurrence in one launch); a and b stay in device memory until the loop ends, and the
 tridiagonal problem is solved in FP64 with ``scipy.linalg.eigh_tridiagonal``
 as in the reference.  Other operators go through their own ``dot``.
 """
@@ -40,7 +40,20 @@ def _device_loop(op, v0, m, dtype, eps, store_Q, Q_out=None):
     n = op.shape[0]
     code = L.dtype_code(dtype)
     st = stream_handle()
-    q0 = L.to_device(v0, dtype).reshape(n).clone()
+    kind = _run_kind(op, dtype)
+    q0 = L.to_device(v0, dtype).reshape(n)
+    if kind is not None:
+        # a small operator: normalisation and recurrence in one launch
+        direct = Q_out is not None and Q_out.is_contiguous()
+        Q = (Q_out if direct else L.empty((m, n), dtype)) if store_Q else None
+        ab = L.zeros((m, 2, 2), np.float64)
+        rc = lib.qsx_lanczos_small(*_run_args(*kind, dtype), code, n, m, ptr(q0), float(eps), ptr(Q), ptr(ab), st)
+        if rc != L.QSX_ERR_UNSUPPORTED:
+            L.check(rc, "qsx_lanczos_small")
+            if Q_out is not None and not direct:
+                Q = Q_out.copy_(Q)
+            return _finish(ab, m, eps, Q)
+    q0 = q0.clone()
     qn = nrm2_dev(q0)
     if abs(qn - 1.0) > eps:
         _scale_div(q0, qn, dtype)
@@ -54,21 +67,14 @@ def _device_loop(op, v0, m, dtype, eps, store_Q, Q_out=None):
         qbuf = None
     r = L.empty(n, dtype)
     ab = L.zeros((m, 2, 2), np.float64)  # [i, 0] = a_i, [i, 1] = b_i (2 doubles each)
-    kind = _run_kind(op, dtype)
     if kind is not None and m >= 8:
         # the whole recurrence as one device launch sequence, captured once per
         # operator and shape and replayed (the workspace keeps its addresses)
         ws = _workspace(op, dtype, n, m, store_Q)
         Qbuf, r, ab = ws["Q"], ws["r"], ws["ab"]
         Qbuf[0].copy_(q0)
-        ctx, csr = kind
-        if csr is None:
-            args = (0, ctx.h, None, None, None, 0, 0, 0, 0)
-        else:
-            d = csr._data_for(dtype)
-            args = (1, None, ptr(csr.indptr), ptr(csr.indices), ptr(d), csr.idx64,
-                    L.dtype_code(L.np_dtype(d.dtype)), csr.nnz, 0)
-        rc = lib.qsx_lanczos_run(*args, code, n, m, ptr(Qbuf), int(bool(store_Q)), ptr(r), ptr(ab), 1, st)
+        rc = lib.qsx_lanczos_run(*_run_args(*kind, dtype), 0, code, n, m, ptr(Qbuf), int(bool(store_Q)), ptr(r),
+                                 ptr(ab), 1, st)
         L.check(rc, "qsx_lanczos_run")
         if store_Q:
             Q.copy_(Qbuf)
@@ -125,6 +131,14 @@ def _run_kind(op, dtype):
     if isinstance(op, DeviceCSR):
         return None, op
     return None
+
+
+def _run_args(ctx, csr, dtype):
+    """Operator arguments of ``qsx_lanczos_run`` / ``qsx_lanczos_small``."""
+    if csr is None:
+        return (0, ctx.h, None, None, None, 0, 0, 0)
+    d = csr._data_for(dtype)
+    return (1, None, ptr(csr.indptr), ptr(csr.indices), ptr(d), csr.idx64, L.dtype_code(L.np_dtype(d.dtype)), csr.nnz)
 
 
 def _host_loop(A, v0, m, dtype, eps):

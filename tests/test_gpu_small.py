@@ -1,0 +1,107 @@
+"""The one-workgroup Taylor loop and Lanczos recurrence of small operators,
+at the edges of their row ranges, against 64-bit host arithmetic."""
+
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+from models import chain_maps, xxz_static
+
+pytestmark = pytest.mark.gpu
+
+EPS = {np.dtype(np.float32): 2.0 ** -24, np.dtype(np.complex64): 2.0 ** -24,
+       np.dtype(np.float64): 2.0 ** -53, np.dtype(np.complex128): 2.0 ** -53}
+KW = dict(check_symm=False, check_herm=False, check_pcon=False)
+
+
+def _hermitian(rng, n, cplx, bands=(0, 1, 7)):
+    """Banded Hermitian matrix with some empty rows and norm of order one."""
+    A = sp.lil_matrix((n, n), dtype=np.complex128 if cplx else np.float64)
+    for b in bands:
+        for i in range(n - b):
+            if rng.random() < 0.8:
+                z = rng.normal() * 0.3 + (1j * rng.normal() * 0.3 if cplx and b else 0)
+                A[i, i + b] = z
+                A[i + b, i] = np.conj(z)
+    return A.tocsr()
+
+
+def _vec(rng, n, dtype):
+    x = rng.normal(size=n)
+    if np.dtype(dtype).kind == "c":
+        x = x + 1j * rng.normal(size=n)
+    return (x / np.linalg.norm(x)).astype(dtype)
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 1023, 1024, 1025, 2048, 2049, 4095, 4096, 4097])
+@pytest.mark.parametrize("mdt,vdt,a", [(np.float64, np.complex128, -3.0j), (np.complex128, np.complex128, -0.4j),
+                                       (np.float64, np.float64, -0.7), (np.float32, np.complex64, -1.1j),
+                                       (np.complex64, np.complex64, -0.3j), (np.float32, np.float32, -0.5)])
+def test_small_expm(n, mdt, vdt, a):
+    from scipy.sparse.linalg import expm_multiply
+    from quspin_amd import _lib as L
+    from quspin_amd.operators._devop import DeviceCSR
+    from quspin_amd.tools.evolution import expm_multiply_parallel
+    rng = np.random.default_rng(n)
+    A = _hermitian(rng, n, np.dtype(mdt).kind == "c").astype(mdt)
+    E = expm_multiply_parallel(DeviceCSR.from_scipy(A, mdt), a=a, dtype=vdt)
+    x = _vec(rng, n, vdt)
+    got = L.to_host(E.dot(L.to_device(x)))
+    wide = A.astype(np.complex128 if np.iscomplexobj(A) else np.float64)
+    exact = expm_multiply(a * wide, x.astype(np.complex128))
+    # each stage: the truncation tolerance and one rounding per term of partial sums of at most e^|a A|
+    radius = abs(a) * float(abs(wide).sum(axis=0).max()) / E.partition[1]
+    bound = E.partition[1] * (E.partition[0] + 2) * EPS[np.dtype(vdt)] * min(np.exp(radius), 1e4)
+    assert np.linalg.norm(got - exact) <= bound * max(np.linalg.norm(exact), np.linalg.norm(x))
+
+
+@pytest.mark.parametrize("n,m", [(2, 1), (40, 9), (64, 20), (65, 20), (1024, 12), (1025, 12), (2049, 12), (4096, 12),
+                                 (4097, 12)])
+@pytest.mark.parametrize("dtype", [np.float64, np.complex128, np.complex64])
+def test_small_lanczos(n, m, dtype):
+    from quspin_amd import _lib as L
+    from quspin_amd.operators._devop import DeviceCSR
+    from quspin_amd.tools.lanczos import _host_loop, lanczos_full, lanczos_iter
+    rng = np.random.default_rng(n + m)
+    A = _hermitian(rng, n, np.dtype(dtype).kind == "c").astype(dtype)
+    x = 2.5 * _vec(rng, n, dtype)  # not normalised
+    E, V, Q = lanczos_full(DeviceCSR.from_scipy(A, dtype), L.to_device(x), m)
+    wide = A.astype(np.complex128)
+    a, b, mm, Qh = _host_loop(wide, x.astype(np.complex128), m, np.complex128, 0.0)
+    Eh = np.linalg.eigvalsh(np.diag(a) + np.diag(b[:-1], 1) + np.diag(b[:-1], -1))
+    # the first vectors to rounding grown by at most a factor of 8 per step here
+    tol = 64 * EPS[np.dtype(dtype)]
+    k = min(m, 5)
+    assert np.abs(L.to_host(Q)[:k] - Qh[:k]).max() <= tol * 8 ** k
+    assert np.abs(E - Eh).max() <= 200 * EPS[np.dtype(dtype)] * max(1.0, np.abs(Eh).max()) * m
+    E2, V2 = lanczos_iter(DeviceCSR.from_scipy(A, dtype), L.to_device(x), m, return_vec_iter=False)
+    assert np.array_equal(E, E2)
+    out = L.empty((m, 2 * n), dtype)[:, :n]  # rows apart
+    E3, _, Q3 = lanczos_full(DeviceCSR.from_scipy(A, dtype), L.to_device(x), m, out=out)
+    assert np.array_equal(E, E3) and np.array_equal(L.to_host(Q3), L.to_host(Q))
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32, np.complex128])
+def test_small_packed_rows_match_the_large_path(dtype, monkeypatch):
+    """A matrix-free sector: the one-launch forms against the launch-per-step
+    forms of the same operator (a forced schedule has no packed rows)."""
+    from quspin_amd import _lib as L
+    from quspin_amd.basis import spin_basis_general
+    from quspin_amd.operators import quantum_LinearOperator
+    from quspin_amd.tools.evolution import expm_multiply_parallel
+    from quspin_amd.tools.lanczos import lanczos_full
+    m = chain_maps(12)
+    basis = spin_basis_general(12, Nup=6, pauli=0, kblock=(m["T"], 0 if np.dtype(dtype).kind == "f" else 5))
+    x = _vec(np.random.default_rng(2), basis.Ns, dtype)
+    got = []
+    for forced in (None, "rows"):
+        if forced:
+            monkeypatch.setenv("QSX_SCHEDULE", forced)
+        Q = quantum_LinearOperator(xxz_static(12, Delta=0.8), basis=basis, dtype=dtype, **KW)
+        F = expm_multiply_parallel(Q, a=-0.6, dtype=dtype).dot(L.to_device(x))
+        E, V, _ = lanczos_full(Q, L.to_device(x), 20)
+        sched = Q._qsx_operator().config[(np.dtype(dtype), 1)]["schedule"]
+        assert (sched == "packed") == (forced is None)
+        got.append((L.to_host(F), E))
+    assert np.abs(got[0][0] - got[1][0]).max() <= 200 * EPS[np.dtype(dtype)]
+    assert np.abs(got[0][1] - got[1][1]).max() <= 4000 * EPS[np.dtype(dtype)]
