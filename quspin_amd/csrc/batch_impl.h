@@ -426,6 +426,182 @@ __global__ void __launch_bounds__(256) k_csr_wave(BatchArgs B) {
   }
 }
 
+// The CSR form for vectors that fill at most half a wavefront (CW columns per
+// lane): G lanes per row, 64 / G rows of the chunk side by side.  The rows of
+// a pass are consecutive, and so are their entries: they go through LDS, 128
+// at a time, read lane-parallel and, for the next pass, requested before this
+// pass' gathers are used; each lane keeps U gathers in flight.
+constexpr int WAVE_CAP = 128;  // entries staged per wavefront
+
+template <typename VT, int G, int CW, bool EPI>
+__global__ void __launch_bounds__(256) k_csr_wave_g(BatchArgs B) {
+  __shared__ int32_t s_col[4][WAVE_CAP];
+  __shared__ VT s_val[4][WAVE_CAP];
+  constexpr bool CPLX = VTr<VT>::cplx;
+  constexpr int RG = 64 / G;
+  constexpr int U = CW * sizeof(VT) >= 16 ? 4 : 8;
+  constexpr int PF = WAVE_CAP / 64;
+  const int64_t ci = wave_chunk_index<(sizeof(VT) <= 8)>(B);
+  if (ci >= B.nchunk) return;
+  const WaveChunk ch = uniform_chunk(B.chunk[ci]);
+  const int k = ch.sec;
+  const CsrSec S = B.csr[k];
+  const int lane = lane_id(), w = threadIdx.x >> 6;
+  const int l = lane % G, g = lane / G;
+  double2 coef_s = B.alpha, shift = make_double2(0.0, 0.0), dsc = B.xdscale;
+  if constexpr (EPI) {
+    if (!taylor_term_setup(B, k, lane, coef_s, shift, dsc)) return;
+  }
+  const double* __restrict__ xdiag = B.xdiag;
+  const int64_t base = uniform64(B.row_off[k]);
+  const VT* __restrict__ X = (const VT*)B.x + B.col0;
+  VT* __restrict__ Y = (VT*)B.y + B.col0;
+  VT* __restrict__ FF = EPI ? (VT*)B.F + B.col0 : nullptr;
+  const int32_t* __restrict__ ind = uniform_ptr(S.indices);
+  const VT* __restrict__ val = uniform_ptr((const VT*)S.data);
+  const bool col_ok = l * CW < B.ncol;
+  const int lc = col_ok ? l * CW : 0;
+  double maxB = 0.0, maxF = 0.0;
+  const int64_t rp = (lane <= ch.n) ? ld_idx(uniform_ptr(S.indptr), __builtin_amdgcn_readfirstlane(S.idx64),
+                                             ch.begin + lane) : 0;
+  int32_t c_nx[PF];
+  VT v_nx[PF];
+  auto request = [&](int64_t k0, int64_t k1) {
+#pragma unroll
+    for (int p = 0; p < PF; ++p) {
+      const int64_t kk = k0 + p * 64 + lane;
+      c_nx[p] = kk < k1 ? ind[kk] : 0;
+      v_nx[p] = kk < k1 ? val[kk] : vzero<VT>();
+    }
+  };
+  int64_t kb = rlane64(rp, 0);
+  int64_t ke = rlane64(rp, RG < ch.n ? RG : ch.n);
+  request(kb, ke);
+  for (int q0 = 0; q0 < ch.n; q0 += RG) {
+    const int q = q0 + g;
+    const bool live = q < ch.n;
+    const int qs = live ? q : ch.n - 1;
+    // (every lane shuffles: a source lane outside the branch would give nothing)
+    const int64_t k0 = __shfl(rp, qs, 64), kx = __shfl(rp, qs + 1, 64), k1 = live ? kx : k0;
+    const int64_t r_local = ch.begin + qs, row = base + r_local;
+    const VecRun<VT, CW> xr = *(const VecRun<VT, CW>*)(X + row * B.ld + lc);
+    VecRun<VT, CW> fr;  // F's run is requested with the row's own x, ahead of the gathers
+    if constexpr (EPI) fr = *(const VecRun<VT, CW>*)(FF + row * B.ld + lc);
+    double2 acc[CW];
+#pragma unroll
+    for (int c = 0; c < CW; ++c) acc[c] = make_double2(0.0, 0.0);
+    const int64_t kn = ke;  // the next pass' entries
+    const int64_t kne = q0 + RG < ch.n ? rlane64(rp, q0 + 2 * RG < ch.n ? q0 + 2 * RG : ch.n) : ke;
+    for (int64_t c0 = kb; c0 < ke; c0 += WAVE_CAP) {
+      if (c0 != kb) request(c0, ke);
+      wave_lds_sync();
+#pragma unroll
+      for (int p = 0; p < PF; ++p) {
+        s_col[w][p * 64 + lane] = c_nx[p];
+        s_val[w][p * 64 + lane] = v_nx[p];
+      }
+      wave_lds_sync();
+      if (c0 + WAVE_CAP >= ke) request(kn, kne);
+      const int64_t n = ke - c0 < WAVE_CAP ? ke - c0 : WAVE_CAP;
+      const int e0 = (int)(k0 > c0 ? k0 - c0 : 0);
+      const int e1 = k1 - c0 < n ? (int)(k1 - c0) : (int)n;  // may be <= e0
+      for (int e = e0; e < e1; e += U) {
+        VecRun<VT, CW> xv[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int ee = e + u < e1 ? e + u : e;
+          xv[u] = *(const VecRun<VT, CW>*)(X + (base + s_col[w][ee]) * B.ld + lc);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          if (e + u < e1) {
+            const double2 m = to_d2<VT>(s_val[w][e + u]);
+#pragma unroll
+            for (int c = 0; c < CW; ++c) {
+              const double2 x = to_d2<VT>(xv[u].a[c]);
+              if constexpr (CPLX) acc[c] = cadd(acc[c], cmul(m, x));
+              else acc[c].x += m.x * x.x;
+            }
+          }
+        }
+      }
+    }
+    if (kb == ke) request(kn, kne);
+    kb = kn;
+    ke = kne;
+    const double2 xw = xdiag ? make_double2(dsc.x * xdiag[row], dsc.y * xdiag[row]) : make_double2(0.0, 0.0);
+    double rb = 0.0, rf = 0.0;
+    if (live && col_ok) {
+      const int64_t o = row * B.ld + lc;
+      VecRun<VT, CW> yr;
+      if constexpr (!EPI) {
+        if (B.beta) yr = *(const VecRun<VT, CW>*)(Y + o);
+      }
+#pragma unroll
+      for (int c = 0; c < CW; ++c) {
+        const double2 x = to_d2<VT>(xr.a[c]);
+        if (xdiag) {
+          if constexpr (CPLX) acc[c] = cadd(acc[c], cmul(xw, x));
+          else acc[c].x += xw.x * x.x;
+        }
+        double2 res;
+        if constexpr (CPLX) res = cadd(cmul(coef_s, acc[c]), cmul(shift, x));
+        else res = make_double2(coef_s.x * acc[c].x + shift.x * x.x, 0.0);
+        if constexpr (!EPI) {
+          if (B.beta) res = cadd(res, to_d2<VT>(yr.a[c]));
+          VTr<VT>::st(&yr.a[c], res);
+        } else {
+          VTr<VT>::st(&yr.a[c], res);
+          const double2 rs = VTr<VT>::rnd(res);  // the stored (rounded) term enters F
+          const double2 f = VTr<VT>::rnd(cadd(to_d2<VT>(fr.a[c]), rs));
+          VTr<VT>::st(&fr.a[c], f);
+          rb += vabs<VT>(rs);
+          rf += vabs<VT>(f);
+        }
+      }
+      *(VecRun<VT, CW>*)(Y + o) = yr;
+      if constexpr (EPI) *(VecRun<VT, CW>*)(FF + o) = fr;
+    }
+    if constexpr (EPI) {
+      maxB = fmax(maxB, grp_sum<G>(rb));
+      maxF = fmax(maxF, grp_sum<G>(rf));
+    }
+  }
+  if constexpr (EPI) {
+#pragma unroll
+    for (int o = G; o < 64; o <<= 1) {
+      maxB = fmax(maxB, __shfl_xor(maxB, o, 64));
+      maxF = fmax(maxF, __shfl_xor(maxF, o, 64));
+    }
+    if (lane == 0) taylor_norms_out(B, k, maxB, maxF);
+  }
+}
+
+template <typename VT, int CW, bool EPI>
+void launch_csr_wave_w(const BatchArgs& B, dim3 grid, hipStream_t st) {
+  const int n = (B.ncol + CW - 1) / CW;
+  if (n <= 8) hipLaunchKernelGGL((k_csr_wave_g<VT, 8, CW, EPI>), grid, dim3(256), 0, st, B);
+  else if (n <= 16) hipLaunchKernelGGL((k_csr_wave_g<VT, 16, CW, EPI>), grid, dim3(256), 0, st, B);
+  else hipLaunchKernelGGL((k_csr_wave_g<VT, 32, CW, EPI>), grid, dim3(256), 0, st, B);
+}
+
+// k_csr_wave_g where a row of at most 64 columns leaves room for a second one
+// in the wavefront: up to 32 columns, or up to 64 with two 8-byte elements per
+// lane (an even number of columns on 16-byte boundaries).  All 20 momentum
+// sectors of the L = 20 Heisenberg chain, complex64 H.V: 32 columns 153 -> 57
+// us, 64 columns 139 -> 100 us; L = 22, 64 columns 549 -> 462 us.
+template <typename VT, bool EPI>
+void launch_csr_wave(const BatchArgs& B, dim3 grid, hipStream_t st) {
+  if constexpr (sizeof(VT) == 8) {
+    if (B.ncol % 2 == 0 && B.ld % 2 == 0 && B.col0 % 2 == 0 && ((uintptr_t)B.x | (uintptr_t)B.y | (uintptr_t)B.F) % 16 == 0) {
+      launch_csr_wave_w<VT, 2, EPI>(B, grid, st);
+      return;
+    }
+  }
+  if (B.ncol <= 32) { launch_csr_wave_w<VT, 1, EPI>(B, grid, st); return; }
+  hipLaunchKernelGGL((k_csr_wave<VT, EPI>), grid, dim3(256), 0, st, B);
+}
+
 // ---- Taylor-loop bookkeeping over the stacked sectors ---------------------
 
 // SCALE = false: B = F and ||F|| -> nB[k][0][0] (loop start).
@@ -490,8 +666,8 @@ void launch_hv_wave_t(const BatchArgs& B, int lookup, bool fermion, dim3 grid, h
     if (stage_kind == 1) { hipLaunchKernelGGL((k_batch_stage<VT, false>), grid, dim3(256), 0, st, B); return; } \
     if (stage_kind == 2) { hipLaunchKernelGGL((k_batch_stage<VT, true>), grid, dim3(256), 0, st, B); return; }  \
     if (B.csr) {                                                                                          \
-      if (epi) hipLaunchKernelGGL((k_csr_wave<VT, true>), grid, dim3(256), 0, st, B);                     \
-      else hipLaunchKernelGGL((k_csr_wave<VT, false>), grid, dim3(256), 0, st, B);                        \
+      if (epi) launch_csr_wave<VT, true>(B, grid, st);                                                    \
+      else launch_csr_wave<VT, false>(B, grid, st);                                                       \
       return;                                                                                             \
     }                                                                                                     \
     if (N <= 32) {                                                                                        \

@@ -224,15 +224,17 @@ BATCH_SCHEDULES = tuple((c, x) for x in (0, 1) for c in (4, 8, 16, 32))
 
 def choose_batch_schedule(batch, reps=3):
     """Chunk size and chunk order for a sector batch: timed on the batch's own
-    sectors (one H.V launch per candidate and repetition), cached like the
-    single-operator choices.  ``QSX_BATCH_CHUNK`` / ``QSX_BATCH_XCD`` force
-    values."""
+    sectors, cached like the single-operator choices.  The CSR form is timed
+    on Taylor terms, whose norms cost an atomic pair per chunk that the plain
+    product does not have (26 sectors of L = 26 x 64 complex64 vectors: chunks
+    of 4 rows give the fastest product, 7.6 ms, and a step of 1.79 s; chunks of
+    16 a step of 1.15 s).  ``QSX_BATCH_CHUNK`` / ``QSX_BATCH_XCD`` force values."""
     fc, fx = os.environ.get("QSX_BATCH_CHUNK"), os.environ.get("QSX_BATCH_XCD")
     if fc or fx:
         return int(fc or 16), int(fx or 0)
     if os.environ.get("QSX_TUNE", "on") == "off" or batch.rows < 65536:
         return 16, 0
-    key = _batch_key(batch.ops, batch.vdt, batch.nvec) + "_" + batch.form
+    key = _batch_key(batch.ops, batch.vdt, batch.nvec) + "_" + batch.form + "_terms"
     if key in _mem:
         return tuple(_mem[key]["schedule"])
     disk = _load_file()
@@ -241,18 +243,28 @@ def choose_batch_schedule(batch, reps=3):
         return tuple(disk[key]["schedule"])
     t = L.torch()
     x = t.ones((batch.rows, batch.nvec), dtype=L.torch_dtype(batch.vdt), device="cuda")
-    y = t.empty_like(x)
+    work = t.empty(2 * x.numel(), dtype=x.dtype, device="cuda")
     st = t.cuda.current_stream()
+    terms = batch.form == "csr" and batch.nvec <= 64  # what the Taylor loop takes
+    n = len(batch.ops)
     res = []
+
+    def once():
+        if terms:
+            # four terms of a tiny step: tol 0 runs them all
+            batch.expm_inplace(x, work, [(4, 1)] * n, [0.0] * n, [0.0] * n, 1e-6, graph=False)
+        else:
+            batch.apply(x, work[:x.numel()].view_as(x))
+
     for ch, xs in BATCH_SCHEDULES:
         if batch.form == "csr" and ch > 63:
             continue
         batch.set_schedule(ch, xs)
-        batch.apply(x, y)
+        once()
         e0, e1 = t.cuda.Event(enable_timing=True), t.cuda.Event(enable_timing=True)
         e0.record(st)
         for _ in range(reps):
-            batch.apply(x, y)
+            once()
         e1.record(st)
         t.cuda.synchronize()
         res.append((e0.elapsed_time(e1) / reps, (ch, xs)))

@@ -107,3 +107,57 @@ def test_expm_block_equals_single_columns(nv, dtype):
     # the loop's truncation tolerance and one rounding per term, with a margin
     tol = 40 * EPS[np.dtype(dtype)] * 2
     assert np.abs(got - exact).max() <= tol * np.abs(X).max() * 4
+
+
+@pytest.mark.parametrize("nv", [1, 2, 3, 8, 9, 16, 17, 31, 32, 33, 34, 63, 64, 70])
+@pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
+def test_sector_batch_csr_rows_side_by_side(nv, dtype):
+    """The CSR form of a sector batch at the edges of its column groups:
+    products against each sector's own matrix, and a Taylor step against the
+    per-sector path.  The long-range couplings give passes of more staged
+    entries than one round holds."""
+    from models import chain_maps
+    from quspin_amd import _lib as L
+    from quspin_amd.basis import spin_basis_general
+    from quspin_amd.operators import quantum_LinearOperator
+    from quspin_amd.operators._devop import SectorBatch
+    from quspin_amd.tools.evolution import expm_multiply_parallel, expm_multiply_sectors
+    size = 10
+    pairs = [[1.0 / min((j - i) % size, (i - j) % size), i, j] for i in range(size) for j in range(i + 1, size)]
+    half = [[0.5 * J, i, j] for J, i, j in pairs]
+    static = [["+-", half], ["-+", half], ["zz", pairs]]
+    kw = dict(check_symm=False, check_herm=False, check_pcon=False)
+    ops = [quantum_LinearOperator(static, basis=spin_basis_general(size, Nup=4 + (k % 2), pauli=0,
+                                                                   kblock=(chain_maps(size)["T"], k)), dtype=dtype,
+                                  **kw) for k in (0, 3, 7)]
+    mf = [op._qsx_operator() for op in ops]
+    rng = np.random.default_rng(nv)
+    for chunk in (1, 5, 16):
+        batch = SectorBatch(mf, dtype, nv, form="csr", chunk_rows=chunk)
+        x = [_vectors(rng, op.Ns, nv, dtype) for op in ops]
+        X = batch.stack(x)
+        Y = batch.empty()
+        batch.apply(X, Y, a=0.5 - 0.25j)
+        y0 = L.to_host(Y).copy()
+        batch.apply(X, Y, a=0.5 - 0.25j, beta=1)
+        y1 = L.to_host(Y)
+        at = 0
+        for op, xs in zip(mf, x):
+            A = op.to_csr(dtype).to_scipy()
+            exact = (0.5 - 0.25j) * (A.astype(np.complex128) @ xs.astype(np.complex128))
+            rows = slice(at, at + op.Ns)
+            bound = _bound(A, xs, dtype)
+            assert np.all(np.abs(y0[rows] - exact) <= bound)
+            assert np.all(np.abs(y1[rows] - 2 * exact) <= 4 * bound)
+            at += op.Ns
+    if nv > 64:
+        return
+    E = expm_multiply_sectors(ops, a=-0.4j, dtype=dtype, nvec=nv, form="csr", chunk_rows=5)
+    x = [_vectors(rng, op.Ns, nv, dtype) for op in ops]
+    F = L.to_host(E.dot(x))
+    at = 0
+    for op, xs in zip(ops, x):
+        one = L.to_host(expm_multiply_parallel(op, a=-0.4j, dtype=dtype).dot(L.to_device(xs)))
+        assert np.abs(F[at:at + op.Ns] - one.reshape(F[at:at + op.Ns].shape)).max() <= \
+            100 * EPS[np.dtype(dtype)] * np.abs(xs).max() * 4
+        at += op.Ns
