@@ -87,6 +87,14 @@ __device__ __forceinline__ double2 cmul(double2 a, double2 b) {
 __device__ __forceinline__ double2 cadd(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ double2 cconj(double2 a) { return make_double2(a.x, -a.y); }
 
+// A norm's per-element maximum without a square root per element: |z|^2 of a
+// complex element (|x| of a real one) is compared, and the root taken of the
+// maximum (sqrt is monotone and correctly rounded, so the value is the same).
+template <bool CPLX>
+__device__ __forceinline__ double norm_key(double2 v) { return CPLX ? v.x * v.x + v.y * v.y : fabs(v.x); }
+template <bool CPLX>
+__device__ __forceinline__ double norm_of_key(double k) { return CPLX ? sqrt(k) : k; }
+
 // sqrt of a small non-negative integer (stabiliser sizes): exact table for
 // n < 64, hardware sqrt above.
 __constant__ double c_sqrt_tab[64] = {
@@ -1910,8 +1918,8 @@ k_split2_strips(HvArgs A) {
         const double2 rs = VTr<VT>::rnd(res);
         const double2 f = VTr<VT>::rnd(cadd(ld_stream<VT>(F + row), rs));
         st_stream<VT>(F + row, f);
-        maxB = fmax(maxB, CPLX ? sqrt(rs.x * rs.x + rs.y * rs.y) : fabs(rs.x));
-        maxF = fmax(maxF, CPLX ? sqrt(f.x * f.x + f.y * f.y) : fabs(f.x));
+        maxB = fmax(maxB, norm_key<CPLX>(rs));
+        maxF = fmax(maxF, norm_key<CPLX>(f));
       }
     }
   }
@@ -1933,6 +1941,8 @@ k_split2_strips(HvArgs A) {
         mb = fmax(mb, s_m[0][i]);
         mf = fmax(mf, s_m[1][i]);
       }
+      mb = norm_of_key<CPLX>(mb);
+      mf = norm_of_key<CPLX>(mf);
       // non-negative doubles order as their bit patterns
       atomicMax((unsigned long long*)A.epi_nB, (unsigned long long)__double_as_longlong(mb));
       atomicMax((unsigned long long*)A.epi_nF, (unsigned long long)__double_as_longlong(mf));

@@ -244,7 +244,7 @@ constexpr int KRON_UP_ROWS = 4;  // up rows per wave in the column-strip pass
 // column d = 64 s + l, so every partner-row read is one coalesced segment of
 // the strip; the partner reads of the four rows are issued together.
 template <typename MT, typename VT, bool EPI, typename FT>
-__global__ void __launch_bounds__(256) k_kron_up(KronArgs K, int64_t nunits, int64_t groups,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EPI ? 6 : 1))) k_kron_up(KronArgs K, int64_t nunits, int64_t groups,
                                                  const int32_t* __restrict__ iu, const MT* __restrict__ du) {
   constexpr int RW = KRON_UP_ROWS;
   const CsrArgs& A = K.A;
@@ -362,12 +362,13 @@ __global__ void __launch_bounds__(256) k_kron_up(KronArgs K, int64_t nunits, int
         const double2 rs = VTr<VT>::rnd(res);
         const double2 fs = VTr<FT>::rnd(cadd(fo[r], rs));
         st_stream<FT>((FT*)A.F + row, fs);
-        maxB = fmax(maxB, VTr<VT>::cplx ? cabs2(rs) : fabs(rs.x));
-        maxF = fmax(maxF, VTr<VT>::cplx ? cabs2(fs) : fabs(fs.x));
+        maxB = fmax(maxB, norm_key<VTr<VT>::cplx>(rs));
+        maxF = fmax(maxF, norm_key<VTr<VT>::cplx>(fs));
       }
     }
   }
-  if constexpr (EPI) block_norm_partials(A, maxB, maxF);
+  if constexpr (EPI)
+    block_norm_partials(A, norm_of_key<VTr<VT>::cplx>(maxB), norm_of_key<VTr<VT>::cplx>(maxF));
 }
 
 static bool kron_two_pass(const qsx_kron* K, int64_t vsize) {

@@ -133,12 +133,12 @@ __global__ void __launch_bounds__(256) k_packed_rows(HvArgs A) {
         const double2 rs = VTr<VT>::rnd(res);  // the stored (rounded) term enters F
         const double2 f = VTr<VT>::rnd(cadd(VTr<VT>::ld(F + r), rs));
         VTr<VT>::st(F + r, f);
-        maxB = fmax(maxB, CPLX ? cabs2(rs) : fabs(rs.x));
-        maxF = fmax(maxF, CPLX ? cabs2(f) : fabs(f.x));
+        maxB = fmax(maxB, norm_key<CPLX>(rs));
+        maxF = fmax(maxF, norm_key<CPLX>(f));
       }
     }
   }
-  if constexpr (EPI) epi_norms_out(A, maxB, maxF);
+  if constexpr (EPI) epi_norms_out(A, norm_of_key<CPLX>(maxB), norm_of_key<CPLX>(maxF));
 }
 
 // Several vectors, (Ns, nvec) row-major: a block takes one slice, its entries
