@@ -362,6 +362,15 @@ int qsx_lanczos_div(int dtype, const void* r, const double* b, void* q, int64_t 
 int qsx_lanczos_run(int op_kind, void* hv_ctx, const void* indptr, const void* indices, const void* data, int idx64,
                     int mat_dtype, int64_t nnz, int group, int dtype, int64_t n, int m, void* Q, int store_Q, void* r,
                     double* ab, int use_graph, void* stream);
+/* The recurrence of qsx_lanczos_run on a context bound to packed rows, two
+ * launches per step, from v0 (divided by its norm when that is off 1 by more
+ * than eps).  Q: (m, n) with store_Q, else (3, n); r: (2, n); ab as there;
+ * work: qsx_lanczos_packed_work() doubles.  QSX_ERR_UNSUPPORTED, nothing
+ * launched: the context is not bound to packed rows. */
+int64_t qsx_lanczos_packed_work(void);
+int qsx_lanczos_packed(const void* hv_ctx, int dtype, int64_t n, int m, const void* v0, double eps, void* Q,
+                       int store_Q, void* r, double* ab, double* work, void* stream);
+
 /* The recurrence of qsx_lanczos_run for a small operator in one launch, from
  * v0 (divided by its norm when that is off 1 by more than eps): a_i and b_i
  * into ab as there, q_0 .. q_{m-1} into Q (m, n) unless Q is NULL.

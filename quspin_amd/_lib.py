@@ -61,6 +61,8 @@ SIGNATURES = {
     "qsx_hv_pack_count": (_i32, [_vp, _vp, _vp, _i64, C.POINTER(_i64), C.POINTER(_i32), C.POINTER(_i32), _vp]),
     "qsx_hv_pack_fill": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp]),
     "qsx_hv_ctx_set_packed": (_i32, [_vp, _vp, _vp, _i64, _vp, _i32, _i32]),
+    "qsx_lanczos_packed_work": (_i64, []),
+    "qsx_lanczos_packed": (_i32, [_vp, _i32, _i64, _i32, _vp, _dbl, _vp, _i32, _vp, _vp, _vp, _vp]),
     "qsx_lanczos_small": (_i32, [_i32, _vp, _vp, _vp, _vp, _i32, _i32, _i64, _i32, _i64, _i32, _vp, _dbl, _vp, _vp,
                                  _vp]),
     "qsx_table_info": (_i32, [_vp, _i64, _vp, _i32, C.POINTER(_i64), C.POINTER(_i32), C.POINTER(_i32),

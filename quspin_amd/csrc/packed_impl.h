@@ -59,19 +59,69 @@ __device__ __forceinline__ int pk_slot(PackDict* D, double2 v) {
 // (hv.hip); false when its product takes another form.
 bool qsx_hv_ctx_packed(const void* hv_ctx, HvArgs* A, int* dtype, int64_t* entries);
 
-// A lane's four-byte entries with U gathers in flight.  Rows of the wave's
-// slice are consecutive lanes, so entry loads are 256-byte segments.
+template <typename VT>
+using PkLut = typename std::conditional<VTr<VT>::cplx, double2, double>::type;
+
+template <typename VT>
+__device__ __forceinline__ void pk_stage_lut(const HvArgs& A, PkLut<VT>* lut) {
+  for (int i = threadIdx.x; i < A.pk_nlut; i += 256) {
+    if constexpr (VTr<VT>::cplx) lut[i] = A.pk_lut[i];
+    else lut[i] = A.pk_lut[i].x;
+  }
+}
+
+__device__ __forceinline__ double2 pk_diag(const HvArgs& A, int64_t r) {
+  if (!A.diag_arr) return make_double2(0.0, 0.0);
+  return A.diag_arr_cplx ? ld_stream<double2>((const double2*)A.diag_arr + r)
+                         : ld_stream<double>((const double*)A.diag_arr + r);
+}
+
+// Off-diagonal sum of row rc = 64 sl + lane (the last row for lanes past it):
+// the row's four-byte entries with U gathers in flight.  The rows of a slice
+// are consecutive lanes, so entry loads are 256-byte segments.
+template <typename VT>
+__device__ __forceinline__ double2 pk_row(const HvArgs& A, const PkLut<VT>* lut, const VT* __restrict__ vin, int64_t sl,
+                                          int lane, int64_t rc) {
+  constexpr int U = 8;
+  const int bits = A.pk_bits;
+  const uint32_t cmask = (1u << bits) - 1u;
+  const int64_t o0 = A.pk_off[sl];
+  const int wid = (int)((A.pk_off[sl + 1] - o0) >> 6);
+  const uint32_t* __restrict__ en = A.pk_ent + o0 + lane;
+  double2 acc = make_double2(0.0, 0.0);
+  for (int e0 = 0; e0 < wid; e0 += U) {
+    uint32_t ev[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) ev[u] = e0 + u < wid ? en[(int64_t)(e0 + u) * 64] : (uint32_t)rc;
+    VT xv[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) xv[u] = vin[ev[u] & cmask];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const double2 x = VTr<VT>::ld(&xv[u]);
+      const PkLut<VT> c = lut[ev[u] >> bits];
+      if constexpr (VTr<VT>::cplx) acc = cadd(acc, cmul(c, x));
+      else acc.x += c * x.x;
+    }
+  }
+  return acc;
+}
+
+// One vector, one lane per row.
 //
-// Bound by the gathers of x (an L2 line per lane and element where the
-// columns of neighbouring rows differ) and the stream of entries.  EPI: the
-// launch is a Taylor term: truncation test of the previous term, F += the
-// stored term, norms into the slots.
+// Bound by the gathers of x (an L2 line per lane and element where the columns
+// of neighbouring rows differ) and the stream of entries.  Heisenberg L = 28
+// k = 0 p = z = +1, float64: 13.1 us against 27.3 us through the sector table;
+// L = 34 827 against 1,162 us.  Eight gathers in flight (16: 14.9 us, 24: 14.0;
+// 4: 13.1); entries through the caches (non-temporal 15.6 us); blocks in runs
+// per XCD inside a shared window (dispatch order 13.4 us, one run per XCD
+// 14.2); entries in term order (sorted by column 13.8).  EPI: the launch is a
+// Taylor term: truncation test of the previous term, F += the stored term,
+// norms into the slots.
 template <typename VT, bool EPI>
 __global__ void __launch_bounds__(256) k_packed_rows(HvArgs A) {
   constexpr bool CPLX = VTr<VT>::cplx;
-  using LT = typename std::conditional<CPLX, double2, double>::type;
-  constexpr int U = 8;
-  __shared__ LT lut[PK_LUT_MAX];
+  __shared__ PkLut<VT> lut[PK_LUT_MAX];
   if (A.skip && *A.skip) return;
   if constexpr (EPI) {
     if (A.chk_c1 && *A.chk_c1 + *A.chk_c2 <= A.tol * *A.chk_F) {
@@ -79,48 +129,21 @@ __global__ void __launch_bounds__(256) k_packed_rows(HvArgs A) {
       return;
     }
   }
-  for (int i = threadIdx.x; i < A.pk_nlut; i += 256) {
-    if constexpr (CPLX) lut[i] = A.pk_lut[i];
-    else lut[i] = A.pk_lut[i].x;
-  }
+  pk_stage_lut<VT>(A, lut);
   __syncthreads();
   const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   const int64_t nsl = (A.Ns + 63) >> 6;
   const VT* __restrict__ vin = (const VT*)A.v_in;
   VT* __restrict__ vout = (VT*)A.v_out;
-  const int bits = A.pk_bits;
-  const uint32_t cmask = (bits < 32 ? 1u << bits : 0u) - 1u;
   double maxB = 0.0, maxF = 0.0;
   const int64_t bi = xcd_chunked(blockIdx.x, gridDim.x, gridDim.x >= 16384 ? 256 : 64);
-  for (int64_t sl = bi * 4 + w; sl < nsl; sl += (int64_t)gridDim.x * 4) {
-    const int64_t r = sl * 64 + lane;
+  const int64_t sl = bi * 4 + w;
+  const int64_t r = sl * 64 + lane;
+  if (sl < nsl) {
     const int64_t rc = r < A.Ns ? r : A.Ns - 1;  // lanes past the last row read in bounds, store nothing
-    const int64_t o0 = A.pk_off[sl];
-    const int wid = (int)((A.pk_off[sl + 1] - o0) >> 6);
-    const uint32_t* __restrict__ en = A.pk_ent + o0 + lane;
-    double2 dg = make_double2(0.0, 0.0);
-    if (A.diag_arr) {
-      if (A.diag_arr_cplx) dg = ld_stream<double2>((const double2*)A.diag_arr + rc);
-      else dg = ld_stream<double>((const double*)A.diag_arr + rc);
-    }
+    const double2 dg = pk_diag(A, rc);
     const double2 xr = VTr<VT>::ld(vin + rc);
-    double2 acc = make_double2(0.0, 0.0);
-    for (int e0 = 0; e0 < wid; e0 += U) {
-      uint32_t ev[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        ev[u] = e0 + u < wid ? en[(int64_t)(e0 + u) * 64] : (uint32_t)rc;
-      VT xv[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) xv[u] = vin[ev[u] & cmask];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const double2 x = VTr<VT>::ld(&xv[u]);
-        const LT c = lut[ev[u] >> bits];
-        if constexpr (CPLX) acc = cadd(acc, cmul(c, x));
-        else acc.x += c * x.x;
-      }
-    }
+    const double2 acc = pk_row<VT>(A, lut, vin, sl, lane, rc);
     if (r < A.Ns) {
       const double2 dsum = cadd(cmul(dg, A.alpha_diag), A.shift);
       double2 res;
@@ -133,12 +156,69 @@ __global__ void __launch_bounds__(256) k_packed_rows(HvArgs A) {
         const double2 rs = VTr<VT>::rnd(res);  // the stored (rounded) term enters F
         const double2 f = VTr<VT>::rnd(cadd(VTr<VT>::ld(F + r), rs));
         VTr<VT>::st(F + r, f);
-        maxB = fmax(maxB, norm_key<CPLX>(rs));
-        maxF = fmax(maxF, norm_key<CPLX>(f));
+        maxB = norm_key<CPLX>(rs);
+        maxF = norm_key<CPLX>(f);
       }
     }
   }
   if constexpr (EPI) epi_norms_out(A, norm_of_key<CPLX>(maxB), norm_of_key<CPLX>(maxF));
+}
+
+// One Lanczos step up to its dot, from the residual r of the step before
+// (not normalised) and the nb partials of ||r||^2:
+//   b = ||r||, q = r / b (stored), s = H q - b q_prev (stored),
+//   the block's partial of Re <q, s>.
+// H q is formed as (H r) / b, so the division and the gathers share one
+// launch: the partials are summed after the gathers, hidden behind the other
+// blocks' loads.  first: r is the start vector, divided only when its norm is
+// off 1 by more than eps, and no b is recorded.
+template <typename VT>
+__global__ void __launch_bounds__(256) k_packed_lz(HvArgs A, const double* __restrict__ pnrm, int nb,
+                                                   VT* __restrict__ q, const VT* __restrict__ qprev, double* bout,
+                                                   double eps, int first, double* __restrict__ pdot) {
+  constexpr bool CPLX = VTr<VT>::cplx;
+  __shared__ PkLut<VT> lut[PK_LUT_MAX];
+  pk_stage_lut<VT>(A, lut);
+  __syncthreads();
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  const int64_t nsl = (A.Ns + 63) >> 6;
+  const VT* __restrict__ vin = (const VT*)A.v_in;
+  VT* __restrict__ vout = (VT*)A.v_out;
+  const int64_t bi = xcd_chunked(blockIdx.x, gridDim.x, 64);
+  double b = 0.0, dot = 0.0;
+  bool have = false;
+  // every block makes the same number of rounds, so the sum's barriers match
+  const int64_t rounds = (nsl + 4 * (int64_t)gridDim.x - 1) / (4 * (int64_t)gridDim.x);
+  for (int64_t it = 0; it < rounds; ++it) {
+    const int64_t sl = (it * gridDim.x + bi) * 4 + w;
+    const int64_t r = sl * 64 + lane;
+    const bool live = r < A.Ns;
+    double2 xr = make_double2(0.0, 0.0), h = make_double2(0.0, 0.0), qp = make_double2(0.0, 0.0);
+    if (sl < nsl) {
+      const int64_t rc = live ? r : A.Ns - 1;
+      const double2 dg = pk_diag(A, rc);
+      xr = VTr<VT>::ld(vin + rc);
+      if (qprev) qp = VTr<VT>::ld(qprev + rc);
+      h = pk_row<VT>(A, lut, vin, sl, lane, rc);
+      if constexpr (CPLX) h = cadd(h, cmul(dg, xr));
+      else h.x += dg.x * xr.x;
+    }
+    if (!have) {
+      b = sqrt(sum_partials(pnrm, nb));
+      have = true;
+      if (blockIdx.x == 0 && threadIdx.x == 0 && bout) bout[0] = b;
+      if (first && fabs(b - 1.0) <= eps) b = 1.0;
+    }
+    if (live) {
+      const double2 qq = VTr<VT>::rnd(make_double2(xr.x / b, xr.y / b));
+      VTr<VT>::st(q + r, qq);
+      double2 s = VTr<VT>::rnd(make_double2(h.x / b, h.y / b));
+      if (qprev) s = VTr<VT>::rnd(make_double2(s.x - b * qp.x, s.y - b * qp.y));
+      VTr<VT>::st(vout + r, s);
+      dot += qq.x * s.x + qq.y * s.y;
+    }
+  }
+  block_partial(dot, pdot);
 }
 
 // Several vectors, (Ns, nvec) row-major: a block takes one slice, its entries
@@ -150,7 +230,7 @@ constexpr int PK_STAGE = 32;  // entries per row staged; wider slices read from 
 template <typename VT, int G, int CW, bool EPI>
 __global__ void __launch_bounds__(256) k_packed_mm(HvArgs A) {
   constexpr bool CPLX = VTr<VT>::cplx;
-  using LT = typename std::conditional<CPLX, double2, double>::type;
+  using LT = PkLut<VT>;
   constexpr int U = CW * sizeof(VT) >= 16 ? 4 : 8;
   constexpr int RB = 256 / G;
   __shared__ LT lut[PK_LUT_MAX];
@@ -169,15 +249,12 @@ __global__ void __launch_bounds__(256) k_packed_mm(HvArgs A) {
   const bool staged = wid <= PK_STAGE;
   if (staged)
     for (int i = threadIdx.x; i < wid * 64; i += 256) s_ent[i] = ent[i];
-  for (int i = threadIdx.x; i < A.pk_nlut; i += 256) {
-    if constexpr (CPLX) lut[i] = A.pk_lut[i];
-    else lut[i] = A.pk_lut[i].x;
-  }
+  pk_stage_lut<VT>(A, lut);
   __syncthreads();
   const VT* __restrict__ vin = (const VT*)A.v_in;
   VT* __restrict__ vout = (VT*)A.v_out;
   const int bits = A.pk_bits;
-  const uint32_t cmask = (bits < 32 ? 1u << bits : 0u) - 1u;
+  const uint32_t cmask = (1u << bits) - 1u;
   const int64_t nv = A.nvec;
   const int lane = threadIdx.x % G;
   double maxB = 0.0, maxF = 0.0;

@@ -13,7 +13,7 @@
 #include <string>
 #include <tuple>
 
-#include "sparse_impl.h"
+#include "packed_impl.h"
 
 // ---------------------------------------------------------------------------
 // CSR SpMV dispatch
@@ -561,6 +561,17 @@ __global__ void __launch_bounds__(256) k_lzr_nrm(const double* __restrict__ pdot
     VTr<VT>::st(r + i, rv);
     rv = VTr<VT>::rnd(rv);
     s2 += rv.x * rv.x + rv.y * rv.y;
+  }
+  block_partial(s2, pnrm);
+}
+
+// partials of ||x||^2
+template <typename VT>
+__global__ void __launch_bounds__(256) k_lzr_nrm2(const VT* __restrict__ x, int64_t n, double* __restrict__ pnrm) {
+  double s2 = 0.0;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+    const double2 v = VTr<VT>::ld(x + i);
+    s2 += v.x * v.x + v.y * v.y;
   }
   block_partial(s2, pnrm);
 }
@@ -1644,5 +1655,56 @@ extern "C" int qsx_lanczos_run(int op_kind, void* hv_ctx, const void* indptr, co
     }
   }
   QSX_CHECK_HIP(hipGraphLaunch(it->second.ex, st));
+  return QSX_OK;
+}
+
+// The recurrence of qsx_lanczos_run on an operator's packed rows, two launches
+// per step instead of four: the product with the division by b_{i-1}, the
+// b_{i-1} q_{i-1} subtraction and the partials of a_i (k_packed_lz), then the
+// a_i q_i subtraction and the partials of b_i.  v0 is the start vector (divided
+// by its norm when that is off 1 by more than eps), Q (m, n) with store_Q, else
+// three vectors; r: two vectors; work: QSX_LZ_WORK doubles.  Launched directly:
+// a step is longer than its launches take.  QSX_ERR_UNSUPPORTED, nothing
+// launched: the context is not bound to packed rows.
+constexpr int LZ_MAX_BLOCKS = 2048;
+extern "C" int64_t qsx_lanczos_packed_work(void) { return LZ_MAX_BLOCKS + 2 * 1024; }
+
+extern "C" int qsx_lanczos_packed(const void* hv_ctx, int dtype, int64_t n, int m, const void* v0, double eps, void* Q,
+                                  int store_Q, void* r, double* ab, double* work, void* stream) {
+  if (!hv_ctx || n < 1 || m < 1 || !v0 || !Q || !r || !ab || !work) {
+    qsx_set_error("qsx_lanczos_packed: bad arguments");
+    return QSX_ERR_ARG;
+  }
+  HvArgs A;
+  int dt = -1;
+  int64_t entries = 0;
+  if (!qsx_hv_ctx_packed(hv_ctx, &A, &dt, &entries) || dt != dtype || A.Ns != n || A.nvec != 1) {
+    qsx_set_error("qsx_lanczos_packed: the context is not bound to packed rows of this size");
+    return QSX_ERR_UNSUPPORTED;
+  }
+  hipStream_t st = (hipStream_t)stream;
+  const size_t esz = (dtype == QSX_F32) ? 4 : (dtype == QSX_F64 || dtype == QSX_C64) ? 8 : 16;
+  const int nb = lz_grid(n);
+  const int64_t np = qsx_grid(n, 256);
+  const int nd = (int)(np < LZ_MAX_BLOCKS ? np : LZ_MAX_BLOCKS);
+  double* pdot = work;
+  double* pnrm = work + LZ_MAX_BLOCKS;
+  auto qi = [&](int i) -> void* { return (char*)Q + esz * (size_t)n * (size_t)(store_Q ? i : (i % 3)); };
+  QSX_VT_SWITCH(dtype, hipLaunchKernelGGL(k_lzr_nrm2<VT>, dim3(nb), dim3(256), 0, st, (const VT*)v0, n, pnrm));
+  QSX_LAUNCH_CHECK();
+  for (int i = 0; i < m; ++i) {
+    A.v_in = i == 0 ? v0 : (char*)r + esz * (size_t)n * (size_t)((i - 1) & 1);
+    A.v_out = (char*)r + esz * (size_t)n * (size_t)(i & 1);
+    double* bp = i > 0 ? ab + 4 * (int64_t)(i - 1) + 2 : nullptr;
+    QSX_VT_SWITCH(dtype, hipLaunchKernelGGL(k_packed_lz<VT>, dim3(nd), dim3(256), 0, st, A, (const double*)pnrm, nb,
+                                            (VT*)qi(i), i > 0 ? (const VT*)qi(i - 1) : (const VT*)nullptr, bp, eps,
+                                            i == 0 ? 1 : 0, pdot));
+    QSX_LAUNCH_CHECK();
+    QSX_VT_SWITCH(dtype, hipLaunchKernelGGL(k_lzr_nrm<VT>, dim3(nb), dim3(256), 0, st, (const double*)pdot, nd,
+                                            (const VT*)qi(i), (VT*)A.v_out, n, ab + 4 * (int64_t)i, pnrm));
+    QSX_LAUNCH_CHECK();
+  }
+  hipLaunchKernelGGL(k_lzr_fin, dim3(1), dim3(256), 0, st, (const double*)pnrm, nb, ab + 4 * (int64_t)(m - 1) + 2);
+  QSX_LAUNCH_CHECK();
   return QSX_OK;
 }

@@ -53,6 +53,19 @@ def _device_loop(op, v0, m, dtype, eps, store_Q, Q_out=None):
             if Q_out is not None and not direct:
                 Q = Q_out.copy_(Q)
             return _finish(ab, m, eps, Q)
+        if kind[0] is not None and kind[0].cfg["schedule"] == "packed":
+            # packed rows: normalisation on the device, two launches per step, vectors straight into Q
+            Qb = Q if store_Q else L.empty((min(m, 3), n), dtype)
+            if direct:
+                q0 = q0.clone()  # the start vector may be a row of ``out``
+            r = L.empty((2, n), dtype)
+            work = L.empty(int(lib.qsx_lanczos_packed_work()), np.float64)
+            rc = lib.qsx_lanczos_packed(kind[0].h, code, n, m, ptr(q0), float(eps), ptr(Qb), int(bool(store_Q)),
+                                        ptr(r), ptr(ab), ptr(work), st)
+            L.check(rc, "qsx_lanczos_packed")
+            if Q_out is not None and not direct:
+                Q = Q_out.copy_(Q)
+            return _finish(ab, m, eps, Q)
     q0 = q0.clone()
     qn = nrm2_dev(q0)
     if abs(qn - 1.0) > eps:

@@ -105,3 +105,46 @@ def test_small_packed_rows_match_the_large_path(dtype, monkeypatch):
         got.append((L.to_host(F), E))
     assert np.abs(got[0][0] - got[1][0]).max() <= 200 * EPS[np.dtype(dtype)]
     assert np.abs(got[0][1] - got[1][1]).max() <= 4000 * EPS[np.dtype(dtype)]
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.complex128, np.complex64])
+@pytest.mark.parametrize("blocks,Nup,L_", [(None, 8, 16), ("k", 9, 19), (None, 5, 15), (None, 11, 22)])
+def test_packed_lanczos_two_launches_per_step(dtype, blocks, Nup, L_, monkeypatch):
+    """Sectors above the one-launch sizes (4,862 to 705,432 states; more rows
+    than one round of the capped grid at the largest): a and b, the vectors
+    and lanczos_iter against the host recurrence in 64 bits, and a start
+    vector that is a row of ``out``."""
+    from quspin_amd import _lib as L
+    from quspin_amd.basis import spin_basis_general
+    from quspin_amd.operators import quantum_LinearOperator
+    from quspin_amd.tools.lanczos import _host_loop, lanczos_full, lanczos_iter
+    kw = {"kblock": (chain_maps(L_)["T"], 3)} if blocks else {}
+    if blocks and np.dtype(dtype).kind != "c":
+        return
+    basis = spin_basis_general(L_, Nup=Nup, pauli=0, **kw)
+    h = None if blocks else np.linspace(-1, 1, L_)
+    monkeypatch.setattr("quspin_amd.tuning.time_candidates",
+                        lambda op, ctx, vdt, nvec, reps=5: {"lookup": "search", "schedule": "packed"})
+    monkeypatch.setenv("QSX_TUNE_CACHE", "/nonexistent/tune.json")
+    monkeypatch.setattr("quspin_amd.tuning._mem", {})
+    Q = quantum_LinearOperator(xxz_static(L_, h=h), basis=basis, dtype=dtype, **KW)
+    rng = np.random.default_rng(4)
+    m = 12
+    A = Q._qsx_operator().to_csr(np.complex128).to_scipy()
+    for scale in (1.0, 3.0):
+        x = (scale * _vec(rng, basis.Ns, dtype)).astype(dtype)
+        xd = L.to_device(x)
+        E, V, K = lanczos_full(Q, xd, m)
+        assert Q._qsx_operator().config[(np.dtype(dtype), 1)]["schedule"] == "packed"
+        assert np.array_equal(L.to_host(xd), x)
+        a, b, _, Kh = _host_loop(A, x.astype(np.complex128), m, np.complex128, 0.0)
+        Eh = np.linalg.eigvalsh(np.diag(a) + np.diag(b[:-1], 1) + np.diag(b[:-1], -1))
+        # rounding of a step grows by at most a factor of 8 per step here; two more roundings of q and H q
+        assert np.abs(L.to_host(K)[:5] - Kh[:5]).max() <= 128 * EPS[np.dtype(dtype)] * 8 ** 5
+        assert np.abs(E - Eh).max() <= 400 * EPS[np.dtype(dtype)] * np.abs(Eh).max() * m
+        E2, _ = lanczos_iter(Q, xd, m, return_vec_iter=False)
+        assert np.array_equal(E, E2)
+        out = L.empty((m, basis.Ns), dtype)
+        out[0].copy_(xd)
+        E3, _, K3 = lanczos_full(Q, out[0], m, out=out)
+        assert np.array_equal(E, E3) and np.array_equal(L.to_host(K3), L.to_host(K))
