@@ -200,17 +200,24 @@ def torch():
     return _torch
 
 
+_device_ok = False
+
+
 def require_device():
-    t = torch()
-    if not t.cuda.is_available():
-        raise RuntimeError("quspin_amd needs a ROCm GPU (no CPU fallback exists)")
-    load()
-    return t
+    global _device_ok
+    if not _device_ok:
+        if not torch().cuda.is_available():
+            raise RuntimeError("quspin_amd needs a ROCm GPU (no CPU fallback exists)")
+        load()
+        _device_ok = True
+    return _torch
 
 
 def stream_handle():
     t = torch()
-    return _vp(t.cuda.current_stream().cuda_stream)
+    # the raw handle: a Stream object takes 3-4 us to build, a third of a
+    # product on a small sector
+    return _vp(t._C._cuda_getCurrentRawStream(t.cuda.current_device()))
 
 
 def ptr(x):
@@ -230,20 +237,32 @@ def dtype_code(dt):
     return _NP2CODE[dt]
 
 
-def torch_dtype(dt):
+# numpy dtype -> torch dtype and back, filled once torch is there (a product
+# on a small sector takes less time than building them per call)
+_NP2TORCH = {}
+_TORCH2NP = {}
+
+
+def _dtype_maps():
     t = torch()
-    return {np.dtype(np.float32): t.float32, np.dtype(np.float64): t.float64,
-            np.dtype(np.complex64): t.complex64, np.dtype(np.complex128): t.complex128,
-            np.dtype(np.int32): t.int32, np.dtype(np.int64): t.int64,
-            np.dtype(np.uint8): t.uint8, np.dtype(np.int8): t.int8,
-            np.dtype(np.int16): t.int16}[np.dtype(dt)]
+    _NP2TORCH.update({np.dtype(np.float32): t.float32, np.dtype(np.float64): t.float64,
+                      np.dtype(np.complex64): t.complex64, np.dtype(np.complex128): t.complex128,
+                      np.dtype(np.int32): t.int32, np.dtype(np.int64): t.int64,
+                      np.dtype(np.uint8): t.uint8, np.dtype(np.int8): t.int8,
+                      np.dtype(np.int16): t.int16})
+    _TORCH2NP.update({v: k for k, v in _NP2TORCH.items()})
+
+
+def torch_dtype(dt):
+    if not _NP2TORCH:
+        _dtype_maps()
+    return _NP2TORCH[np.dtype(dt)]
 
 
 def np_dtype(tdt):
-    t = torch()
-    return np.dtype({t.float32: np.float32, t.float64: np.float64, t.complex64: np.complex64,
-                     t.complex128: np.complex128, t.int32: np.int32, t.int64: np.int64,
-                     t.uint8: np.uint8, t.int8: np.int8, t.int16: np.int16}[tdt])
+    if not _TORCH2NP:
+        _dtype_maps()
+    return _TORCH2NP[tdt]
 
 
 def is_device_tensor(x):

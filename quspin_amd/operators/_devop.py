@@ -8,6 +8,7 @@ All arithmetic runs in ``libquspin_hip.so``; torch only holds the buffers.
 """
 
 import ctypes as C
+import math
 
 import numpy as np
 import scipy.sparse as sp
@@ -71,7 +72,7 @@ class DeviceCSR:
         """y = a*A*x (+ y when beta)."""
         vdt = _vec_dtype_code(x)
         mdt = L.dtype_code(self.dtype)
-        nvec = int(np.prod(x.shape[1:])) if x.dim() > 1 else 1
+        nvec = math.prod(x.shape[1:])
         ac = complex(a)
         data = self._data_for(L.np_dtype(x.dtype))
         mdt_use = L.dtype_code(L.np_dtype(data.dtype))
@@ -117,7 +118,7 @@ class DeviceCSR:
     def expm_inplace(self, v, work, s, m_star, tol, mu, a):
         """Taylor loop of ``_wrapper_expm_multiply[_batch]`` on device."""
         vdt = _vec_dtype_code(v)
-        nvec = int(np.prod(v.shape[1:])) if v.dim() > 1 else 1
+        nvec = math.prod(v.shape[1:])
         data = self._data_for(L.np_dtype(v.dtype))
         mdt = L.dtype_code(L.np_dtype(data.dtype))
         mu, a = complex(mu), complex(a)
@@ -236,7 +237,7 @@ class MatrixFreeOp:
 
     def apply(self, x, y, a=1.0, beta=0, a_diag=None):
         vdt = L.np_dtype(x.dtype)
-        nvec = int(np.prod(x.shape[1:])) if x.dim() > 1 else 1
+        nvec = math.prod(x.shape[1:])
         ctx = self._context(vdt, nvec)
         ac = complex(a)
         ad = ac if a_diag is None else complex(a_diag)
@@ -299,7 +300,7 @@ class MatrixFreeOp:
 
     def expm_inplace(self, v, work, s, m_star, tol, mu, a):
         vdt = L.np_dtype(v.dtype)
-        nvec = int(np.prod(v.shape[1:])) if v.dim() > 1 else 1
+        nvec = math.prod(v.shape[1:])
         ctx = self._context(vdt, nvec)
         mu, a = complex(mu), complex(a)
         rc = L.load().qsx_expm_multiply_mf(ctx.h, self.Ns, int(s), int(m_star), float(tol), mu.real, mu.imag,

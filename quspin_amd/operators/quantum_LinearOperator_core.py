@@ -166,6 +166,12 @@ class quantum_LinearOperator(LinearOperator):
         return self._op_for(self._conjugated, self._transposed)
 
     def _apply(self, other, out, a, a_diag, beta):
+        if out is None and L.is_device_tensor(other) and other.is_contiguous() and \
+                L.np_dtype(other.dtype) == self._dtype:
+            # the common case: a device vector of the operator's own dtype
+            y = L.empty(tuple(other.shape), self._dtype)
+            self._qsx_operator().apply(other, y, a=a, beta=beta, a_diag=a_diag)
+            return y
         on_dev = L.is_device_tensor(other)
         odt = L.np_dtype(other.dtype) if on_dev else np.asanyarray(other).dtype
         result_dtype = np.result_type(self._dtype, odt)
