@@ -243,9 +243,14 @@ constexpr int KRON_UP_ROWS = 4;  // up rows per wave in the column-strip pass
 // H_up rows are wave-uniform, read through the scalar cache) and lane l
 // column d = 64 s + l, so every partner-row read is one coalesced segment of
 // the strip; the partner reads of the four rows are issued together.
+//
+// Held to 80 registers (six waves per SIMD) in the fused form for elements of
+// eight bytes or fewer: complex64 with its sum in complex128 needs 84 free.
+// complex128 needs 90, and held to 80 loses 7 % of a driven L = 14 step (5.28
+// -> 5.70 ms), so it keeps five.
 template <typename MT, typename VT, bool EPI, typename FT>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EPI ? 6 : 1))) k_kron_up(KronArgs K, int64_t nunits, int64_t groups,
-                                                 const int32_t* __restrict__ iu, const MT* __restrict__ du) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EPI && sizeof(VT) <= 8 ? 6 : 1)))
+k_kron_up(KronArgs K, int64_t nunits, int64_t groups, const int32_t* __restrict__ iu, const MT* __restrict__ du) {
   constexpr int RW = KRON_UP_ROWS;
   const CsrArgs& A = K.A;
   double2 a_t = A.a, mu_t = A.mu, xs = A.xdscale;
