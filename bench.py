@@ -45,7 +45,9 @@ MEASURED_TRAFFIC = {(28, "table", "rows", "float64"): 68.5e6, (28, "table", "bat
                     (28, "table", "batch14x", "float64"): 45.8e6, (34, "table", "batch14x", "float64"): 7.05e9,
                     (34, "table", "rows", "float64"): 7.42e9, (34, "table", "batch4", "float64"): 7.35e9,
                     (34, "table", "batch8", "float64"): 7.32e9, (34, "table", "batch14", "float64"): 7.30e9,
-                    ("csr", 34, "float64"): 11.99e9}
+                    ("csr", 34, "float64"): 11.99e9,
+                    # packed rows (k_packed_rows): profiles/k_packed_rows_heisenberg_L28_L34_kpz.md
+                    (28, "search", "packed", "float64"): 50.6e6, (34, "table", "packed", "float64"): 6.27e9}
 # The same for the precision workload's term kernels (full launches, per
 # launch): profiles/k_csr_spmv_expm_hubbard_L14_xxz_L28.md
 C3_TRAFFIC = {("mf", "complex64", "rows"): 3.76e9, ("mf", "complex128", "rows"): 7.44e9,
@@ -54,6 +56,22 @@ C3_TRAFFIC = {("mf", "complex64", "rows"): 3.76e9, ("mf", "complex128", "rows"):
 # ... and of one batched H.V of the 26-sector workload (CSR form, all sectors):
 # profiles/k_csr_wave_batched_heisenberg_L26_64vec.md
 C4_TRAFFIC = {("csr", "fp32"): 59.1e9, ("csr", "fp64"): 161.6e9}
+
+
+def hv_limit(L, schedule):
+    """What bounds the matrix-free product, from the profiles."""
+    if schedule == "packed":
+        if L <= 30:
+            return ("gathers of x from a cache-resident vector and one launch's latency: the entries stream once "
+                    "(profiles/k_packed_rows_heisenberg_L28_L34_kpz.md); the HBM-bound size is c2_scaled_L34")
+        return ("L2-miss traffic: the entries stream once, the gathers of x miss L2 "
+                "(profiles/k_packed_rows_heisenberg_L28_L34_kpz.md)")
+    if L <= 30:
+        return ("cache-resident working set: divergent gathers (about one cache line per lane for each applied "
+                "term's table entry and x element) through each CU's vector memory path "
+                "(profiles/k_hv_rows_heisenberg_L28_kpz.md); the HBM-bound size is c2_scaled_L34")
+    return ("L2-miss traffic of the sector-table reads (one 32 B sector per applied term; "
+            "profiles/k_hv_rows_heisenberg_L34_kpz.md)")
 
 
 def chain_static(L, J=1.0, Delta=1.0):
@@ -232,11 +250,7 @@ def main():
                      "frac": round(achieved / HBM_PEAK_GBS, 5), "traffic": traffic,
                      "alg_bytes_per_state": s_i + 1 + 16,
                      "achieved_with_folded_diag": round(achieved_fd, 2),
-                     "limit": ("cache-resident working set: divergent gathers (about one cache line per lane "
-                               "for each applied term's table entry and x element) through each CU's vector "
-                               "memory path; halving the L2 misses (schedule batch14x) leaves the time unchanged "
-                               "(profiles/k_hv_rows_heisenberg_L28_kpz.md); the HBM-bound size is "
-                               "c2_scaled_L34") if L <= 30 else "sector-table reads from HBM"},
+                     "limit": hv_limit(L, cfg.get("schedule"))},
         "cpu_baseline": cpu,
         "lanczos": lz,
         "c2_scaled_L34": scaled,
@@ -249,10 +263,9 @@ def main():
 def run_c2_scaled(steps, L=34):
     """The headline chain at L=34: Sz=0, k=0, p=+1, z=+1 (17,179,435 states,
     64-bit state words; 429 MB of algorithmic bytes per product, above the
-    256 MB MALL).  Matrix-free quantum_LinearOperator.dot (sector table,
-    4-byte entries) and hamiltonian.dot on the device CSR of the same
-    operator, each timed over `steps` launches with HIP events; the two
-    results are compared."""
+    256 MB MALL).  Matrix-free quantum_LinearOperator.dot and hamiltonian.dot
+    on the device CSR of the same operator, each timed over `steps` launches
+    with HIP events; the two results are compared."""
     import time
     import torch
     from quspin_amd.basis import spin_basis_general
@@ -313,8 +326,7 @@ def run_c2_scaled(steps, L=34):
                                         "unit": "GB/s", "frac": round(alg / ms / 1e6 / HBM_PEAK_GBS, 5),
                                         "traffic": traffic, "alg_bytes_per_state": 25,
                                         "achieved_with_folded_diag": round((alg + 8 * Ns) / ms / 1e6, 2),
-                                        "limit": "L2-miss traffic of the sector-table reads (one 32 B sector per "
-                                                 "applied term; profiles/k_hv_rows_heisenberg_L34_kpz.md)"}},
+                                        "limit": hv_limit(L, cfg.get("schedule"))}},
            "csr": {"matvecs_per_s": round(1000.0 / ms_csr, 2), "ms_per_step": round(ms_csr, 5), "nnz": int(M.nnz),
                    "assembly_s": round(t_csr, 3),
                    "roofline": {"bound": "hbm", "achieved": round(alg_csr / ms_csr / 1e6, 2), "peak": HBM_PEAK_GBS,
