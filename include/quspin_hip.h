@@ -157,7 +157,7 @@ int qsx_hv_ctx_set_table(qsx_hv_ctx* ctx, const void* table, int entry_bytes, in
 int qsx_hv_ctx_set_schedule(qsx_hv_ctx* ctx, int sched);
 /* Packed rows: the off-diagonal elements of the context's operator evaluated
  * once, four bytes each (column and coefficient id) in slices of 64 rows.
- * qsx_hv_pack_count (work: device, qsx_hv_pack_work_bytes(Ns) bytes) fills the
+ * qsx_hv_pack_count (work: device, qsx_hv_pack_work_bytes(ctx) bytes) fills the
  * slice offsets off (device int64[(Ns + 63) / 64 + 1]) and gives the number
  * of entries, of coefficients and the column bits; qsx_hv_pack_fill, with the
  * same off and work, writes the entries (device uint32) and the coefficients
@@ -166,7 +166,7 @@ int qsx_hv_ctx_set_schedule(qsx_hv_ctx* ctx, int sched);
  * commute with the group, or too many distinct coefficients).  The buffers
  * serve every context of the same basis, list and flags; the caller keeps
  * them alive while they are bound (ent NULL unbinds). */
-int64_t qsx_hv_pack_work_bytes(int64_t Ns);
+int64_t qsx_hv_pack_work_bytes(const qsx_hv_ctx* ctx);
 int qsx_hv_pack_count(const qsx_hv_ctx* ctx, int64_t* off, void* work, int64_t work_bytes, int64_t* entries,
                       int* n_lut, int* idx_bits, void* stream);
 int qsx_hv_pack_fill(const qsx_hv_ctx* ctx, int64_t* off, void* work, void* ent, void* lut, void* stream);

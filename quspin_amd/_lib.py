@@ -57,7 +57,7 @@ SIGNATURES = {
     "qsx_hv_ctx_set_table": (_i32, [_vp, _vp, _i32, _i32, _vp, _i32]),
     "qsx_hv_ctx_set_diag": (_i32, [_vp, _vp, _i32]),
     "qsx_hv_ctx_set_schedule": (_i32, [_vp, _i32]),
-    "qsx_hv_pack_work_bytes": (_i64, [_i64]),
+    "qsx_hv_pack_work_bytes": (_i64, [_vp]),
     "qsx_hv_pack_count": (_i32, [_vp, _vp, _vp, _i64, C.POINTER(_i64), C.POINTER(_i32), C.POINTER(_i32), _vp]),
     "qsx_hv_pack_fill": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp]),
     "qsx_hv_ctx_set_packed": (_i32, [_vp, _vp, _vp, _i64, _vp, _i32, _i32]),

@@ -172,6 +172,9 @@ __global__ void __launch_bounds__(256) k_packed_rows(HvArgs A) {
 // launch: the partials are summed after the gathers, hidden behind the other
 // blocks' loads.  first: r is the start vector, divided only when its norm is
 // off 1 by more than eps, and no b is recorded.
+// Bound by the gathers of r and, below a few hundred thousand rows, by the two
+// launches of a step.  Heisenberg L = 28 k = 0 p = z = +1, float64, 40 steps:
+// 1,056 us against 1,432 us for product, division and two updates apart.
 template <typename VT>
 __global__ void __launch_bounds__(256) k_packed_lz(HvArgs A, const double* __restrict__ pnrm, int nb,
                                                    VT* __restrict__ q, const VT* __restrict__ qprev, double* bout,

@@ -213,7 +213,7 @@ class MatrixFreeOp:
             self._pk = None
             limit = tuning.packed_limit(self)
             lib = L.load()
-            nwork = lib.qsx_hv_pack_work_bytes(self.Ns)
+            nwork = lib.qsx_hv_pack_work_bytes(ctx.h)
             if nwork > 0 and 4 * self.Ns <= limit:
                 off = L.empty((self.Ns + 63) // 64 + 1, np.int64)
                 work = L.empty((nwork + 7) // 8, np.int64)

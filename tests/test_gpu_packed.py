@@ -199,3 +199,28 @@ def test_packed_taylor_terms(name, nv):
     exact = scipy.linalg.expm(-0.9j * A) @ x
     # unitary, about 30 terms, each rounded once; the largest partial sums are e^|a||A - mu| / 2
     assert np.abs(got - exact).max() <= 1e-12 * np.abs(x).max()
+
+
+@pytest.mark.parametrize("L_", [19, 20])
+def test_packed_elements_kept_or_evaluated_twice(monkeypatch, L_):
+    """Either side of the size up to which a build keeps the evaluated
+    elements (64 MiB at 24 bytes per row and term: 42 MB, 89 MB) gives the
+    product of the general kernel.  Both sum at most 20 products of
+    coefficients 0.5 and unit-scale elements in FP64: 2 x 22 roundings."""
+    from quspin_amd import _lib as L
+    from quspin_amd.basis import spin_basis_general
+    from quspin_amd.operators import quantum_LinearOperator
+    basis = spin_basis_general(L_, Nup=L_ // 2, pauli=0)
+    x = _vec(np.random.default_rng(L_), basis.Ns, 1, np.float64)
+    xd = L.to_device(x)
+    y = {}
+    for sched in ("packed", "rows"):
+        monkeypatch.setenv("QSX_LOOKUP", "search")
+        monkeypatch.setenv("QSX_SCHEDULE", sched)
+        Q = quantum_LinearOperator(xxz_static(L_, Delta=0.7), basis=basis, dtype=np.float64, **KW)
+        y[sched] = L.to_host(Q.dot(xd))
+        op = Q._qsx_operator()
+        assert next(iter(op.config.values()))["schedule"] == sched
+        assert (getattr(op, "_pk", None) is not None) == (sched == "packed")
+    bound = 44 * 2.0 ** -53 * (0.5 * L_ + 0.25 * L_) * np.abs(x).max()
+    assert np.abs(y["packed"] - y["rows"]).max() <= bound
