@@ -5,7 +5,8 @@
 //   off[r / 64] + 64 e + r % 64 :  column | id << idx_bits,
 // id pointing into a table of the operator's distinct coefficients (id 0 = 0,
 // the padding of rows shorter than their slice, which carries the row's own
-// index as its column).  A symmetry-reduced operator has few distinct
+// index as its column; the products take its x for 0, so that a vector element
+// that is not finite stays out of the rows it has no element in).  A symmetry-reduced operator has few distinct
 // coefficients (couplings x characters x ratios of stabiliser sizes), so the
 // table sits in LDS and an element costs four streamed bytes and its gather.
 //
@@ -76,6 +77,21 @@ __device__ __forceinline__ double2 pk_diag(const HvArgs& A, int64_t r) {
                          : ld_stream<double>((const double*)A.diag_arr + r);
 }
 
+// The gathered element of an entry, next to 0 for a row's padding (id 0, whose
+// weight 0 would make a NaN of an element that is not finite): clearing the
+// upper word of a double leaves a subnormal, one select instead of two.
+__device__ __forceinline__ double pk_keep(double v, uint32_t id) {
+  return __hiloint2double(id ? __double2hiint(v) : 0, __double2loint(v));
+}
+__device__ __forceinline__ double2 pk_x(const float* x, uint32_t id) { return make_double2(id ? *x : 0.0f, 0.0); }
+__device__ __forceinline__ double2 pk_x(const double* x, uint32_t id) { return make_double2(pk_keep(*x, id), 0.0); }
+__device__ __forceinline__ double2 pk_x(const float2* x, uint32_t id) {
+  return make_double2(id ? x->x : 0.0f, id ? x->y : 0.0f);
+}
+__device__ __forceinline__ double2 pk_x(const double2* x, uint32_t id) {
+  return make_double2(pk_keep(x->x, id), pk_keep(x->y, id));
+}
+
 // Off-diagonal sum of row rc = 64 sl + lane (the last row for lanes past it):
 // the row's four-byte entries with U gathers in flight.  The rows of a slice
 // are consecutive lanes, so entry loads are 256-byte segments.
@@ -98,8 +114,9 @@ __device__ __forceinline__ double2 pk_row(const HvArgs& A, const PkLut<VT>* lut,
     for (int u = 0; u < U; ++u) xv[u] = vin[ev[u] & cmask];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const double2 x = VTr<VT>::ld(&xv[u]);
-      const PkLut<VT> c = lut[ev[u] >> bits];
+      const uint32_t id = ev[u] >> bits;
+      const double2 x = pk_x(&xv[u], id);
+      const PkLut<VT> c = lut[id];
       if constexpr (VTr<VT>::cplx) acc = cadd(acc, cmul(c, x));
       else acc.x += c * x.x;
     }
@@ -290,10 +307,11 @@ __global__ void __launch_bounds__(256) k_packed_mm(HvArgs A) {
         for (int u = 0; u < U; ++u) xv[u] = *(const VecRun<VT, CW>*)(vin + (int64_t)(ev[u] & cmask) * nv + j);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          const LT m = lut[ev[u] >> bits];
+          const uint32_t id = ev[u] >> bits;
+          const LT m = lut[id];
 #pragma unroll
           for (int c = 0; c < CW; ++c) {
-            const double2 x = VTr<VT>::ld(&xv[u].a[c]);
+            const double2 x = pk_x(&xv[u].a[c], id);
             if constexpr (CPLX) acc[c] = cadd(acc[c], cmul(m, x));
             else acc[c].x += m * x.x;
           }

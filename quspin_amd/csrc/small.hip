@@ -108,11 +108,9 @@ struct PackedRows {
     const uint32_t* e;
     int wid;  // one value per wave: its rows are one slice
     double2 d;
-    uint32_t v[KR];
+    uint32_t v[KR];  // column | id << 16; the padding's column is n, where xs holds a 0
   };
-  __device__ static void mac(double2& acc, uint32_t ev, uint32_t cmask, int bits, const VT* xs, const LT* lut) {
-    const double2 x = VTr<VT>::ld(xs + (ev & cmask));
-    const LT c = lut[ev >> bits];
+  __device__ static void mac(double2& acc, LT c, double2 x) {
     if constexpr (VTr<VT>::cplx) acc = cadd(acc, cmul(c, x));
     else acc.x += c * x.x;
   }
@@ -126,19 +124,25 @@ struct PackedRows {
       else R.d.x = ((const double*)A.diag)[r];
     }
 #pragma unroll
-    for (int u = 0; u < KR; ++u) R.v[u] = u < R.wid ? R.e[u * 64] : (uint32_t)r;
+    for (int u = 0; u < KR; ++u) {
+      const uint32_t ev = u < R.wid ? R.e[u * 64] : 0u, id = ev >> A.bits;
+      R.v[u] = (id ? ev & ((1u << A.bits) - 1u) : (uint32_t)A.n) | id << 16;
+    }
   }
   __device__ static double2 dot(const SmallArgs& A, const Row& R, int r, const VT* xs, const LT* lut) {
     constexpr bool CPLX = VTr<VT>::cplx;
-    const uint32_t cmask = (1u << A.bits) - 1u;
     const double2 xr = VTr<VT>::ld(xs + r);
     double2 acc;
     if constexpr (CPLX) acc = cmul(R.d, xr);
     else acc = make_double2(R.d.x * xr.x, 0.0);
 #pragma unroll
     for (int u = 0; u < KR; ++u)
-      if (u < R.wid) mac(acc, R.v[u], cmask, A.bits, xs, lut);
-    for (int u = KR; u < R.wid; ++u) mac(acc, R.e[u * 64], cmask, A.bits, xs, lut);
+      if (u < R.wid) mac(acc, lut[R.v[u] >> 16], VTr<VT>::ld(xs + (R.v[u] & 0xffffu)));
+    const uint32_t cmask = (1u << A.bits) - 1u;
+    for (int u = KR; u < R.wid; ++u) {
+      const uint32_t ev = R.e[u * 64], id = ev >> A.bits;
+      mac(acc, lut[id], pk_x(xs + (ev & cmask), id));
+    }
     return acc;
   }
 };
@@ -166,6 +170,7 @@ __global__ void __launch_bounds__(SMALL_T) k_small_expm(SmallArgs A) {
   typename OP::Row row[E];
   double2 f[E];
   small_lut<OP>(A, lut);
+  if (threadIdx.x == 0) VTr<VT>::st(xs + n, make_double2(0.0, 0.0));
 #pragma unroll
   for (int e = 0; e < E; ++e) {
     const int i = threadIdx.x + e * nt;
@@ -260,6 +265,7 @@ __global__ void __launch_bounds__(SMALL_T) k_small_lanczos(SmallArgs A) {
   typename OP::Row row[E];
   double2 q[E], qp[E], r[E];
   small_lut<OP>(A, lut);
+  if (threadIdx.x == 0) VTr<VT>::st(xs + n, make_double2(0.0, 0.0));
   int par = 0;
   // block sum in a fixed order; a barrier as max2 above
   auto sum1 = [&](double p) {
@@ -335,7 +341,7 @@ void launch_small(const SmallArgs& A, hipStream_t st) {
   const int E = A.n <= SMALL_T ? 1 : A.n <= 2 * SMALL_T ? 2 : 4;
   int nt = ((A.n + E - 1) / E + 63) / 64 * 64;
   if (nt > SMALL_T) nt = SMALL_T;
-  const size_t lds = (size_t)A.n * sizeof(VT);
+  const size_t lds = (size_t)(A.n + 1) * sizeof(VT);  // the vector and the padding's 0
 #define QSX_SMALL(EE)                                                                             \
   if constexpr (LZ) hipLaunchKernelGGL((k_small_lanczos<OPE<EE>, VT, EE>), dim3(1), dim3(nt), lds, st, A); \
   else hipLaunchKernelGGL((k_small_expm<OPE<EE>, VT, EE>), dim3(1), dim3(nt), lds, st, A)

@@ -224,3 +224,30 @@ def test_packed_elements_kept_or_evaluated_twice(monkeypatch, L_):
         assert (getattr(op, "_pk", None) is not None) == (sched == "packed")
     bound = 44 * 2.0 ** -53 * (0.5 * L_ + 0.25 * L_) * np.abs(x).max()
     assert np.abs(y["packed"] - y["rows"]).max() <= bound
+
+@pytest.mark.parametrize("nv", [1, 3, 8])
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+def test_packed_non_finite_vector(bad, nv):
+    """An element that is not finite reaches the rows that have an element (or
+    a diagonal) in its column, and no padding of its own row makes a NaN of an
+    infinite one."""
+    from quspin_amd import _lib as L
+    from quspin_amd.operators import quantum_LinearOperator
+    basis, static, _ = _case("free")
+    for dtype in (np.float64, np.float32):
+        op = quantum_LinearOperator(static, basis=basis, dtype=dtype, **KW)._qsx_operator()
+        A = op.to_csr(np.float64).to_scipy()
+        # the first row with fewer elements than another of its slice
+        off = np.array([(A.indices[A.indptr[i]:A.indptr[i + 1]] != i).sum() for i in range(basis.Ns)])
+        r = next(i for i in range(basis.Ns) if off[i] < off[i // 64 * 64:i // 64 * 64 + 64].max() and A[i, i] != 0)
+        x = _vec(np.random.default_rng(nv), basis.Ns, nv, dtype)
+        x[r] = bad
+        y = L.empty(x.shape, dtype)
+        op.apply(L.to_device(x), y)
+        assert op.config[(np.dtype(dtype), nv)]["schedule"] == "packed"
+        y = L.to_host(y)
+        hit = np.flatnonzero(A[:, [r]].toarray().ravel())
+        want = bad * np.sign(A[:, [r]].toarray()[hit])
+        np.testing.assert_array_equal(y[hit].reshape(len(hit), -1), np.broadcast_to(want, (len(hit), nv)))
+        rest = np.setdiff1d(np.arange(basis.Ns), hit)
+        assert np.isfinite(y[rest]).all()
