@@ -14,7 +14,7 @@ int qsx_hv_ctx_pack_args(const qsx_hv_ctx* X, HvArgs* A, int* N, int* nmaps, int
 __global__ void __launch_bounds__(256) k_pack_clear(PackDict* D) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i < PK_SLOTS) D->key[i] = 0ull;
-  if (i == 0) { D->n_lut = 0; D->bad = 0; D->total = 0; }
+  if (i == 0) { D->n_lut = 0; D->bad = 0; D->total = 0; D->used = 0; }
 }
 
 // What pass 0 keeps of every element where the work buffer has room: its
@@ -26,7 +26,8 @@ struct PackStash {
 };
 
 // PASS 0: enter every coefficient into the dictionary, off[slice] = 64 x the
-// slice's widest row.  PASS 1: write the entries (ids assigned).
+// slice's widest row.  PASS 1: write the entries (ids assigned).  A row stops
+// at its first element after the build is refused.
 template <typename I, int M, bool FERM, int LK, int PASS>
 __global__ void __launch_bounds__(256) k_pack_rows(HvArgs A, PackDict* D, int64_t* __restrict__ off,
                                                    uint32_t* __restrict__ ent, int bits, PackStash S) {
@@ -48,19 +49,20 @@ __global__ void __launch_bounds__(256) k_pack_rows(HvArgs A, PackDict* D, int64_
     const RowRank rr = row_rank_if<I, LK>(A, sb, s);
     double2 last = make_double2(0.0, 0.0);
     int slot = -1;
-    for (int t = 0; t < A.n_off; ++t) {
+    bool go = true;
+    for (int t = 0; t < A.n_off && go; ++t) {
       term_element<I, M, FERM, LK, true>(A, sb, rr, A.off + t, s, rsq, A.off_conj, [&](int64_t c, double2 coef) {
         if (slot < 0 || coef.x != last.x || coef.y != last.y) {  // neighbouring terms often share the value
           slot = pk_slot(D, coef);
           last = coef;
         }
-        if (slot < 0) { D->bad = 1; return; }
+        if (slot < 0) { go = false; return; }
         if constexpr (PASS == 1) {
           const double2 v = D->val[slot];
           if (v.x != coef.x || v.y != coef.y) D->bad = 1;
           if (k < wid) ent[o0 + (int64_t)k * 64 + lane] = (uint32_t)c | ((uint32_t)D->id[slot] << bits);
         } else if (S.v) {
-          if (k >= A.n_off) { D->bad = 1; return; }
+          if (k >= A.n_off) { D->bad = 1; go = false; return; }
           const int64_t o = (sl * A.n_off + k) * 64 + lane;
           S.v[o] = coef;
           S.cs[o] = make_int2((int)c, slot);

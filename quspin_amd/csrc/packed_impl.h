@@ -19,6 +19,10 @@
 
 constexpr int PK_SLOTS = 4096;   // hash slots of the coefficient dictionary
 constexpr int PK_LUT_MAX = 1024; // distinct coefficients (16 KB of LDS)
+// Probes of a lookup: with at most a quarter of the slots taken, linear
+// probing's longest chain is about 13, so 64 are only reached once more values
+// came in than the form takes.
+constexpr int PK_PROBES = 64;
 
 // dictionary scratch of a build, in device memory
 struct PackDict {
@@ -26,8 +30,9 @@ struct PackDict {
   double2 val[PK_SLOTS];
   int32_t id[PK_SLOTS];
   int32_t n_lut;      // entries with id 0
-  int32_t bad;        // dictionary full, or two values with one hash
+  int32_t bad;        // refused: too many values, or two with one hash
   int64_t total;      // entries of all slices
+  int32_t used;       // slots taken
 };
 
 __device__ __forceinline__ unsigned long long pk_hash(double2 v) {
@@ -40,19 +45,27 @@ __device__ __forceinline__ unsigned long long pk_hash(double2 v) {
   return h | 1ull;
 }
 
-// Slot of value v, entered when it is new; -1 when every slot is taken.
+// Slot of value v, entered when it is new; -1 when the build is refused
+// already, or by this value.  An operator of many distinct couplings would
+// otherwise pay a walk over the full table for every further element.
 __device__ __forceinline__ int pk_slot(PackDict* D, double2 v) {
   const unsigned long long h = pk_hash(v);
   int s = (int)(h >> 1) & (PK_SLOTS - 1);
-  for (int p = 0; p < PK_SLOTS; ++p) {
+  if (__hip_atomic_load(&D->bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return -1;
+  for (int p = 0; p < PK_PROBES; ++p) {
     unsigned long long k = __hip_atomic_load(&D->key[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (k == 0) {
       k = atomicCAS(&D->key[s], 0ull, h);
-      if (k == 0) { D->val[s] = v; return s; }
+      if (k == 0) {
+        D->val[s] = v;
+        if (atomicAdd(&D->used, 1) < PK_LUT_MAX - 1) return s;  // id 0 is the padding's
+        break;
+      }
     }
     if (k == h) return s;
     s = (s + 1) & (PK_SLOTS - 1);
   }
+  __hip_atomic_store(&D->bad, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   return -1;
 }
 

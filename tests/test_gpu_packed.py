@@ -131,23 +131,55 @@ def test_packed_flags(name, transposed, conjugated):
         _check(L.to_host(y), A, x, 1.0, None, np.complex128)
 
 
-def test_packed_dictionary_overflow_takes_the_general_kernels():
-    """More distinct coefficients than the dictionary holds: refused, and the
-    product runs as it did."""
+def _distinct_four_body(L):
+    """Every four-site coupling of six strings with a value of its own."""
     from itertools import combinations
-    from quspin_amd import _lib as L
-    from quspin_amd.basis import spin_basis_general
-    from quspin_amd.operators import quantum_LinearOperator
-    basis = spin_basis_general(10, pauli=0)
     J = 1.0
     static = []
     for opstr in ("xxxx", "xxxz", "xxzz", "zxxx", "xzzx", "zxzx"):
         bonds = []
-        for sites in combinations(range(10), 4):
+        for sites in combinations(range(L), 4):
             J += 0.001
             bonds.append([J] + list(sites))
         static.append([opstr, bonds])
-    Q = quantum_LinearOperator(static, basis=basis, dtype=np.float64, **KW)
+    return static
+
+
+def test_packed_build_stops_when_the_dictionary_is_full():
+    """More values (2,970 couplings, 5,445 with signs) than the dictionary has
+    slots: the rows stop soon after the 1,023rd value, about a quarter of the
+    way through the terms, and the operator is refused."""
+    from quspin_amd import _lib as L
+    from quspin_amd.basis import spin_basis_general
+    from quspin_amd.operators import quantum_LinearOperator
+    basis = spin_basis_general(12, pauli=0)
+    op = quantum_LinearOperator(_distinct_four_body(12), basis=basis, dtype=np.float64, **KW)._qsx_operator()
+    ctx = op._new_ctx(np.dtype(np.float64), 1)
+    lib = L.load()
+    nwork = lib.qsx_hv_pack_work_bytes(ctx.h)
+    nsl = basis.Ns // 64
+    off, work = L.empty(nsl + 1, np.int64), L.empty((nwork + 7) // 8, np.int64)
+    ent, nl, bits = L._i64(), L._i32(), L._i32()
+    rc = lib.qsx_hv_pack_count(ctx.h, L.ptr(off), L.ptr(work), nwork, L.C.byref(ent), L.C.byref(nl), L.C.byref(bits),
+                               L.stream_handle())
+    assert rc == L.QSX_ERR_UNSUPPORTED
+    widths = np.diff(L.to_host(off)) // 64
+    assert op.oplist.n_off == 2970 and widths.min() >= 0 and widths.max() <= 1500
+    x = _vec(np.random.default_rng(0), basis.Ns, 1, np.float64)
+    y = L.empty(x.shape, np.float64)
+    op.apply(L.to_device(x), y)
+    assert op._pk is None
+    _check(L.to_host(y), op.to_csr().to_scipy(), x, 1.0, None, np.float64)
+
+
+def test_packed_dictionary_overflow_takes_the_general_kernels():
+    """More distinct coefficients (1,260) than the form takes (1,023): refused,
+    and the product runs as it did."""
+    from quspin_amd import _lib as L
+    from quspin_amd.basis import spin_basis_general
+    from quspin_amd.operators import quantum_LinearOperator
+    basis = spin_basis_general(10, pauli=0)
+    Q = quantum_LinearOperator(_distinct_four_body(10), basis=basis, dtype=np.float64, **KW)
     op = Q._qsx_operator()
     x = _vec(np.random.default_rng(0), basis.Ns, 1, np.float64)
     y = L.empty(x.shape, np.float64)
