@@ -336,19 +336,35 @@ __global__ void __launch_bounds__(SMALL_T) k_small_lanczos(SmallArgs A) {
   }
 }
 
+// LDS a workgroup of the current device may take: complex128 Lanczos above
+// 3,056 rows asks for more than 64 KB.
+size_t lds_limit() {
+  int dev = 0, v = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
+    return 65536;
+  return (size_t)v;
+}
+
+// False, nothing launched: more LDS than the device has for a workgroup, or
+// more rows than the form takes.
 template <template <int> class OPE, typename VT, bool LZ, bool FOUR>
-void launch_small(const SmallArgs& A, hipStream_t st) {
+bool launch_small(const SmallArgs& A, hipStream_t st) {
   const int E = A.n <= SMALL_T ? 1 : A.n <= 2 * SMALL_T ? 2 : 4;
   int nt = ((A.n + E - 1) / E + 63) / 64 * 64;
   if (nt > SMALL_T) nt = SMALL_T;
   const size_t lds = (size_t)(A.n + 1) * sizeof(VT);  // the vector and the padding's 0
+  constexpr size_t fixed = sizeof(typename OPE<1>::LT) * OPE<1>::LUT + (LZ ? 2 : 4) * sizeof(double) * (SMALL_T / 64);
+  if (lds + fixed > 65536 && lds + fixed > lds_limit()) return false;
 #define QSX_SMALL(EE)                                                                             \
   if constexpr (LZ) hipLaunchKernelGGL((k_small_lanczos<OPE<EE>, VT, EE>), dim3(1), dim3(nt), lds, st, A); \
   else hipLaunchKernelGGL((k_small_expm<OPE<EE>, VT, EE>), dim3(1), dim3(nt), lds, st, A)
   if (E == 1) { QSX_SMALL(1); }
   else if (E == 2) { QSX_SMALL(2); }
   else if constexpr (FOUR) { QSX_SMALL(4); }
+  else return false;
 #undef QSX_SMALL
+  return true;
 }
 
 template <typename MT, typename VT>
@@ -362,23 +378,22 @@ struct PackedOf {
 
 template <bool LZ>
 bool launch_small_csr(const SmallArgs& A, int mdt, int vdt, hipStream_t st) {
-  if (vdt == QSX_F32 && mdt == QSX_F32) launch_small<CsrOf<float, float>::template Op, float, LZ, false>(A, st);
-  else if (vdt == QSX_F64 && mdt == QSX_F64) launch_small<CsrOf<double, double>::template Op, double, LZ, false>(A, st);
-  else if (vdt == QSX_C64 && mdt == QSX_F32) launch_small<CsrOf<float, float2>::template Op, float2, LZ, false>(A, st);
-  else if (vdt == QSX_C64 && mdt == QSX_C64) launch_small<CsrOf<float2, float2>::template Op, float2, LZ, false>(A, st);
-  else if (vdt == QSX_C128 && mdt == QSX_F64) launch_small<CsrOf<double, double2>::template Op, double2, LZ, false>(A, st);
-  else if (vdt == QSX_C128 && mdt == QSX_C128) launch_small<CsrOf<double2, double2>::template Op, double2, LZ, false>(A, st);
-  else return false;
-  return true;
+  if (vdt == QSX_F32 && mdt == QSX_F32) return launch_small<CsrOf<float, float>::template Op, float, LZ, false>(A, st);
+  if (vdt == QSX_F64 && mdt == QSX_F64) return launch_small<CsrOf<double, double>::template Op, double, LZ, false>(A, st);
+  if (vdt == QSX_C64 && mdt == QSX_F32) return launch_small<CsrOf<float, float2>::template Op, float2, LZ, false>(A, st);
+  if (vdt == QSX_C64 && mdt == QSX_C64) return launch_small<CsrOf<float2, float2>::template Op, float2, LZ, false>(A, st);
+  if (vdt == QSX_C128 && mdt == QSX_F64) return launch_small<CsrOf<double, double2>::template Op, double2, LZ, false>(A, st);
+  if (vdt == QSX_C128 && mdt == QSX_C128) return launch_small<CsrOf<double2, double2>::template Op, double2, LZ, false>(A, st);
+  return false;
 }
 
 template <bool LZ>
 bool launch_small_packed(const SmallArgs& A, int vdt, hipStream_t st) {
   switch (vdt) {
-    case QSX_F32: launch_small<PackedOf<float>::template Op, float, LZ, LZ>(A, st); return true;
-    case QSX_F64: launch_small<PackedOf<double>::template Op, double, LZ, LZ>(A, st); return true;
-    case QSX_C64: launch_small<PackedOf<float2>::template Op, float2, LZ, LZ>(A, st); return true;
-    case QSX_C128: launch_small<PackedOf<double2>::template Op, double2, LZ, LZ>(A, st); return true;
+    case QSX_F32: return launch_small<PackedOf<float>::template Op, float, LZ, LZ>(A, st);
+    case QSX_F64: return launch_small<PackedOf<double>::template Op, double, LZ, LZ>(A, st);
+    case QSX_C64: return launch_small<PackedOf<float2>::template Op, float2, LZ, LZ>(A, st);
+    case QSX_C128: return launch_small<PackedOf<double2>::template Op, double2, LZ, LZ>(A, st);
     default: return false;
   }
 }
