@@ -376,7 +376,8 @@ int qsx_lanczos_packed(const void* hv_ctx, int dtype, int64_t n, int m, const vo
  * into ab as there, q_0 .. q_{m-1} into Q (m, n) unless Q is NULL.
  * QSX_ERR_UNSUPPORTED, nothing launched: an assembled matrix of more than
  * 2,048 rows or 24,576 entries, a context of more than 4,096 rows or 49,152
- * packed elements or not bound to packed rows. */
+ * packed elements (above 2,048 rows: 32,768 real, 20,480 complex) or not bound
+ * to packed rows, or more LDS than the device has for a workgroup. */
 int qsx_lanczos_small(int op_kind, const void* hv_ctx, const void* indptr, const void* indices, const void* data,
                       int idx64, int mat_dtype, int64_t nnz, int dtype, int64_t n, int m, const void* v0, double eps,
                       void* Q, double* ab, void* stream);

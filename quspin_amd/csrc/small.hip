@@ -16,15 +16,22 @@
 namespace {
 
 constexpr int SMALL_T = 1024;  // threads
-// Sizes up to which one workgroup wins over a launch per term or step; a row
-// beyond a thread's second leaves too few registers for its elements.
-// Measured on XXZ sectors without symmetries, t = 1 steps (about 65 terms) and
-// 30 Lanczos steps, launches -> one workgroup:
+// Sizes up to which one workgroup wins over a launch per term or two per step;
+// a row beyond a thread's second leaves too few registers for its elements.
+// Measured on sectors without symmetries, t = 1 steps (about 65 terms) and 30
+// Lanczos steps, launches -> one workgroup:
 //   assembled     924 rows 593 -> 215 us, 1,716 rows 607 -> 424, 3,432 rows 617 -> 985
 //   packed rows   924 rows 423 -> 225 us, 1,716 rows 450 -> 292, 3,432 rows 450 -> 642
-//   Lanczos, packed 924 rows 591 -> 229 us, 3,432 rows 602 -> 370 (a step is four launches)
+//   Lanczos, packed, rows / entries, float64 and complex128:
+//     924 / 9,216     302 -> 109 us, 310 -> 118     2,002 / 34,560  337 -> 178, 336 -> 211
+//     3,876 / 30,592  255 -> 202,    254 -> 268     4,060 / 24,576  251 -> 177, 285 -> 236
+//     3,432 / 36,224  262 -> 249,    268 -> 312     3,060 / 46,848  318 -> 309, 308 -> 365
+//   float32 and complex64 at the last three: 255 -> 192 us, 290 -> 310;
+//   266 -> 278, 288 -> 425; 309 -> 338, 328 -> 499 (two rows per thread, 2,002
+//   / 34,560: 309 -> 193, 368 -> 258)
 constexpr int SMALL_N = 2048, SMALL_NNZ = 24576;
-constexpr int SMALL_N_LZ = 4096, SMALL_NNZ_LZ = 49152;  // Lanczos on packed rows
+// Lanczos on packed rows: up to two rows per thread, and up to four
+constexpr int SMALL_N_LZ = 4096, SMALL_NNZ_LZ = 49152, SMALL_NNZ_LZ4 = 32768, SMALL_NNZ_LZ4_CPLX = 20480;
 
 struct SmallArgs {
   // CSR form
@@ -412,7 +419,13 @@ bool ctx_args(const void* hv_ctx, bool lanczos, SmallArgs& A, int& dtype) {
   HvArgs H;
   int64_t entries = 0;
   if (!qsx_hv_ctx_packed(hv_ctx, &H, &dtype, &entries)) return false;
-  if (lanczos ? H.Ns < 1 || H.Ns > SMALL_N_LZ || entries > SMALL_NNZ_LZ : !small_size(H.Ns, entries)) return false;
+  if (lanczos) {
+    const bool cplx = dtype == QSX_C64 || dtype == QSX_C128;
+    const int64_t most = H.Ns <= 2 * SMALL_T ? SMALL_NNZ_LZ : cplx ? SMALL_NNZ_LZ4_CPLX : SMALL_NNZ_LZ4;
+    if (H.Ns < 1 || H.Ns > SMALL_N_LZ || entries > most) return false;
+  } else if (!small_size(H.Ns, entries)) {
+    return false;
+  }
   std::memset(&A, 0, sizeof(A));
   A.off = H.pk_off; A.ent = H.pk_ent; A.lut = H.pk_lut; A.n_lut = H.pk_nlut; A.bits = H.pk_bits;
   A.diag = H.diag_arr; A.diag_cplx = H.diag_arr_cplx;

@@ -144,6 +144,27 @@ def test_small_lanczos_packed_rows_per_thread(dtype, L_, Nup, monkeypatch):
     assert np.abs(E - Eh).max() <= 200 * EPS[np.dtype(dtype)] * np.abs(Eh).max() * m
 
 
+@pytest.mark.parametrize("dtype,small", [(np.float64, True), (np.float32, True), (np.complex128, False),
+                                         (np.complex64, False)])
+def test_small_lanczos_limit_by_type(dtype, small, monkeypatch):
+    """3,876 rows of at most 8 elements (30,592 in slices): one launch in real
+    types, two per step in complex ones, and the same tridiagonal matrix."""
+    from quspin_amd import _lib as L
+    from quspin_amd.basis import spin_basis_general
+    from quspin_amd.operators import quantum_LinearOperator
+    from quspin_amd.tools.lanczos import _host_loop, lanczos_iter
+    basis = spin_basis_general(19, Nup=4, pauli=0)
+    Q = quantum_LinearOperator(xxz_static(19), basis=basis, dtype=dtype, **KW)
+    A = Q._qsx_operator().to_csr(np.complex128).to_scipy()
+    x = _vec(np.random.default_rng(5), basis.Ns, dtype)
+    codes, m = _small_codes(monkeypatch), 10
+    E, V = lanczos_iter(Q, L.to_device(x), m, return_vec_iter=False)
+    assert codes == [L.QSX_OK if small else L.QSX_ERR_UNSUPPORTED]
+    a, b, _, _ = _host_loop(A, x.astype(np.complex128), m, np.complex128, 0.0)
+    Eh = np.linalg.eigvalsh(np.diag(a) + np.diag(b[:-1], 1) + np.diag(b[:-1], -1))
+    assert np.abs(E - Eh).max() <= 400 * EPS[np.dtype(dtype)] * np.abs(Eh).max() * m
+
+
 @pytest.mark.parametrize("dtype", [np.float64, np.complex128, np.complex64])
 @pytest.mark.parametrize("blocks,Nup,L_", [(None, 8, 16), ("k", 9, 19), (None, 6, 15), (None, 11, 22)])
 def test_packed_lanczos_two_launches_per_step(dtype, blocks, Nup, L_, monkeypatch):
