@@ -9,6 +9,7 @@ All arithmetic runs in ``libquspin_hip.so``; torch only holds the buffers.
 
 import ctypes as C
 import math
+import threading
 
 import numpy as np
 import scipy.sparse as sp
@@ -129,21 +130,37 @@ class DeviceCSR:
         L.check(rc, "qsx_expm_multiply_csr")
 
 
+class _PackedRows:
+    """Packed rows of one operator list and pair of flags on one basis:
+    ``held`` is (offsets, entries, coefficients, column bits), or None while
+    they are not built and where there are none."""
+
+    def __init__(self):
+        self.lock = threading.Lock()
+        self.tried = False
+        self.held = None
+
+
 class MatrixFreeOp:
     """Fused matrix-free H.v over a device basis and operator list.
 
     ``transposed``/``conjugated`` act on the off-diagonal terms, ``diag_conj``
-    on the diagonal terms; ``diag`` is an optional extra device diagonal."""
+    on the diagonal terms; ``diag`` is an optional extra device diagonal.
+    ``rows``: packed rows by flags, a dict shared by the operators of one list
+    (an adjoint made for one product does not evaluate the elements again)."""
 
     is_matrix_free = True
 
-    def __init__(self, basis, oplist, dtype, transposed=False, conjugated=False, diag_conj=False, diag=None):
+    def __init__(self, basis, oplist, dtype, transposed=False, conjugated=False, diag_conj=False, diag=None,
+                 rows=None):
         self.basis = basis
         self.oplist = oplist
         self.dtype = np.dtype(dtype)
         self.transposed, self.conjugated, self.diag_conj = bool(transposed), bool(conjugated), bool(diag_conj)
         self.diag = diag
         self._ctx = {}
+        self._rows = {} if rows is None else rows
+        self._packed_rows = self._rows.setdefault((self.transposed, self.conjugated), _PackedRows())
         self.shape = (basis.Ns, basis.Ns)
 
     @property
@@ -204,31 +221,48 @@ class MatrixFreeOp:
     def _configure(self, ctx, cfg):
         ctx.configure(cfg, self.basis, self._packed(ctx) if cfg.get("schedule") == "packed" else None)
 
+    def adjoint(self):
+        return MatrixFreeOp(self.basis, self.oplist, self.dtype, transposed=not self.transposed,
+                            conjugated=not self.conjugated, diag_conj=not self.diag_conj, diag=self.diag,
+                            rows=self._rows)
+
+    @property
+    def _pk(self):
+        return self._packed_rows.held
+
     def _packed(self, ctx):
         """The operator's packed rows (offsets, entries, coefficients, column
         bits), evaluated once through ``ctx`` (``qsx_hv_pack_*``) and shared
         by its contexts; None when it has none or they would take more than
         ``tuning.packed_limit`` bytes."""
-        if not hasattr(self, "_pk"):
-            self._pk = None
-            limit = tuning.packed_limit(self)
-            lib = L.load()
-            nwork = lib.qsx_hv_pack_work_bytes(ctx.h)
-            if nwork > 0 and 4 * self.Ns <= limit:
-                off = L.empty((self.Ns + 63) // 64 + 1, np.int64)
-                work = L.empty((nwork + 7) // 8, np.int64)
-                ent, nl, bits = L._i64(), L._i32(), L._i32()
-                rc = lib.qsx_hv_pack_count(ctx.h, ptr(off), ptr(work), nwork, C.byref(ent), C.byref(nl),
-                                           C.byref(bits), stream_handle())
-                if rc == L.QSX_OK and 4 * ent.value <= limit:
-                    entries = L.empty(max(ent.value, 1), np.int32)
-                    lut = L.empty(nl.value, np.complex128)
-                    rc = lib.qsx_hv_pack_fill(ctx.h, ptr(off), ptr(work), ptr(entries), ptr(lut), stream_handle())
-                    if rc == L.QSX_OK:
-                        self._pk = (off, entries, lut, bits.value)
-                if rc != L.QSX_ERR_UNSUPPORTED:
-                    L.check(rc, "qsx_hv_pack")
-        return self._pk
+        P = self._packed_rows
+        with P.lock:
+            if not P.tried:
+                P.held = self._build_packed(ctx)
+                P.tried = True
+            return P.held
+
+    def _build_packed(self, ctx):
+        limit = tuning.packed_limit(self)
+        lib = L.load()
+        nwork = lib.qsx_hv_pack_work_bytes(ctx.h)
+        if nwork <= 0 or 4 * self.Ns > limit:
+            return None
+        off = L.empty((self.Ns + 63) // 64 + 1, np.int64)
+        work = L.empty((nwork + 7) // 8, np.int64)
+        ent, nl, bits = L._i64(), L._i32(), L._i32()
+        rc = lib.qsx_hv_pack_count(ctx.h, ptr(off), ptr(work), nwork, C.byref(ent), C.byref(nl), C.byref(bits),
+                                   stream_handle())
+        if rc == L.QSX_OK:
+            if 4 * ent.value > limit:
+                return None
+            entries = L.empty(max(ent.value, 1), np.int32)
+            lut = L.empty(nl.value, np.complex128)
+            rc = lib.qsx_hv_pack_fill(ctx.h, ptr(off), ptr(work), ptr(entries), ptr(lut), stream_handle())
+        if rc == L.QSX_ERR_UNSUPPORTED:
+            return None
+        L.check(rc, "qsx_hv_pack")
+        return off, entries, lut, bits.value
 
     @property
     def config(self):

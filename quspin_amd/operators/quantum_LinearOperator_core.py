@@ -73,7 +73,7 @@ class quantum_LinearOperator(LinearOperator):
         self._public_static_list = list(static_list)
         self._static_list = _consolidate_static(static_list)
         self._oplist = self._basis._compile_oplist(self._static_list)
-        self._ops = {}
+        self._ops, self._rows = {}, {}
 
     # -------------------------------------------------------------- props
     @property
@@ -138,7 +138,7 @@ class quantum_LinearOperator(LinearOperator):
             off = [t for t in self._static_list if not self._diagonal_term(*t)]
             self._static_list = off
             self._oplist = self._basis._compile_oplist(off)
-        self._ops = {}
+        self._ops, self._rows = {}, {}
 
     def _diagonal_term(self, opstr, indx, J):
         """True for a term that changes no state (its flips cancel), which
@@ -157,7 +157,8 @@ class quantum_LinearOperator(LinearOperator):
         key = (bool(transposed), bool(conjugated))
         if key not in self._ops:
             self._ops[key] = MatrixFreeOp(self._basis, self._oplist, self._dtype, transposed=key[0],
-                                          conjugated=key[1], diag_conj=False, diag=self._user_diag)
+                                          conjugated=key[1], diag_conj=False, diag=self._user_diag,
+                                          rows=self._rows)
         return self._ops[key]
 
     def _qsx_operator(self):
@@ -230,6 +231,8 @@ class quantum_LinearOperator(LinearOperator):
 
     # ------------------------------------------------------- transforms
     def _copy_flags(self):
+        # contexts are the copy's own (their scratch may be in use by another
+        # thread); the packed rows of the shared term list are not (``_rows``)
         new = object.__new__(quantum_LinearOperator)
         new.__dict__.update(self.__dict__)
         new._ops = {}

@@ -29,7 +29,7 @@ class LazyOperatorNormInfo:
 
     def __init__(self, op, A_1_norm, a, mu, dtype, ell=2, adjoint=None):
         self._op = op
-        self._adj = adjoint
+        self._adj, self._adj_op = adjoint, None
         self._a = a
         self._mu = mu
         self._dtype = np.dtype(dtype)
@@ -52,7 +52,9 @@ class LazyOperatorNormInfo:
     @property
     def linear_operator(self):
         a, mu = self._a, self._mu
-        adj = self._adj() if self._adj is not None else None
+        if self._adj_op is None and self._adj is not None:
+            self._adj_op = self._adj()
+        adj = self._adj_op
         return LinearOperator(
             self._op.shape, dtype=self._dtype,
             matvec=lambda v: self._mv(self._op, v, a, mu),
@@ -141,8 +143,7 @@ class expm_multiply_parallel:
     def _adjoint(self):
         op = self._op
         if isinstance(op, MatrixFreeOp):
-            return MatrixFreeOp(op.basis, op.oplist, op.dtype, transposed=not op.transposed,
-                                conjugated=not op.conjugated, diag_conj=not op.diag_conj, diag=op.diag)
+            return op.adjoint()
         if not hasattr(self, "_adj_csr"):
             self._adj_csr = csr_transpose(op, conj=True)
         return self._adj_csr

@@ -4,6 +4,7 @@ bases, operator strings, flags and scales the product takes."""
 
 import numpy as np
 import pytest
+import scipy.sparse as sp
 
 from models import chain_maps, hubbard_static, ladder_maps, xxz_static
 
@@ -283,3 +284,53 @@ def test_packed_non_finite_vector(bad, nv):
         np.testing.assert_array_equal(y[hit].reshape(len(hit), -1), np.broadcast_to(want, (len(hit), nv)))
         rest = np.setdiff1d(np.arange(basis.Ns), hit)
         assert np.isfinite(y[rest]).all()
+
+
+def _count_builds(monkeypatch):
+    from quspin_amd import _lib as L
+    lib, calls = L.load(), []
+    f = lib.qsx_hv_pack_count
+    monkeypatch.setattr(lib, "qsx_hv_pack_count", lambda *a: (calls.append(1), f(*a))[1])
+    return calls
+
+
+def test_packed_rows_shared_by_adjoints_and_copies(monkeypatch):
+    """``rmatvec``, ``.H``, ``.T`` and copies evaluate the elements once per
+    pair of flags; a replaced diagonal starts anew and leaves copies alone."""
+    from quspin_amd import _lib as L
+    from quspin_amd.operators import quantum_LinearOperator
+    basis, static, _ = _case("momentum")
+    calls = _count_builds(monkeypatch)
+    Q = quantum_LinearOperator(static, basis=basis, dtype=np.complex128, **KW)
+    A = Q._qsx_operator().to_csr().to_scipy()
+    x = _vec(np.random.default_rng(8), basis.Ns, 1, np.complex128)
+    xd = L.to_device(x)
+    for _ in range(20):  # long enough to have built whatever it builds
+        _check(L.to_host(Q.dot(xd)), A, x, 1.0, None, np.complex128)
+        _check(Q.rmatvec(x), A.conj().T.tocsr(), x, 1.0, None, np.complex128)
+        _check(L.to_host(Q.H.dot(xd)), A.conj().T.tocsr(), x, 1.0, None, np.complex128)
+        _check(L.to_host(Q.copy().dot(xd)), A, x, 1.0, None, np.complex128)
+    assert len(calls) <= 2 and Q._op_for(False, False)._pk is not None
+    for _ in range(20):
+        Q.T.dot(xd)
+    assert len(calls) <= 3
+    C = Q.copy()
+    Q.set_diagonal(np.ones(basis.Ns))
+    _check(L.to_host(C.dot(xd)), A, x, 1.0, None, np.complex128)
+    hops = quantum_LinearOperator(static[:2], basis=basis, dtype=np.complex128, **KW)
+    D = hops._qsx_operator().to_csr().to_scipy() + sp.identity(basis.Ns)
+    _check(L.to_host(Q.dot(xd)), D.tocsr(), x, 1.0, None, np.complex128)
+
+
+def test_packed_norm_estimates_share_the_adjoint(monkeypatch):
+    """The partition of a Taylor loop estimates 1-norms of several powers: one
+    build for the operator and one for its adjoint, also for a second ``a``."""
+    from quspin_amd.operators import quantum_LinearOperator
+    from quspin_amd.tools.evolution import expm_multiply_parallel
+    basis, static, _ = _case("momentum")
+    calls = _count_builds(monkeypatch)
+    Q = quantum_LinearOperator(static, basis=basis, dtype=np.complex128, **KW)
+    E = expm_multiply_parallel(Q, a=-20.0j)
+    E.set_a(-35.0j)
+    expm_multiply_parallel(Q, a=-30.0j)
+    assert 1 <= len(calls) <= 2
