@@ -10,6 +10,7 @@ All arithmetic runs in ``libquspin_hip.so``; torch only holds the buffers.
 import ctypes as C
 import math
 import threading
+import weakref
 
 import numpy as np
 import scipy.sparse as sp
@@ -130,6 +131,19 @@ class DeviceCSR:
         L.check(rc, "qsx_expm_multiply_csr")
 
 
+_rows_lock = threading.RLock()
+
+
+def _rows_budget(basis):
+    """[bytes of packed rows held on this basis]"""
+    return basis.__dict__.setdefault("_packed_held", [0])
+
+
+def _rows_release(budget, nbytes):
+    with _rows_lock:
+        budget[0] -= nbytes
+
+
 class _PackedRows:
     """Packed rows of one operator list and pair of flags on one basis:
     ``held`` is (offsets, entries, coefficients, column bits), or None while
@@ -139,6 +153,17 @@ class _PackedRows:
         self.lock = threading.Lock()
         self.tried = False
         self.held = None
+
+    def reserve(self, basis, nbytes):
+        """Whether the rows of all operators on the basis, these with them,
+        stay within ``tuning.packed_total``; counted until these are freed."""
+        budget = _rows_budget(basis)
+        with _rows_lock:
+            if budget[0] + nbytes > tuning.packed_total(basis):
+                return False
+            budget[0] += nbytes
+        weakref.finalize(self, _rows_release, budget, nbytes)
+        return True
 
 
 class MatrixFreeOp:
@@ -233,12 +258,16 @@ class MatrixFreeOp:
     def _packed(self, ctx):
         """The operator's packed rows (offsets, entries, coefficients, column
         bits), evaluated once through ``ctx`` (``qsx_hv_pack_*``) and shared
-        by its contexts; None when it has none or they would take more than
-        ``tuning.packed_limit`` bytes."""
+        by its contexts; None when it has none, when they would take more than
+        ``tuning.packed_limit`` bytes (``packed_total`` with the others of the
+        basis) or when the device has no memory for them."""
         P = self._packed_rows
         with P.lock:
             if not P.tried:
-                P.held = self._build_packed(ctx)
+                try:
+                    P.held = self._build_packed(ctx)
+                except L.torch().OutOfMemoryError:
+                    P.held = None  # the other forms need no memory of their own
                 P.tried = True
             return P.held
 
@@ -254,7 +283,7 @@ class MatrixFreeOp:
         rc = lib.qsx_hv_pack_count(ctx.h, ptr(off), ptr(work), nwork, C.byref(ent), C.byref(nl), C.byref(bits),
                                    stream_handle())
         if rc == L.QSX_OK:
-            if 4 * ent.value > limit:
+            if 4 * ent.value > limit or not self._packed_rows.reserve(self.basis, 4 * ent.value):
                 return None
             entries = L.empty(max(ent.value, 1), np.int32)
             lut = L.empty(nl.value, np.complex128)

@@ -35,8 +35,9 @@ _mem = {}
 SCHEDULES = {"rows": 0, "queue": 1, "rows2": 2, "rows4": 3, "rows8": 4, "batch4": 5, "batch8": 6, "split": 7,
              "chunk4": 8, "chunk8": 9, "batch14": 10, "split2": 11, "batch14x": 12, "packed": 13}
 
-# packed rows of sectors without symmetry maps, and of small sectors
-PACKED_BYTES = 64 << 20
+# packed rows of sectors without symmetry maps, and of small sectors: of one
+# operator, and of all operators on a basis together
+PACKED_BYTES, PACKED_TOTAL = 64 << 20, 1 << 30
 
 
 def packed_limit(op):
@@ -46,6 +47,12 @@ def packed_limit(op):
     if not len(b._pers) or 4 * op.oplist.n_off * b.Ns <= PACKED_BYTES:
         return PACKED_BYTES
     return max(PACKED_BYTES, b.lookup_table_bytes())
+
+
+def packed_total(basis):
+    """Bytes the packed rows of all operators on a basis may take together:
+    what its sector table, of which there is one, would take, or 1 GiB."""
+    return max(PACKED_TOTAL, basis.lookup_table_bytes())
 
 
 def _cache_path():

@@ -334,3 +334,50 @@ def test_packed_norm_estimates_share_the_adjoint(monkeypatch):
     E.set_a(-35.0j)
     expm_multiply_parallel(Q, a=-30.0j)
     assert 1 <= len(calls) <= 2
+
+
+def test_packed_rows_of_one_basis_share_a_limit(monkeypatch):
+    """Operators beyond the basis' limit take the other forms; freed rows make room."""
+    import gc
+    from quspin_amd import _lib as L, tuning
+    from quspin_amd.operators import quantum_LinearOperator
+    basis, static, _ = _case("momentum")
+    x = _vec(np.random.default_rng(9), basis.Ns, 1, np.complex128)
+
+    def made(scale):
+        op = quantum_LinearOperator([[o, [[scale * b[0]] + b[1:] for b in bb]] for o, bb in static], basis=basis,
+                                    dtype=np.complex128, **KW)._qsx_operator()
+        y = L.empty(x.shape, np.complex128)
+        op.apply(L.to_device(x), y)
+        _check(L.to_host(y), op.to_csr().to_scipy(), x, 1.0, None, np.complex128)
+        return op
+    first = made(1.0)
+    one = 4 * int(first._pk[1].numel())
+    monkeypatch.setattr(tuning, "packed_total", lambda b: 2 * one)
+    second, third = made(2.0), made(3.0)
+    assert second._pk is not None and third._pk is None
+    del first
+    gc.collect()
+    assert made(4.0)._pk is not None
+
+
+def test_packed_rows_without_memory(monkeypatch):
+    """No memory for the build: the product takes another form."""
+    import torch
+    from quspin_amd import _lib as L
+    from quspin_amd.operators import quantum_LinearOperator
+    basis, static, _ = _case("momentum")
+    op = quantum_LinearOperator(static, basis=basis, dtype=np.complex128, **KW)._qsx_operator()
+    x = _vec(np.random.default_rng(10), basis.Ns, 1, np.complex128)
+    y = L.empty(x.shape, np.complex128)
+    real = L.empty
+
+    def empty(shape, dtype):
+        if np.dtype(dtype) == np.int64:
+            raise torch.OutOfMemoryError("no memory")
+        return real(shape, dtype)
+    monkeypatch.setattr(L, "empty", empty)
+    op.apply(L.to_device(x), y)
+    monkeypatch.undo()
+    assert op._pk is None
+    _check(L.to_host(y), op.to_csr().to_scipy(), x, 1.0, None, np.complex128)
