@@ -156,10 +156,10 @@ class _PackedRows:
 
     def reserve(self, basis, nbytes):
         """Whether the rows of all operators on the basis, these with them,
-        stay within ``tuning.packed_total``; counted until these are freed."""
+        stay within ``tuning.packed_fits``; counted until these are freed."""
         budget = _rows_budget(basis)
         with _rows_lock:
-            if budget[0] + nbytes > tuning.packed_total(basis):
+            if not tuning.packed_fits(basis, budget[0] + nbytes):
                 return False
             budget[0] += nbytes
         weakref.finalize(self, _rows_release, budget, nbytes)
@@ -259,7 +259,7 @@ class MatrixFreeOp:
         """The operator's packed rows (offsets, entries, coefficients, column
         bits), evaluated once through ``ctx`` (``qsx_hv_pack_*``) and shared
         by its contexts; None when it has none, when they would take more than
-        ``tuning.packed_limit`` bytes (``packed_total`` with the others of the
+        ``tuning.packed_limit`` bytes (``packed_fits`` with the others of the
         basis) or when the device has no memory for them."""
         P = self._packed_rows
         with P.lock:

@@ -353,7 +353,7 @@ def test_packed_rows_of_one_basis_share_a_limit(monkeypatch):
         return op
     first = made(1.0)
     one = 4 * int(first._pk[1].numel())
-    monkeypatch.setattr(tuning, "packed_total", lambda b: 2 * one)
+    monkeypatch.setattr(tuning, "PACKED_TOTAL", 2 * one)
     second, third = made(2.0), made(3.0)
     assert second._pk is not None and third._pk is None
     del first
