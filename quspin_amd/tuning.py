@@ -49,10 +49,10 @@ def packed_limit(op):
     return max(PACKED_BYTES, b.lookup_table_bytes())
 
 
-def packed_total(basis):
-    """Bytes the packed rows of all operators on a basis may take together:
-    what its sector table, of which there is one, would take, or 1 GiB."""
-    return max(PACKED_TOTAL, basis.lookup_table_bytes())
+def packed_fits(basis, nbytes):
+    """Whether the packed rows of all operators on a basis may take ``nbytes``
+    together: 1 GiB, or what its sector table, of which there is one, would."""
+    return nbytes <= PACKED_TOTAL or nbytes <= basis.lookup_table_bytes()
 
 
 def _cache_path():
