@@ -167,17 +167,32 @@ def choose(op, ctx, vdt, nvec):
     if op.basis.Ns < 4096:
         return static_rule(op, vdt, nvec)
     key = signature(op, vdt, nvec)
-    if key in _mem:
-        return _mem[key]
-    disk = _load_file()
-    if key in disk:
-        _mem[key] = disk[key]
-        return disk[key]
+    known = _cached(key)
+    if known is not None and known["schedule"] != "packed":
+        return known
+    # whether there are packed rows depends on the coefficients, which the key
+    # does not hold: operators refused them have a choice of their own
+    if op._packed(ctx) is None:
+        key += "_unpacked"
+        known = _cached(key)
+    if known is not None:
+        return known
     best = time_candidates(op, ctx, vdt, nvec)
     _mem[key] = best
+    disk = _load_file()
     disk[key] = best
     _save_file(disk)
     return best
+
+
+def _cached(key):
+    """The choice kept under ``key``, in memory or in the file, or None."""
+    if key not in _mem:
+        disk = _load_file()
+        if key not in disk:
+            return None
+        _mem[key] = disk[key]
+    return _mem[key]
 
 
 def time_candidates(op, ctx, vdt, nvec, reps=5):
