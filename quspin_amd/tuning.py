@@ -244,6 +244,20 @@ def time_candidates(op, ctx, vdt, nvec, reps=5):
 BATCH_SCHEDULES = tuple((c, x) for x in (0, 1) for c in (4, 8, 16, 32))
 
 
+def _batch_work(batch, terms):
+    """What a sector batch is timed on: four Taylor terms (up to 64 vectors,
+    what the loop takes), or one product."""
+    t = L.torch()
+    x = t.ones((batch.rows, batch.nvec), dtype=L.torch_dtype(batch.vdt), device="cuda")
+    n = len(batch.ops)
+    if terms and batch.nvec <= 64:
+        work = t.empty(2 * x.numel(), dtype=x.dtype, device="cuda")
+        # a tiny step: tol 0 runs all four
+        return lambda: batch.expm_inplace(x, work, [(4, 1)] * n, [0.0] * n, [0.0] * n, 1e-6, graph=False)
+    y = t.empty_like(x)
+    return lambda: batch.apply(x, y)
+
+
 def choose_batch_schedule(batch, reps=3):
     """Chunk size and chunk order for a sector batch: timed on the batch's own
     sectors, cached like the single-operator choices.  The CSR form is timed
@@ -264,19 +278,9 @@ def choose_batch_schedule(batch, reps=3):
         _mem[key] = disk[key]
         return tuple(disk[key]["schedule"])
     t = L.torch()
-    x = t.ones((batch.rows, batch.nvec), dtype=L.torch_dtype(batch.vdt), device="cuda")
-    work = t.empty(2 * x.numel(), dtype=x.dtype, device="cuda")
+    once = _batch_work(batch, batch.form == "csr")
     st = t.cuda.current_stream()
-    terms = batch.form == "csr" and batch.nvec <= 64  # what the Taylor loop takes
-    n = len(batch.ops)
     res = []
-
-    def once():
-        if terms:
-            # four terms of a tiny step: tol 0 runs them all
-            batch.expm_inplace(x, work, [(4, 1)] * n, [0.0] * n, [0.0] * n, 1e-6, graph=False)
-        else:
-            batch.apply(x, work[:x.numel()].view_as(x))
 
     for ch, xs in BATCH_SCHEDULES:
         if batch.form == "csr" and ch > 63:
@@ -304,15 +308,16 @@ def _batch_key(ops, vdt, nvec):
 
 
 def choose_batch_form(cls, ops, vdt, nvec):
-    """'mf' or 'csr' for a sector batch: both forms are built and timed with
-    their own tuned schedules (cached; ``QSX_BATCH_FORM`` forces one)."""
+    """'mf' or 'csr' for a sector batch: both forms are built and timed on the
+    same work (Taylor terms) with their own tuned schedules (cached;
+    ``QSX_BATCH_FORM`` forces one)."""
     forced = os.environ.get("QSX_BATCH_FORM")
     if forced:
         return forced
     rows = sum(op.Ns for op in ops)
     if os.environ.get("QSX_TUNE", "on") == "off" or rows < 65536:
         return "csr" if nvec >= 8 else "mf"
-    key = _batch_key(ops, vdt, nvec) + "_form"
+    key = _batch_key(ops, vdt, nvec) + "_form_terms"
     if key in _mem:
         return _mem[key]["form"]
     disk = _load_file()
@@ -323,18 +328,17 @@ def choose_batch_form(cls, ops, vdt, nvec):
     res = []
     for form in ("mf", "csr"):
         b = cls(ops, vdt, nvec, form=form)
-        x = t.ones((b.rows, b.nvec), dtype=L.torch_dtype(b.vdt), device="cuda")
-        y = t.empty_like(x)
-        b.apply(x, y)
+        once = _batch_work(b, True)
+        once()
         st = t.cuda.current_stream()
         e0, e1 = t.cuda.Event(enable_timing=True), t.cuda.Event(enable_timing=True)
         e0.record(st)
         for _ in range(3):
-            b.apply(x, y)
+            once()
         e1.record(st)
         t.cuda.synchronize()
         res.append((round(e0.elapsed_time(e1) / 3, 5), form))
-        del b, x, y
+        del b, once
     ms, best = min(res)
     entry = {"form": best, "timings": [[f, m_] for m_, f in res]}
     _mem[key] = entry

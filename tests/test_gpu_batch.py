@@ -242,3 +242,30 @@ def test_batched_expm_with_empty_sectors(form):
         assert g.shape == (bases[k].Ns, nv)
         if bases[k].Ns:
             np.testing.assert_allclose(g, expm(-2.0j * dense[k]) @ xs[k], rtol=0, atol=1e-11)
+
+
+def test_form_is_timed_on_the_same_work(monkeypatch, tmp_path):
+    """The two forms of a sector batch are compared on Taylor terms, which the
+    schedule of the CSR form is chosen for, and a verdict kept from a
+    comparison of plain products is not taken."""
+    from quspin_amd import tuning
+    from quspin_amd.basis import spin_basis_general
+    from quspin_amd.operators import quantum_LinearOperator
+    from quspin_amd.operators._devop import SectorBatch
+    monkeypatch.setenv("QSX_TUNE_CACHE", str(tmp_path / "tune.json"))
+    ops = [quantum_LinearOperator(xxz_static(18), basis=spin_basis_general(18, Nup=9, pauli=0,
+                                                                           kblock=(chain_maps(18)["T"], k)),
+                                  dtype=np.complex64, check_symm=False, check_herm=False,
+                                  check_pcon=False)._qsx_operator() for k in range(18)] * 2
+    monkeypatch.setattr(tuning, "_mem", {tuning._batch_key(ops, np.complex64, 16) + "_form": {"form": "neither"}})
+    terms = []
+    run = SectorBatch.expm_inplace
+
+    def expm_inplace(self, *args, **kw):
+        terms.append(self.form)
+        return run(self, *args, **kw)
+    monkeypatch.setattr(SectorBatch, "expm_inplace", expm_inplace)
+    form = tuning.choose_batch_form(SectorBatch, ops, np.complex64, 16)
+    assert form in ("mf", "csr") and {"mf", "csr"} <= set(terms)
+    entry = next(e for e in tuning._mem.values() if "form" in e and e["form"] != "neither")
+    assert form == min(entry["timings"], key=lambda t: t[1])[0]
