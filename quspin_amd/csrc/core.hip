@@ -647,27 +647,35 @@ extern "C" int qsx_normalization(qsx_core* c, const void* states, void* out, int
 // rank order) the basis index of its representative and the code of the
 // group element reaching it; absent states hold all ones.
 // ---------------------------------------------------------------------------
+// Single exit on purpose in both functions: with a return per mode gfx950 code
+// was generated in which the trailing one (mode 2) never wrote its value, so
+// the table of a basis without particle conservation was filled from words
+// that were not set, which read out of range.
 template <typename I>
 __device__ __forceinline__ I sector_state(const RankDev* __restrict__ R, int64_t rk) {
-  if (R->mode == 0) return R->Np == 0 ? (I)0 : unrank_comb<I>(R, rk, R->Np, R->N);
-  if (R->mode == 1) {
+  const int mode = R->mode;
+  I s = (I)rk;
+  if (mode == 0) {
+    s = unrank_comb<I>(R, rk, R->Np, R->N);  // Np = 0: no bits
+  } else if (mode == 1) {
     const int64_t iu = rk / R->cdn, id = rk % R->cdn;
-    const I up = R->Nup == 0 ? (I)0 : unrank_comb<I>(R, iu, R->Nup, R->L);
-    const I dn = R->Ndn == 0 ? (I)0 : unrank_comb<I>(R, id, R->Ndn, R->L);
-    return (up << R->L) | dn;
+    s = (unrank_comb<I>(R, iu, R->Nup, R->L) << R->L) | unrank_comb<I>(R, id, R->Ndn, R->L);
   }
-  return (I)rk;
+  return s;
 }
 
 template <typename I>
 __device__ __forceinline__ I sector_next(const RankDev* __restrict__ R, I s, int64_t rk_next) {
-  if (R->mode == 0) return R->Np == 0 ? s : gosper_next<I>(s);
-  if (R->mode == 1) {
-    if (rk_next % R->cdn == 0) return sector_state<I>(R, rk_next);
+  const int mode = R->mode;
+  I t = s + 1;
+  if (mode == 0) {
+    t = R->Np == 0 ? s : gosper_next<I>(s);
+  } else if (mode == 1) {
     const I mlo = (((I)1) << R->L) - 1;
-    return (s & ~mlo) | gosper_next<I>(s & mlo);
+    if (rk_next % R->cdn == 0) t = sector_state<I>(R, rk_next);
+    else t = (s & ~mlo) | gosper_next<I>(s & mlo);
   }
-  return s + 1;
+  return t;
 }
 
 // Coefficient classes of the table: the distinct normalisations n > 0 of

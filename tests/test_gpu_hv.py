@@ -570,3 +570,47 @@ def test_spinful_without_double_occupancy_vs_oracle():
         H = _oracle_H(B, static, fermion=True, spinful_L=L)
         v = _vec(B.Ns, np.complex128, seed=6)
         np.testing.assert_allclose(Q.dot(v), H @ v, atol=1e-12, rtol=0)
+
+
+@pytest.mark.parametrize("L,blocks", [(9, {"k": 2}), (10, {"k": 0}), (8, {"k": 0, "p": 1, "z": 0}), (7, {"p": 0})])
+def test_table_without_particle_conservation(L, blocks, monkeypatch):
+    """The sector table of a basis of all 2^L words gives every word the index
+    of its representative, and the products through it are the operator's."""
+    from quspin_amd import _lib as Lb
+    from quspin_amd.basis import spin_basis_general
+    from quspin_amd.operators import quantum_LinearOperator
+    i = np.arange(L)
+    maps = {"k": (i + 1) % L, "p": i[::-1].copy(), "z": -(i + 1)}
+    B = spin_basis_general(L, pauli=0, **{q + "block": (maps[q], v) for q, v in blocks.items()})
+    tab, width, bits, _ = B.lookup_table()
+    entry = Lb.to_host(tab).view(np.uint32 if width == 4 else np.uint64)
+    assert len(entry) == 2 ** L
+    at = {int(s): n for n, s in enumerate(Lb.to_host(B._dev["basis"]).view(np.uint32))}
+
+    def image(s, q):
+        up = [(s >> (L - 1 - j)) & 1 for j in range(L)]
+        return sum((up[m] if m >= 0 else 1 - up[-(m + 1)]) << (L - 1 - j) for j, m in enumerate(maps[q]))
+    none = 0xFFFFFFFF if width == 4 else 2 ** 64 - 1
+    for s in range(2 ** L):
+        orbit, todo = {s}, [s]
+        while todo:
+            t = todo.pop()
+            new = {image(t, q) for q in blocks} - orbit
+            orbit |= new
+            todo += new
+        idx = at.get(max(orbit), -1)
+        e = int(entry[s])
+        assert (e == none) if idx < 0 else (e & ((1 << (bits if width == 4 else 40)) - 1)) == idx
+    static = [["xx", [[0.3, j, (j + 1) % L] for j in range(L)]], ["zz", [[0.7, j, (j + 1) % L] for j in range(L)]],
+              ["x", [[0.2, j] for j in range(L)]]]
+    kw = dict(basis=B, dtype=np.complex128, check_symm=False, check_herm=False, check_pcon=False)
+    A = quantum_LinearOperator(static, **kw)._qsx_operator().to_csr().to_scipy()
+    x = np.random.default_rng(L).normal(size=B.Ns) + 0j
+    monkeypatch.setenv("QSX_LOOKUP", "table")
+    for schedule in ("rows", "batch8", "packed"):
+        monkeypatch.setenv("QSX_SCHEDULE", schedule)
+        Q = quantum_LinearOperator(static, **kw)
+        y = Lb.to_host(Q.dot(Lb.to_device(x)))
+        assert Q._qsx_operator().config[(np.dtype(np.complex128), 1)]["lookup"] == "table"
+        # at most 2 L + 1 products of numbers of order one
+        assert np.abs(y - A @ x).max() <= 64 * L * 2.0 ** -53 * np.abs(x).max()
