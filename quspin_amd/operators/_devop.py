@@ -135,8 +135,8 @@ _rows_lock = threading.RLock()
 
 
 def _rows_budget(basis):
-    """[bytes of packed rows held on this basis]"""
-    return basis.__dict__.setdefault("_packed_held", [0])
+    """[bytes of packed rows held on this basis, builds]"""
+    return basis.__dict__.setdefault("_packed_held", [0, 0])
 
 
 def _rows_release(budget, nbytes):
@@ -147,12 +147,15 @@ def _rows_release(budget, nbytes):
 class _PackedRows:
     """Packed rows of one operator list and pair of flags on one basis:
     ``held`` is (offsets, entries, coefficients, column bits), or None while
-    they are not built and where there are none."""
+    they are not built and where there are none (``too_large``: for their
+    size).  ``products``: vectors that single products took so far."""
 
     def __init__(self):
         self.lock = threading.Lock()
         self.tried = False
         self.held = None
+        self.too_large = False
+        self.products = 0
 
     def reserve(self, basis, nbytes):
         """Whether the rows of all operators on the basis, these with them,
@@ -184,6 +187,7 @@ class MatrixFreeOp:
         self.transposed, self.conjugated, self.diag_conj = bool(transposed), bool(conjugated), bool(diag_conj)
         self.diag = diag
         self._ctx = {}
+        self._retired = []  # contexts replaced when the rows were built: a capture may hold their buffers
         self._rows = {} if rows is None else rows
         self._packed_rows = self._rows.setdefault((self.transposed, self.conjugated), _PackedRows())
         self.shape = (basis.Ns, basis.Ns)
@@ -234,14 +238,45 @@ class MatrixFreeOp:
             L.check(L.load().qsx_hv_ctx_set_diag(ctx.h, ptr(d), cplx), "qsx_hv_ctx_set_diag")
         return ctx
 
-    def _context(self, vdt, nvec):
+    def _context(self, vdt, nvec, products=None):
+        """The context for vectors of this dtype and number, for a loop or
+        for ``products`` single products (``_packs_now``)."""
         key = (vdt, nvec)
-        if key not in self._ctx:
+        ctx = self._ctx.get(key)
+        if ctx is not None and not ctx.later:
+            return ctx
+        now = self._packs_now(nvec, products)
+        if ctx is None or now:
+            if ctx is not None:
+                self._retired.append(ctx)
             ctx = self._new_ctx(vdt, nvec)
-            cfg = tuning.choose(self, ctx, vdt, nvec)
+            cfg = dict(tuning.choose(self, ctx, vdt, nvec, now))
+            ctx.later = cfg.pop("later", False)
             self._configure(ctx, cfg)
             self._ctx[key] = ctx
-        return self._ctx[key]
+        return ctx
+
+    def _packs_now(self, nvec, products):
+        """Whether the packed rows may be built by this call.  A build costs
+        about as much as ``tuning.PACK_AFTER`` products gain from it, so an
+        operator that is asked for single products (a scan over parameters
+        makes a few with each) has made that many before; a loop, and the
+        first operator on a symmetry-reduced basis, whose other form would
+        need the sector table built and its schedules timed, does not wait.
+        Not while the stream is captured (a build waits for the device)."""
+        P = self._packed_rows
+        if P.tried:
+            return True
+        if L.torch().cuda.is_current_stream_capturing():
+            return False
+        if products is None or (len(self.basis._pers) and not self._later_on_basis()):
+            return True
+        P.products += products * max(int(nvec), 1)
+        return P.products > tuning.PACK_AFTER
+
+    def _later_on_basis(self):
+        """Whether another operator on this basis built packed rows before."""
+        return _rows_budget(self.basis)[1] > 0
 
     def _configure(self, ctx, cfg):
         ctx.configure(cfg, self.basis, self._packed(ctx) if cfg.get("schedule") == "packed" else None)
@@ -272,10 +307,14 @@ class MatrixFreeOp:
             return P.held
 
     def _build_packed(self, ctx):
+        _rows_budget(self.basis)[1] += 1
         limit = tuning.packed_limit(self)
         lib = L.load()
         nwork = lib.qsx_hv_pack_work_bytes(ctx.h)
-        if nwork <= 0 or 4 * self.Ns > limit:
+        if nwork <= 0:
+            return None
+        if 4 * self.Ns > limit:
+            self._packed_rows.too_large = True
             return None
         off = L.empty((self.Ns + 63) // 64 + 1, np.int64)
         work = L.empty((nwork + 7) // 8, np.int64)
@@ -283,7 +322,8 @@ class MatrixFreeOp:
         rc = lib.qsx_hv_pack_count(ctx.h, ptr(off), ptr(work), nwork, C.byref(ent), C.byref(nl), C.byref(bits),
                                    stream_handle())
         if rc == L.QSX_OK:
-            if 4 * ent.value > limit or not self._packed_rows.reserve(self.basis, 4 * ent.value):
+            self._packed_rows.too_large = 4 * ent.value > limit
+            if self._packed_rows.too_large or not self._packed_rows.reserve(self.basis, 4 * ent.value):
                 return None
             entries = L.empty(max(ent.value, 1), np.int32)
             lut = L.empty(nl.value, np.complex128)
@@ -298,10 +338,10 @@ class MatrixFreeOp:
         """Chosen (lookup, schedule) per (dtype, nvec)."""
         return {k: v.cfg for k, v in self._ctx.items()}
 
-    def apply(self, x, y, a=1.0, beta=0, a_diag=None):
+    def apply(self, x, y, a=1.0, beta=0, a_diag=None, products=None):
         vdt = L.np_dtype(x.dtype)
         nvec = math.prod(x.shape[1:])
-        ctx = self._context(vdt, nvec)
+        ctx = self._context(vdt, nvec, products)
         ac = complex(a)
         ad = ac if a_diag is None else complex(a_diag)
         rc = L.load().qsx_hv_ctx_apply(ctx.h, ptr(x), ptr(y), ac.real, ac.imag, ad.real, ad.imag,
@@ -312,7 +352,7 @@ class MatrixFreeOp:
         """Diagonal of the operator as a device vector."""
         ones = L.torch().ones(self.Ns, dtype=L.torch_dtype(dtype), device="cuda")
         out = L.zeros(self.Ns, dtype)
-        self.apply(ones, out, a=0.0, a_diag=1.0)
+        self.apply(ones, out, a=0.0, a_diag=1.0, products=1)
         return out
 
     def _column_norms(self, shift):
@@ -499,6 +539,7 @@ class SectorBatch:
 class _Ctx:
     def __init__(self, h):
         self.h = h
+        self.later = False  # to be replaced once the packed rows are built
         self.cfg = {"lookup": "search", "schedule": "rows"}
 
     def configure(self, cfg, basis, packed=None):

@@ -171,7 +171,7 @@ class quantum_LinearOperator(LinearOperator):
                 L.np_dtype(other.dtype) == self._dtype:
             # the common case: a device vector of the operator's own dtype
             y = L.empty(tuple(other.shape), self._dtype)
-            self._qsx_operator().apply(other, y, a=a, beta=beta, a_diag=a_diag)
+            self._qsx_operator().apply(other, y, a=a, beta=beta, a_diag=a_diag, products=1)
             return y
         on_dev = L.is_device_tensor(other)
         odt = L.np_dtype(other.dtype) if on_dev else np.asanyarray(other).dtype
@@ -184,7 +184,7 @@ class quantum_LinearOperator(LinearOperator):
         else:
             y = L.to_device(out, result_dtype)
         op = self._qsx_operator()
-        op.apply(x, y, a=a, beta=beta, a_diag=a_diag)
+        op.apply(x, y, a=a, beta=beta, a_diag=a_diag, products=1)
         if on_dev or L.is_device_tensor(out):
             return y
         res = L.to_host(y)

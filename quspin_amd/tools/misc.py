@@ -24,7 +24,8 @@ def _matvec(array, other, overwrite_out=False, out=None, a=1.0):
     else:
         y = out if L.is_device_tensor(out) else L.to_device(out, result_dtype)
         beta = 0 if overwrite_out else 1
-    op.apply(x, y, a=a, beta=beta)
+    single = {"products": 1} if op.is_matrix_free else {}
+    op.apply(x, y, a=a, beta=beta, **single)
     if on_dev or L.is_device_tensor(out):
         return y
     res = L.to_host(y)

@@ -13,8 +13,9 @@ half-chain terms per block, then upper-half and crossing terms over column
 strips; "chunk4/8": direct-rank rows with the terms in chunks and predicated
 gathers; all but "rows" for one vector only; "packed": the elements evaluated
 once, four bytes each, and streamed, for one vector or several).  A
-symmetry-reduced operator takes its packed rows where they are no larger than
-its sector table would be (``packed_limit``); the others' candidates are timed on the operator's own
+symmetry-reduced operator, and one on fewer than 4,096 states, takes its packed
+rows where they are no larger than its sector table would be
+(``packed_limit``); the others' candidates are timed on the operator's own
 basis with HIP events (a few launches each) and the winner is cached per
 (basis signature, dtype, nvec) in memory and in a JSON file
 (``QSX_TUNE_CACHE``, default ``~/.cache/quspin_amd/tune.json``).
@@ -38,6 +39,13 @@ SCHEDULES = {"rows": 0, "queue": 1, "rows2": 2, "rows4": 3, "rows8": 4, "batch4"
 # packed rows of sectors without symmetry maps, and of small sectors: of one
 # operator, and of all operators on a basis together
 PACKED_BYTES, PACKED_TOTAL = 64 << 20, 1 << 30
+# Vectors an operator multiplies one product at a time before its packed rows
+# are built, about what a build costs: 924 states 95 us against 6 us gained per
+# product, 63,504 Hubbard states 250 against 15, Heisenberg L = 28 through the
+# sector table 600 against 14.  Without the wait the first product of each
+# further operator on a basis took 250 us in place of 155, 430 in place of 180,
+# and (built by orbit search) 4,950 in place of 1,580.
+PACK_AFTER = 16
 
 
 def packed_limit(op):
@@ -60,10 +68,19 @@ def _cache_path():
                                                          "tune.json"))
 
 
+_file = (None, {})  # (path, time and size) of the file read last, and its contents
+
+
 def _load_file():
+    global _file
+    path = _cache_path()
     try:
-        with open(_cache_path()) as f:
-            return json.load(f)
+        st = os.stat(path)
+        seen = (path, st.st_mtime_ns, st.st_size)
+        if _file[0] != seen:
+            with open(path) as f:
+                _file = (seen, json.load(f))
+        return dict(_file[1])
     except Exception:
         return {}
 
@@ -146,7 +163,10 @@ def _rank_lookup(op):
         (not len(b._pers) and getattr(b, "_spinful", False) and b._Np is not None and len(b._Np) == 1)
 
 
-def choose(op, ctx, vdt, nvec):
+def choose(op, ctx, vdt, nvec, now=True):
+    """Lookup and schedule of an operator.  ``now`` False: packed rows that are
+    not there yet are not built; the best other choice known without timing
+    anything for them is given, marked "later"."""
     forced_l, forced_s = os.environ.get("QSX_LOOKUP"), os.environ.get("QSX_SCHEDULE")
     if forced_l or forced_s:
         cfg = static_rule(op, vdt, nvec)
@@ -157,22 +177,40 @@ def choose(op, ctx, vdt, nvec):
         return cfg
     if os.environ.get("QSX_TUNE", "on") == "off":
         return static_rule(op, vdt, nvec)
-    if len(op.basis._pers) or op.basis.Ns < 4096:
-        # through the sector table where the basis holds it already
-        lookup = "table" if op.basis.has_lookup_table() else "search"
-        if lookup == "table":
+    tuned = op.basis.Ns >= 4096
+    if len(op.basis._pers) or not tuned:
+        if not now:
+            cfg = None
+            if tuned:
+                key = signature(op, vdt, nvec)
+                cfg = _cached(key) or _cached(key + "_unpacked")
+            cfg = dict(cfg or static_rule(op, vdt, nvec), later=True)
+            if cfg["lookup"] != "table" or _make_table(op.basis):
+                return cfg
+        # through the sector table where the basis holds it, or has to: a
+        # second operator's build by orbit search takes longer than the table's
+        lookup = "search"
+        if op.basis.has_lookup_table() or (op._later_on_basis() and not op._packed_rows.tried and _make_table(op.basis)):
+            lookup = "table"
             ctx.configure({"lookup": lookup, "schedule": "rows"}, op.basis)
         if op._packed(ctx) is not None:
             return {"lookup": lookup, "schedule": "packed"}
-    if op.basis.Ns < 4096:
+    if not tuned:
         return static_rule(op, vdt, nvec)
     key = signature(op, vdt, nvec)
     known = _cached(key)
     if known is not None and known["schedule"] != "packed":
         return known
+    if not now:
+        others = [t for t in (known or {}).get("timings", ()) if t[1] != "packed"]
+        if others:
+            lookup, schedule, _ = min(others, key=lambda t: t[2])
+            return {"lookup": lookup, "schedule": schedule, "later": True}
+        if known is None and _cached(key + "_unpacked") is not None:
+            return dict(_cached(key + "_unpacked"), later=True)
     # whether there are packed rows depends on the coefficients, which the key
-    # does not hold: operators refused them have a choice of their own
-    if op._packed(ctx) is None:
+    # does not hold: operators refused them for that have a choice of their own
+    if op._packed(ctx) is None and not op._packed_rows.too_large:
         key += "_unpacked"
         known = _cached(key)
     if known is not None:
@@ -183,6 +221,14 @@ def choose(op, ctx, vdt, nvec):
     disk[key] = best
     _save_file(disk)
     return best
+
+
+def _make_table(basis):
+    """Whether the basis has its sector table, built where it can be."""
+    try:
+        return basis.lookup_table() is not None
+    except L.torch().OutOfMemoryError:
+        return False
 
 
 def _cached(key):

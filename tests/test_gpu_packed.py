@@ -210,8 +210,9 @@ def test_packed_limit_and_replaced_diagonal(monkeypatch):
     _check(L.to_host(Q2.dot(xd)), A, x, 3.0, 3 * before, np.float64)
     monkeypatch.setattr(tuning, "packed_limit", lambda op: 4 * op.Ns)
     Q3 = quantum_LinearOperator(static, basis=basis, dtype=np.float64, **KW)
-    _check(L.to_host(Q3.dot(xd)), A, x, 1.0, before, np.float64)
-    assert Q3._qsx_operator()._pk is None
+    for _ in range(tuning.PACK_AFTER + 2):
+        _check(L.to_host(Q3.dot(xd)), A, x, 1.0, before, np.float64)
+    assert Q3._qsx_operator()._packed_rows.tried and Q3._qsx_operator()._pk is None
 
 
 @pytest.mark.parametrize("nv", [1, 4, 9])
@@ -381,3 +382,60 @@ def test_packed_rows_without_memory(monkeypatch):
     monkeypatch.undo()
     assert op._pk is None
     _check(L.to_host(y), op.to_csr().to_scipy(), x, 1.0, None, np.complex128)
+
+
+@pytest.mark.parametrize("nv", [1, 5])
+@pytest.mark.parametrize("name", ["free", "momentum"])
+def test_rows_are_built_after_single_products(name, nv, monkeypatch):
+    """An operator asked for one product at a time makes ``PACK_AFTER`` vectors
+    without packed rows (the first one on a symmetry-reduced basis builds them
+    at once, the others go through the sector table); every product is the
+    operator's, before and after."""
+    from quspin_amd import _lib as L, tuning
+    from quspin_amd.operators import quantum_LinearOperator
+    basis, static, _ = _case(name)
+    calls = _count_builds(monkeypatch)
+    x = _vec(np.random.default_rng(nv), basis.Ns, nv, np.complex128)
+    xd = L.to_device(x)
+    for i in range(3):
+        Q = quantum_LinearOperator([[o, [[(1 + i) * b[0]] + b[1:] for b in bb]] for o, bb in static], basis=basis,
+                                   dtype=np.complex128, **KW)
+        A = Q._qsx_operator().to_csr().to_scipy()
+        calls.clear()
+        first = name == "momentum" and i == 0
+        for k in range(20):
+            _check(L.to_host(Q.dot(xd)), A, x, 1.0, None, np.complex128)
+            assert len(calls) == (1 if first or (k + 1) * nv > tuning.PACK_AFTER else 0)
+        assert Q._qsx_operator().config[(np.dtype(np.complex128), nv)]["schedule"] == "packed"
+    assert basis.has_lookup_table() == (name == "momentum")
+
+
+def test_a_captured_product_builds_nothing(monkeypatch):
+    """Products of one operator, one of them captured: the capture holds the
+    form without rows and replays its product after the rows are built."""
+    import torch
+    from quspin_amd import _lib as L, tuning
+    from quspin_amd.operators import quantum_LinearOperator
+    basis, static, _ = _case("free")
+    calls = _count_builds(monkeypatch)
+    Q = quantum_LinearOperator(static, basis=basis, dtype=np.float64, **KW)
+    A = Q._qsx_operator().to_csr().to_scipy()
+    x = _vec(np.random.default_rng(3), basis.Ns, 1, np.float64)
+    xd = L.to_device(x)
+    y = torch.empty_like(xd)
+    op = Q._qsx_operator()
+    for _ in range(3):
+        op.apply(xd, y, products=1)
+    monkeypatch.setattr(tuning, "PACK_AFTER", 2)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        op.apply(xd, y, products=1)
+    assert not calls and op._pk is None
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        _check(L.to_host(y), A, x, 1.0, None, np.float64)
+        y.zero_()
+        op.apply(xd, y, products=1)
+        _check(L.to_host(y), A, x, 1.0, None, np.float64)
+    assert len(calls) == 1 and op._pk is not None

@@ -22,6 +22,7 @@ class Op:
         self.builds = 0
         self.basis = types.SimpleNamespace(N=20, Ns=5000, _pers=[], _qs=[], _Np=None)
         self.oplist = types.SimpleNamespace(n_off=20, n_diag=0)
+        self._packed_rows = types.SimpleNamespace(too_large=False)
 
     def _packed(self, ctx):
         self.builds += 1
@@ -65,3 +66,36 @@ def test_no_rows_are_built_where_another_form_won(timed, monkeypatch):
     tuning.choose(Op(True), None, F64, 1)
     op = Op(True)
     assert tuning.choose(op, None, F64, 1)["schedule"] == "split2" and op.builds == 0
+
+
+def test_an_operator_too_large_for_rows_is_not_tried_again(timed):
+    """A refusal for the size holds for every operator of the shape: the choice
+    is kept under the common key and the next operator builds nothing."""
+    op = Op(False)
+    op._packed_rows.too_large = True
+    assert tuning.choose(op, None, F64, 1)["schedule"] == "split2"
+    op = Op(False)
+    assert tuning.choose(op, None, F64, 1)["schedule"] == "split2" and op.builds == 0
+
+
+def test_rows_not_built_yet_take_the_best_other_choice(timed, monkeypatch):
+    """``now`` False: the fastest form besides packed rows, marked to be
+    replaced, and nothing is built or timed; with ``now`` the rows."""
+    timings = [["search", "packed", 1.0], ["search", "rows", 3.0], ["search", "split2", 2.0]]
+    monkeypatch.setattr(tuning, "time_candidates", lambda op, ctx, vdt, nvec, reps=5: {
+        "lookup": "search", "schedule": "packed", "timings": timings})
+    tuning.choose(Op(True), None, F64, 1)
+    op = Op(True)
+    assert tuning.choose(op, None, F64, 1, now=False) == {"lookup": "search", "schedule": "split2", "later": True}
+    assert op.builds == 0
+    assert tuning.choose(op, None, F64, 1)["schedule"] == "packed" and op.builds == 1
+
+
+def test_small_sector_waits_with_the_static_rule(timed):
+    op = Op(True)
+    op.Ns = op.basis.Ns = 900
+    op.basis.has_lookup_table = lambda: False
+    op._later_on_basis = lambda: False
+    cfg = tuning.choose(op, None, F64, 1, now=False)
+    assert cfg == dict(tuning.static_rule(op, F64, 1), later=True) and op.builds == 0
+    assert tuning.choose(op, None, F64, 1)["schedule"] == "packed"
