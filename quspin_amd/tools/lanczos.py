@@ -4,9 +4,11 @@ _expm.py:7-52) with the recurrence on the device.
 For operators the library can run (``hamiltonian``, ``quantum_LinearOperator``,
 scipy matrices, device CSR) each step is one H.v launch plus two fused
 update kernels (r -= b v, a = Re<q,r>; r -= a q, b = ||r||) with FP64
-accumulation (small operators run the whole recurrence in one launch); a and b stay in device memory until the loop ends, and the
-tridiagonal problem is solved in FP64 with ``scipy.linalg.eigh_tridiagonal``
-as in the reference.  Other operators go through their own ``dot``.
+accumulation (small operators run the whole recurrence in one launch, packed
+rows take two per step); a and b stay in device memory until the loop ends, and
+the tridiagonal problem is solved in FP64 with
+``scipy.linalg.eigh_tridiagonal`` as in the reference.  Other operators go
+through their own ``dot``.
 """
 
 import numpy as np
@@ -19,6 +21,10 @@ from ._ftlm import FTLM_static_iteration, LTLM_static_iteration  # noqa: F401
 
 __all__ = ["lanczos_full", "lanczos_iter", "lin_comb_Q_T", "expm_lanczos", "FTLM_static_iteration",
            "LTLM_static_iteration"]
+
+
+# rows above which qsx_lanczos_small refuses every operator
+_SMALL_ROWS = 4096
 
 
 def _dtype_of(A, v0):
@@ -42,18 +48,18 @@ def _device_loop(op, v0, m, dtype, eps, store_Q, Q_out=None):
     st = stream_handle()
     kind = _run_kind(op, dtype)
     q0 = L.to_device(v0, dtype).reshape(n)
-    if kind is not None:
-        # a small operator: normalisation and recurrence in one launch
+    small = kind is not None and n <= _SMALL_ROWS
+    packed = kind is not None and kind[0] is not None and kind[0].cfg["schedule"] == "packed"
+    if small or packed:
+        # (a basis of vectors only where one of the two forms fills it)
         direct = Q_out is not None and Q_out.is_contiguous()
         Q = (Q_out if direct else L.empty((m, n), dtype)) if store_Q else None
         ab = L.zeros((m, 2, 2), np.float64)
-        rc = lib.qsx_lanczos_small(*_run_args(*kind, dtype), code, n, m, ptr(q0), float(eps), ptr(Q), ptr(ab), st)
-        if rc != L.QSX_ERR_UNSUPPORTED:
-            L.check(rc, "qsx_lanczos_small")
-            if Q_out is not None and not direct:
-                Q = Q_out.copy_(Q)
-            return _finish(ab, m, eps, Q)
-        if kind[0] is not None and kind[0].cfg["schedule"] == "packed":
+        rc = L.QSX_ERR_UNSUPPORTED
+        if small:
+            # normalisation and recurrence in one launch
+            rc = lib.qsx_lanczos_small(*_run_args(*kind, dtype), code, n, m, ptr(q0), float(eps), ptr(Q), ptr(ab), st)
+        if rc == L.QSX_ERR_UNSUPPORTED and packed:
             # packed rows: normalisation on the device, two launches per step, vectors straight into Q
             Qb = Q if store_Q else L.empty((min(m, 3), n), dtype)
             if direct:
@@ -62,7 +68,8 @@ def _device_loop(op, v0, m, dtype, eps, store_Q, Q_out=None):
             work = L.empty(int(lib.qsx_lanczos_packed_work()), np.float64)
             rc = lib.qsx_lanczos_packed(kind[0].h, code, n, m, ptr(q0), float(eps), ptr(Qb), int(bool(store_Q)),
                                         ptr(r), ptr(ab), ptr(work), st)
-            L.check(rc, "qsx_lanczos_packed")
+        if rc != L.QSX_ERR_UNSUPPORTED:
+            L.check(rc, "qsx_lanczos_small / _packed")
             if Q_out is not None and not direct:
                 Q = Q_out.copy_(Q)
             return _finish(ab, m, eps, Q)

@@ -208,3 +208,22 @@ def test_packed_lanczos_two_launches_per_step(dtype, blocks, Nup, L_, monkeypatc
         E3, _, K3 = lanczos_full(Q, out[0], m, out=out)
         assert np.array_equal(E, E3) and np.array_equal(L.to_host(K3), L.to_host(K))
     assert L.QSX_OK not in codes
+
+
+def test_lanczos_memory_of_the_captured_sequence():
+    """An operator with neither form holds the result and the workspace's
+    vectors, not a third basis."""
+    import torch
+    from quspin_amd import _lib as L
+    from quspin_amd.operators._devop import DeviceCSR
+    from quspin_amd.tools.lanczos import lanczos_full
+    n, m = 200_000, 40
+    d = sp.diags([np.linspace(-1, 1, n), np.full(n - 1, 0.5), np.full(n - 1, 0.5)], [0, 1, -1]).tocsr()
+    A = DeviceCSR.from_scipy(d, np.float64)
+    x = L.to_device(_vec(np.random.default_rng(0), n, np.float64))
+    torch.cuda.empty_cache()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    lanczos_full(A, x, m)
+    # two bases of m vectors and a few vectors
+    assert torch.cuda.max_memory_allocated() - before <= (2 * m + 8) * n * 8
