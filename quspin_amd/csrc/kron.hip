@@ -655,16 +655,16 @@ int qsx_evolve_steps_with(int64_t Ns, int64_t nvec, const double* xdiag, int nst
                           int64_t ctl_bytes, int64_t part_blocks,
                           int (*term)(const CsrArgs&, const void*, int, int, hipStream_t), const void* term_ctx,
                           const StepOpKey& key, int use_graph, hipStream_t st);
-int qsx_part_reduce_launch(const CsrArgs& A, int64_t nblocks, hipStream_t st);
-bool qsx_norms_direct(int64_t nblocks);
 
+// The norms go straight into the slots (no partials buffer): the blocks of this
+// form are few, or end apart.  Eight driven Hubbard steps, partials and direct:
+// L = 10 (252 blocks) 1.34 / 1.09 ms in complex64, L = 12 (924) 4.34 / 3.91, L =
+// 13 (2,916) 7.89 / 7.55, L = 14 (11,610) 22.8 / 22.5; complex128 1.75 / 1.46,
+// 6.62 / 6.24, 14.05 / 13.68, 47.2 / 46.9.
 static int kron_term(const CsrArgs& A, const void* ctx, int vdt, int fdt, hipStream_t st) {
-  const qsx_kron* K = (const qsx_kron*)ctx;
   CsrArgs B = A;
-  if (qsx_norms_direct(kron_blocks(K, vt_size(vdt)))) B.part = nullptr;
-  const int rc = launch_kron<true>(B, K, vdt, fdt, st);
-  if (rc) return rc;
-  return qsx_part_reduce_launch(B, kron_blocks(K, vt_size(vdt)), st);
+  B.part = nullptr;
+  return launch_kron<true>(B, (const qsx_kron*)ctx, vdt, fdt, st);
 }
 
 extern "C" int qsx_evolve_kron_steps(const qsx_kron* K, const double* xdiag, int nsteps, const void* es, int s_max,

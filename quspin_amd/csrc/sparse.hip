@@ -44,19 +44,19 @@ __global__ void __launch_bounds__(256) k_part_reduce(const double* __restrict__ 
   }
 }
 
-// Whether an expm launch of nblocks blocks puts its norms straight into the
+// Whether a CSR expm launch of nblocks blocks puts its norms straight into the
 // slots (one atomic per block and norm) instead of a partials buffer that a
-// second launch reduces.  Small grids save the launch (XXZ L = 12 step, 4
-// blocks per term: 795 -> 601 us); grids of many rounds spread their atomics
-// over the launch (driven Hubbard L = 14, 11,610 blocks: 59.3 -> 58.3 ms).
-// In between the blocks end together and their atomics queue up behind one
-// address (12 vectors at L = 18, 1,520 blocks: 1.92 -> 2.08 ms), so those keep
-// partials.
-bool qsx_norms_direct(int64_t nblocks) { return nblocks <= 256 || nblocks >= 8192; }
+// second launch reduces.  Few blocks save the launch; from about 600 blocks on
+// the atomics that queue up behind one address cost more than it.  Per Taylor
+// term, partials and direct: XXZ, complex128 vectors, 402 blocks 18.6 / 16.6
+// us, 760 blocks 15.3 / 16.9 (4 vectors) and 19.4 / 20.3 (12), 2,887 blocks
+// 22.6 / 26.9, 11,023 blocks 54.9 / 111.3; eight driven Hubbard steps, complex64,
+// 497 blocks 1.26 / 1.15 ms, 1,668 blocks 1.87 / 2.29, 23,006 blocks 19.7 / 21.7.
+static bool norms_direct(int64_t nblocks) { return nblocks <= 512; }
 
 // Fold the per-block norm partials of one expm launch (nblocks blocks) into
-// its norm slots; used by every expm term kernel.
-int qsx_part_reduce_launch(const CsrArgs& A, int64_t nblocks, hipStream_t st) {
+// its norm slots (nothing to do without partials).
+static int part_reduce_launch(const CsrArgs& A, int64_t nblocks, hipStream_t st) {
   if (!A.part) return QSX_OK;
   hipLaunchKernelGGL(k_part_reduce, dim3(64), dim3(256), 0, st, A.part, nblocks, &A.ctl->done, A.normB, A.normF,
                      A.nsp);
@@ -121,7 +121,7 @@ template <typename MT, typename VT, int CW, bool EPI>
 static int64_t launch_mm_g(CsrArgs& A, hipStream_t st) {
   const int G = mm_group(A.nvec / CW);
   const int64_t nb = mm_blocks(A.Ns, G);
-  if (qsx_norms_direct(nb)) A.part = nullptr;
+  if (norms_direct(nb)) A.part = nullptr;
   const dim3 grid((unsigned)nb), blk(256);
   switch (G) {
     case 2: hipLaunchKernelGGL((k_csr_mm<MT, VT, 2, mm_rpg(2), CW, EPI>), grid, blk, 0, st, A); break;
@@ -168,11 +168,11 @@ static int launch_csr(CsrArgs A, int mdt, int vdt, int G, hipStream_t st, int fd
   int64_t blocks = launch_mm<EPI>(A, mdt, vdt, fdt, st);
   if (blocks > 0) {
     QSX_LAUNCH_CHECK();
-    if constexpr (EPI) return qsx_part_reduce_launch(A, blocks, st);
+    if constexpr (EPI) return part_reduce_launch(A, blocks, st);
     return QSX_OK;
   }
   blocks = csr_blocks(A.Ns, G, EPI);
-  if (qsx_norms_direct(blocks)) A.part = nullptr;
+  if (norms_direct(blocks)) A.part = nullptr;
   // matrix dtype must be the vector dtype or its real counterpart
   if (fdt == vdt) {
     if (vdt == QSX_F32 && mdt == QSX_F32) launch_csr_g<float, float, EPI>(A, G, st);
@@ -192,7 +192,7 @@ static int launch_csr(CsrArgs A, int mdt, int vdt, int G, hipStream_t st, int fd
     return QSX_ERR_ARG;
   }
   QSX_LAUNCH_CHECK();
-  if constexpr (EPI) return qsx_part_reduce_launch(A, blocks, st);
+  if constexpr (EPI) return part_reduce_launch(A, blocks, st);
   return QSX_OK;
 }
 

@@ -192,7 +192,7 @@ __device__ __forceinline__ void spmv_out(const CsrArgs& A, int64_t o, int64_t ro
 
 // Block max of the per-thread row-sum maxima: into part[blockIdx] (two
 // doubles; k_part_reduce folds a launch's partials into the slots), or
-// straight into the slots when there is no partials buffer (small grids).
+// straight into the slots when there is no partials buffer.
 __device__ __forceinline__ void block_norm_partials(const CsrArgs& A, double mb, double mf) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {

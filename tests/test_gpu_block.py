@@ -161,3 +161,24 @@ def test_sector_batch_csr_rows_side_by_side(nv, dtype):
         assert np.abs(F[at:at + op.Ns] - one.reshape(F[at:at + op.Ns].shape)).max() <= \
             100 * EPS[np.dtype(dtype)] * np.abs(xs).max() * 4
         at += op.Ns
+
+
+@pytest.mark.parametrize("nv", [1, 2])
+@pytest.mark.parametrize("blocks", [512, 513, 8192])
+def test_expm_norms_by_grid(blocks, nv):
+    """Taylor loops either side of the number of blocks up to which the norms
+    go straight into their slots, and on a large grid: the truncation that the
+    norms decide gives the exponential of a tridiagonal matrix.  Error: one
+    rounding per term of partial sums of at most e^|a A|, |a A| <= 2."""
+    from scipy.sparse.linalg import expm_multiply
+    from quspin_amd import _lib as L
+    from quspin_amd.operators._devop import DeviceCSR
+    from quspin_amd.tools.evolution import expm_multiply_parallel
+    n = 128 * blocks  # two lanes per row
+    rng = np.random.default_rng(blocks)
+    A = sp.diags([rng.uniform(-1, 1, n), np.full(n - 1, 0.5), np.full(n - 1, 0.5)], [0, 1, -1]).tocsr()
+    E = expm_multiply_parallel(DeviceCSR.from_scipy(A, np.float64), a=-1.0j)
+    x = rng.normal(size=(n,) if nv == 1 else (n, nv)) + 0j
+    got = L.to_host(E.dot(L.to_device(x)))
+    exact = expm_multiply(-1.0j * A, x, traceA=-1.0j * A.diagonal().sum())
+    assert np.abs(got - exact).max() <= 40 * 2.0 ** -53 * np.exp(2.0) * np.abs(x).max()
