@@ -6,6 +6,7 @@
 // and ``_wrapper_expm_multiply[_batch]`` (EMP.html:347-372), whose loop is
 // Al-Mohy & Higham Alg. 3.2 as in scipy ``_expm_multiply_simple_core``
 // (scipy/sparse/linalg/_expm_multiply.py:280-303).
+#include <algorithm>
 #include <cstring>
 #include <atomic>
 #include <map>
@@ -117,9 +118,30 @@ static int64_t mm_blocks(int64_t Ns, int G) {
   return nb < 1 ? 1 : nb > EPI_MAX_BLOCKS ? EPI_MAX_BLOCKS : nb;
 }
 
+// Whether k_csr_mm is the faster form, by estimates in microseconds fitted to
+// both forms over 300 to 250,000 rows of 2 to 256 entries and 2 to 64 vectors
+// of every dtype (1,768 points: within 1 % of the faster one on average), with
+// a floor per tile for float32, whose vectors k_csr_spmv reads cheapest (600,000
+// rows of 3, 5 vectors: 53 us against 34).
+// k_csr_mm walks a row with the few lanes that its vectors fill, and where the
+// rows of a block do not fit one round of staged entries most of its lanes
+// wait for the round that holds theirs; k_csr_spmv has lanes across the row
+// and passes over it once per vector.  Few vectors on long rows go to the
+// latter: 1,000 rows of 200 entries, 2 float64 vectors 391 against 16 us; 30,000
+// rows of 60, 67 against 26 (5 vectors: 25 against 56).
+static bool mm_wins(const CsrArgs& A, int64_t nnz, int G, int CW, size_t esz) {
+  const double nv = (double)A.nvec, k = (double)nnz / (double)A.Ns;
+  const double passes = (double)((A.nvec + G * CW - 1) / (G * CW)) * mm_rpg(G);
+  const double rounds = std::max(1.0, 256.0 / G * k / CSR_MM_CAP);
+  double mm = 1.5 + 0.085 * k * rounds * passes;
+  if (esz == 4) mm = std::max(mm, 2.9e-3 * (double)A.Ns * G / 256.0);
+  return mm <= 0.7 * nv + 3e-6 * (double)nnz * nv;
+}
+
 template <typename MT, typename VT, int CW, bool EPI>
-static int64_t launch_mm_g(CsrArgs& A, hipStream_t st) {
+static int64_t launch_mm_g(CsrArgs& A, int64_t nnz, hipStream_t st) {
   const int G = mm_group(A.nvec / CW);
+  if (!mm_wins(A, nnz, G, CW, sizeof(VT))) return 0;
   const int64_t nb = mm_blocks(A.Ns, G);
   if (norms_direct(nb)) A.part = nullptr;
   const dim3 grid((unsigned)nb), blk(256);
@@ -139,33 +161,34 @@ static int64_t launch_mm_g(CsrArgs& A, hipStream_t st) {
 // the lanes and gathers (XXZ L = 22, 16 float64 vectors 165 -> 122 us, 8
 // vectors 89 -> 67 us; 2 vectors 43 -> 46 us).
 template <typename MT, typename VT, bool EPI>
-static int64_t launch_mm_w(CsrArgs& A, hipStream_t st) {
+static int64_t launch_mm_w(CsrArgs& A, int64_t nnz, hipStream_t st) {
   if constexpr (sizeof(VT) == 8) {
-    if (A.nvec % 2 == 0 && (uintptr_t)A.x % 16 == 0) return launch_mm_g<MT, VT, 2, EPI>(A, st);
+    if (A.nvec % 2 == 0 && (uintptr_t)A.x % 16 == 0) return launch_mm_g<MT, VT, 2, EPI>(A, nnz, st);
   }
-  return launch_mm_g<MT, VT, 1, EPI>(A, st);
+  return launch_mm_g<MT, VT, 1, EPI>(A, nnz, st);
 }
 
-// Several vectors go to k_csr_mm (one dtype for terms and accumulator, columns
-// below 2^31); 0: the caller takes k_csr_spmv, else the blocks launched.
+// Several vectors go to k_csr_mm where it wins (one dtype for terms and
+// accumulator, columns below 2^31); 0: the caller takes k_csr_spmv, else the
+// blocks launched.
 template <bool EPI>
-static int64_t launch_mm(CsrArgs& A, int mdt, int vdt, int fdt, hipStream_t st) {
+static int64_t launch_mm(CsrArgs& A, int64_t nnz, int mdt, int vdt, int fdt, hipStream_t st) {
   if (A.nvec < 2 || fdt != vdt || A.Ns >= INT32_MAX) return 0;
-  if (vdt == QSX_F32 && mdt == QSX_F32) return launch_mm_w<float, float, EPI>(A, st);
-  if (vdt == QSX_F64 && mdt == QSX_F64) return launch_mm_w<double, double, EPI>(A, st);
-  if (vdt == QSX_C64 && mdt == QSX_F32) return launch_mm_w<float, float2, EPI>(A, st);
-  if (vdt == QSX_C64 && mdt == QSX_C64) return launch_mm_w<float2, float2, EPI>(A, st);
-  if (vdt == QSX_C128 && mdt == QSX_F64) return launch_mm_w<double, double2, EPI>(A, st);
-  if (vdt == QSX_C128 && mdt == QSX_C128) return launch_mm_w<double2, double2, EPI>(A, st);
+  if (vdt == QSX_F32 && mdt == QSX_F32) return launch_mm_w<float, float, EPI>(A, nnz, st);
+  if (vdt == QSX_F64 && mdt == QSX_F64) return launch_mm_w<double, double, EPI>(A, nnz, st);
+  if (vdt == QSX_C64 && mdt == QSX_F32) return launch_mm_w<float, float2, EPI>(A, nnz, st);
+  if (vdt == QSX_C64 && mdt == QSX_C64) return launch_mm_w<float2, float2, EPI>(A, nnz, st);
+  if (vdt == QSX_C128 && mdt == QSX_F64) return launch_mm_w<double, double2, EPI>(A, nnz, st);
+  if (vdt == QSX_C128 && mdt == QSX_C128) return launch_mm_w<double2, double2, EPI>(A, nnz, st);
   return 0;
 }
 
 // fdt: dtype of the expm accumulator F (-1: the vector dtype); FP64 F with
 // FP32 vectors is the mixed-precision form.
 template <bool EPI>
-static int launch_csr(CsrArgs A, int mdt, int vdt, int G, hipStream_t st, int fdt = -1) {
+static int launch_csr(CsrArgs A, int64_t nnz, int mdt, int vdt, int G, hipStream_t st, int fdt = -1) {
   if (fdt < 0) fdt = vdt;
-  int64_t blocks = launch_mm<EPI>(A, mdt, vdt, fdt, st);
+  int64_t blocks = launch_mm<EPI>(A, nnz, mdt, vdt, fdt, st);
   if (blocks > 0) {
     QSX_LAUNCH_CHECK();
     if constexpr (EPI) return part_reduce_launch(A, blocks, st);
@@ -220,7 +243,7 @@ extern "C" int qsx_csr_matvec(const void* indptr, const void* indices, const voi
   A.indptr = indptr; A.indices = indices; A.data = data; A.idx64 = idx64; A.Ns = Ns; A.nvec = nvec;
   A.x = x; A.y = y; A.a = make_double2(a_re, a_im); A.mu = make_double2(0, 0); A.beta = accumulate ? 1 : 0;
   const int G = group > 0 ? group : auto_group(Ns, nnz);
-  return launch_csr<false>(A, mat_dtype, vec_dtype, G, (hipStream_t)stream);
+  return launch_csr<false>(A, nnz, mat_dtype, vec_dtype, G, (hipStream_t)stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -1039,7 +1062,7 @@ static int expm_csr_loop(const void* indptr, const void* indices, const void* da
         A.chk_c2 = normB + i * stride + j * nsp;
         A.chk_F = normF + i * stride + j * nsp;
       }
-      const int rc = launch_csr<true>(A, mat_dtype, vec_dtype, G, st);
+      const int rc = launch_csr<true>(A, nnz, mat_dtype, vec_dtype, G, st);
       if (rc) return rc;
     }
     double* nb0 = (i + 1 < s) ? normB + (i + 1) * stride : nullptr;
@@ -1561,7 +1584,7 @@ int csr_term(const CsrArgs& A0, const void* ctx, int vdt, int fdt, hipStream_t q
   A.indices = c->indices;
   A.data = c->data;
   A.idx64 = c->idx64;
-  return launch_csr<true>(A, c->mat_dtype, vdt, c->G, q, fdt);
+  return launch_csr<true>(A, c->nnz, c->mat_dtype, vdt, c->G, q, fdt);
 }
 }  // namespace
 

@@ -285,8 +285,8 @@ __global__ void __launch_bounds__(256) k_csr_spmv(CsrArgs A) {
 // broadcasts; a lane keeps U gathers in flight.  FP64 accumulation.
 //
 // Bound by the gathers: every entry reads one vector row (nvec elements)
-// through L2, and by their latency where nvec is small.  k_csr_spmv, which
-// several vectors used before, walks the whole row once per vector, each lane
+// through L2, and by their latency where nvec is small.  k_csr_spmv, which few
+// vectors on long rows still use, walks the whole row once per vector, each lane
 // of a gather on a line of its own and the matrix re-read per vector: a Taylor
 // term of 12 complex128 vectors on the XXZ L = 18 matrix (48,620 rows) takes
 // 80 us there and 15 us here.

@@ -62,6 +62,27 @@ def test_csr_block_product(mdt, vdt, n, nv):
     assert np.all(np.abs(L.to_host(yd) - exact - y0) <= bound)
 
 
+@pytest.mark.parametrize("vdt", [np.float32, np.float64, np.complex64, np.complex128])
+@pytest.mark.parametrize("n,k,nv", [(30011, 10, 2), (30011, 10, 3), (60000, 24, 2), (1000, 200, 2), (1000, 200, 8),
+                                    (1000, 200, 64), (30000, 60, 3), (30000, 60, 5)])
+def test_csr_block_product_either_side_of_the_rule(vdt, n, k, nv):
+    """Few vectors on short rows of a large matrix (a block's entries in one
+    staged round and in three), and few and many vectors on long rows."""
+    from quspin_amd import _lib as L
+    from quspin_amd.operators._devop import DeviceCSR
+    rng = np.random.default_rng(n + nv)
+    mdt = np.float32 if vdt in (np.float32, np.complex64) else np.float64
+    r = np.repeat(np.arange(n), k)
+    A = sp.csr_matrix((rng.normal(size=n * k).astype(mdt), (r, rng.integers(0, n, n * k))), shape=(n, n))
+    D = DeviceCSR.from_scipy(A, mdt)
+    A = D.to_scipy()  # duplicates summed
+    x = _vectors(rng, n, nv, vdt)
+    y = L.empty((n, nv), vdt)
+    D.apply(L.to_device(x), y)
+    exact = A.astype(np.float64) @ x.astype(np.complex128)
+    assert np.all(np.abs(L.to_host(y) - exact) <= _bound(A, x, vdt))
+
+
 def test_csr_block_long_rows_and_unaligned_vectors():
     """Rows longer than one staged round, and vectors off the 16-byte boundary."""
     from quspin_amd import _lib as L
