@@ -375,7 +375,8 @@ int qsx_lanczos_packed(const void* hv_ctx, int dtype, int64_t n, int m, const vo
  * v0 (divided by its norm when that is off 1 by more than eps): a_i and b_i
  * into ab as there, q_0 .. q_{m-1} into Q (m, n) unless Q is NULL.
  * QSX_ERR_UNSUPPORTED, nothing launched: an assembled matrix of more than
- * 2,048 rows or 24,576 entries, a context of more than 4,096 rows or 49,152
+ * 2,048 rows or 24,576 entries or with rows so long that launches per step are
+ * faster, a context of more than 4,096 rows or 49,152
  * packed elements (above 2,048 rows: 32,768 real, 20,480 complex) or not bound
  * to packed rows, or more LDS than the device has for a workgroup. */
 int qsx_lanczos_small(int op_kind, const void* hv_ctx, const void* indptr, const void* indices, const void* data,

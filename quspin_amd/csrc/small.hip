@@ -7,6 +7,7 @@
 // rows whose other vectors stay in its registers, and the norms and dots are
 // block reductions: two or three barriers per term or step instead of two to
 // four launches.  Same recurrences, roundings and truncation test as there.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -17,7 +18,8 @@ namespace {
 
 constexpr int SMALL_T = 1024;  // threads
 // Sizes up to which one workgroup wins over a launch per term or two per step;
-// a row beyond a thread's second leaves too few registers for its elements.
+// a row beyond a thread's second leaves too few registers for its elements
+// (assembled matrices: small_csr besides).
 // Measured on sectors without symmetries, t = 1 steps (about 65 terms) and 30
 // Lanczos steps, launches -> one workgroup:
 //   assembled     924 rows 593 -> 215 us, 1,716 rows 607 -> 424, 3,432 rows 617 -> 985
@@ -407,6 +409,23 @@ bool launch_small_packed(const SmallArgs& A, int vdt, hipStream_t st) {
 
 bool small_size(int64_t n, int64_t entries) { return n >= 1 && n <= SMALL_N && entries <= SMALL_NNZ; }
 
+// Whether one workgroup wins on an assembled matrix: a term's time here, in
+// microseconds, is that of n rows plus what the entries beyond a thread's
+// registers cost, which are read from memory on every term (fitted to 744 loops
+// over 20 to 2,000 rows of 2 to 200 entries, random and banded, of every
+// dtype).  A launch per term takes 6 to 8 us there, a Lanczos step of launches
+// 13 to 18 (here 3 more than a term).  200 rows of 100 entries 16.8 us here and
+// 7.7 there, 500 of 48 15.7 and 7.2, 500 of 16 2.4 and 7.4.
+bool small_csr(int64_t n, int64_t nnz, int mat_dtype, bool lanczos) {
+  if (!small_size(n, nnz)) return false;
+  const double k = (double)nnz / (double)n;
+  if (n <= SMALL_T) {
+    const double us = 1.0 + 2e-3 * n + (0.08 + 6e-4 * n) * std::max(0.0, k - (mat_dtype == QSX_C128 ? 8 : 16));
+    return us <= (lanczos ? 11.5 : 6.5);
+  }
+  return k <= 12.5 && 1.8e-3 * n + 4e-4 * n * std::max(0.0, k - 4.0) <= (lanczos ? 11.5 : 7.4);
+}
+
 SmallArgs csr_args(const void* indptr, const void* indices, const void* data, int idx64, int64_t n) {
   SmallArgs A;
   std::memset(&A, 0, sizeof(A));
@@ -444,7 +463,7 @@ void taylor_args(SmallArgs& A, const SmallTaylor& T) {
 
 bool qsx_small_expm_csr(const void* indptr, const void* indices, const void* data, int idx64, int mat_dtype, int64_t n,
                         int64_t nnz, int vec_dtype, int64_t nvec, const SmallTaylor& T, hipStream_t st) {
-  if (nvec != 1 || !small_size(n, nnz)) return false;
+  if (nvec != 1 || !small_csr(n, nnz, mat_dtype, false)) return false;
   SmallArgs A = csr_args(indptr, indices, data, idx64, n);
   taylor_args(A, T);
   return launch_small_csr<false>(A, mat_dtype, vec_dtype, st);
@@ -475,7 +494,7 @@ extern "C" int qsx_lanczos_small(int op_kind, const void* hv_ctx, const void* in
   bool ok = false;
   if (op_kind == 0) {
     ok = ctx_args(hv_ctx, true, A, dt) && dt == dtype && A.n == n;
-  } else if (small_size(n, nnz)) {
+  } else if (small_csr(n, nnz, mat_dtype, true)) {
     A = csr_args(indptr, indices, data, idx64, n);
     ok = true;
   }

@@ -227,3 +227,34 @@ def test_lanczos_memory_of_the_captured_sequence():
     lanczos_full(A, x, m)
     # two bases of m vectors and a few vectors
     assert torch.cuda.max_memory_allocated() - before <= (2 * m + 8) * n * 8
+
+
+@pytest.mark.parametrize("n,k,small", [(200, 100, False), (500, 48, False), (500, 14, True), (64, 32, True),
+                                       (1900, 20, False)])
+@pytest.mark.parametrize("dtype", [np.float64, np.complex64])
+def test_small_csr_by_row_length(n, k, small, dtype, monkeypatch):
+    """Assembled matrices with long rows keep a launch per term and step; both
+    sides of the rule give the exponential and the recurrence."""
+    from scipy.sparse.linalg import expm_multiply
+    from quspin_amd import _lib as L
+    from quspin_amd.operators._devop import DeviceCSR
+    from quspin_amd.tools.evolution import expm_multiply_parallel
+    from quspin_amd.tools.lanczos import _host_loop, lanczos_full
+    rng = np.random.default_rng(n)
+    offs = np.unique(np.concatenate([[0], rng.permutation(n - 1)[:k // 2] + 1]))
+    A = sum((sp.diags([np.full(n - d, 0.5 / k)], [d], shape=(n, n)) for d in offs), sp.csr_matrix((n, n)))
+    # circulant bands: every row has about k entries
+    A = (A + sum((sp.diags([np.full(d, 0.5 / k)], [d - n], shape=(n, n)) for d in offs if d), sp.csr_matrix((n, n))))
+    A = (A + A.T).tocsr().astype(np.float32 if dtype == np.complex64 else np.float64)
+    D = DeviceCSR.from_scipy(A)
+    x = _vec(rng, n, dtype)
+    codes, m = _small_codes(monkeypatch), 10
+    E, V, K = lanczos_full(D, L.to_device(x), m)
+    assert codes == [L.QSX_OK if small else L.QSX_ERR_UNSUPPORTED]
+    a, b, _, Kh = _host_loop(A.astype(np.complex128), x.astype(np.complex128), m, np.complex128, 0.0)
+    Eh = np.linalg.eigvalsh(np.diag(a) + np.diag(b[:-1], 1) + np.diag(b[:-1], -1))
+    assert np.abs(E - Eh).max() <= 400 * EPS[np.dtype(dtype)] * max(1.0, np.abs(Eh).max()) * m
+    got = L.to_host(expm_multiply_parallel(D, a=-1.0, dtype=dtype).dot(L.to_device(x)))
+    exact = expm_multiply(-A.astype(np.float64), x.astype(np.complex128))
+    # |A| <= 1.1: partial sums of at most e^1.1, one rounding per term
+    assert np.abs(got - exact).max() <= 40 * EPS[np.dtype(dtype)] * np.exp(1.1) * np.abs(x).max()
