@@ -26,6 +26,7 @@ struct qsx_hv_batch {
   std::vector<int64_t> row_off_h;
   HvArgs* sec_d = nullptr;
   CsrSec* csr_d = nullptr;    // CSR form
+  bool long_rows = false;     // few rows of more than WAVE_LONG entries on average
   int64_t* row_off_d = nullptr;
   WaveChunk* chunk_d = nullptr;
   int64_t nchunk = 0;
@@ -169,7 +170,18 @@ extern "C" int qsx_csr_batch_create(int nsec, const int64_t* Ns, const void* con
     b->row_off_h[k + 1] = b->row_off_h[k] + Ns[k];
   }
   b->total = b->row_off_h[nsec];
-  hipError_t e = hipMalloc((void**)&b->csr_d, sizeof(CsrSec) * nsec);
+  int64_t entries = 0;  // the last offset of every sector
+  hipError_t e = hipSuccess;
+  for (int k = 0; k < nsec && e == hipSuccess; ++k) {
+    if (Ns[k] == 0) continue;
+    int64_t n64 = 0;
+    int32_t n32 = 0;
+    if (sec[k].idx64) e = hipMemcpy(&n64, (const int64_t*)indptr[k] + Ns[k], sizeof(n64), hipMemcpyDeviceToHost);
+    else e = hipMemcpy(&n32, (const int32_t*)indptr[k] + Ns[k], sizeof(n32), hipMemcpyDeviceToHost);
+    entries += n64 + n32;
+  }
+  b->long_rows = entries > WAVE_LONG * b->total && b->total < WAVE_FEW;
+  if (e == hipSuccess) e = hipMalloc((void**)&b->csr_d, sizeof(CsrSec) * nsec);
   if (e == hipSuccess) e = hipMemcpy(b->csr_d, sec.data(), sizeof(CsrSec) * nsec, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMalloc((void**)&b->row_off_d, sizeof(int64_t) * (nsec + 1));
   if (e == hipSuccess)
@@ -231,6 +243,7 @@ static BatchArgs base_args(const qsx_hv_batch* b) {
   B.row_off = b->row_off_d;
   B.chunk = b->chunk_d;
   B.nchunk = b->nchunk;
+  B.long_rows = b->long_rows;
   B.ld = b->nvec;
   B.xdiag = nullptr;
   B.xdscale = make_double2(0.0, 0.0);

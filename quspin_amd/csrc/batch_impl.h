@@ -58,6 +58,7 @@ struct BatchArgs {
   double* nF;
   int64_t nslot;            // s_max * (m_max + 1)
   int mstride;              // m_max + 1
+  int long_rows;            // CSR form: few rows of more than WAVE_LONG entries on average (host: choice of kernel)
 };
 
 __device__ __forceinline__ int lane_id() { return (int)(threadIdx.x & 63); }
@@ -432,6 +433,9 @@ __global__ void __launch_bounds__(256) k_csr_wave(BatchArgs B) {
 // at a time, read lane-parallel and, for the next pass, requested before this
 // pass' gathers are used; each lane keeps U gathers in flight.
 constexpr int WAVE_CAP = 128;  // entries staged per wavefront
+// launch_csr_wave takes rows as long from WAVE_LONG entries on, where there are
+// fewer than WAVE_FEW of them (more fill the chip either way)
+constexpr int WAVE_LONG = 40, WAVE_FEW = 40960;
 
 template <typename VT, int G, int CW, bool EPI>
 __global__ void __launch_bounds__(256) k_csr_wave_g(BatchArgs B) {
@@ -589,16 +593,24 @@ void launch_csr_wave_w(const BatchArgs& B, dim3 grid, hipStream_t st) {
 // in the wavefront: up to 32 columns, or up to 64 with two 8-byte elements per
 // lane (an even number of columns on 16-byte boundaries).  All 20 momentum
 // sectors of the L = 20 Heisenberg chain, complex64 H.V: 32 columns 153 -> 57
-// us, 64 columns 139 -> 100 us; L = 22, 64 columns 549 -> 462 us.
+// us, 64 columns 139 -> 100 us; L = 22, 64 columns 549 -> 462 us.  Long rows
+// leave lanes without entries in a round of WAVE_CAP, which few rows do not
+// hide: one element per lane then (twice the gathers in flight), and complex128
+// above 16 columns keeps a row per wavefront.  Sectors of L = 16 with six neighbours (51 entries per row),
+// complex64, two elements / one / a row per wavefront: 16 columns 69 / 57 / 80
+// us, 32 columns 86 / 66 / 82, 64 columns 110 / - / 84; complex128 24 columns
+// - / 98 / 86.  With more rows other waves hide it: L = 20 with four
+// neighbours, complex64 48 columns 332 / - / 410 us, complex128 24 columns - /
+// 366 / 444.
 template <typename VT, bool EPI>
 void launch_csr_wave(const BatchArgs& B, dim3 grid, hipStream_t st) {
   if constexpr (sizeof(VT) == 8) {
-    if (B.ncol % 2 == 0 && B.ld % 2 == 0 && B.col0 % 2 == 0 && ((uintptr_t)B.x | (uintptr_t)B.y | (uintptr_t)B.F) % 16 == 0) {
+    if (!B.long_rows && B.ncol % 2 == 0 && B.ld % 2 == 0 && B.col0 % 2 == 0 && ((uintptr_t)B.x | (uintptr_t)B.y | (uintptr_t)B.F) % 16 == 0) {
       launch_csr_wave_w<VT, 2, EPI>(B, grid, st);
       return;
     }
   }
-  if (B.ncol <= 32) { launch_csr_wave_w<VT, 1, EPI>(B, grid, st); return; }
+  if (B.ncol <= (B.long_rows && sizeof(VT) == 16 ? 16 : 32)) { launch_csr_wave_w<VT, 1, EPI>(B, grid, st); return; }
   hipLaunchKernelGGL((k_csr_wave<VT, EPI>), grid, dim3(256), 0, st, B);
 }
 

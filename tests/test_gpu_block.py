@@ -130,6 +130,45 @@ def test_expm_block_equals_single_columns(nv, dtype):
     assert np.abs(got - exact).max() <= tol * np.abs(X).max() * 4
 
 
+@pytest.mark.parametrize("nv", [1, 2, 8, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
+def test_sector_batch_long_rows(nv, dtype):
+    """Few rows of more than 40 entries (53 on average): the forms that the
+    choice by row length takes, products and a Taylor loop."""
+    from models import chain_maps
+    from quspin_amd import _lib as L
+    from quspin_amd.basis import spin_basis_general
+    from quspin_amd.operators import quantum_LinearOperator
+    from quspin_amd.operators._devop import SectorBatch
+    from quspin_amd.tools.evolution import expm_multiply_sectors
+    size = 14
+    bonds = [[0.5 / d, i, (i + d) % size] for d in range(1, 8) for i in range(size)]
+    static = [["+-", bonds], ["-+", bonds], ["zz", bonds]]
+    kw = dict(check_symm=False, check_herm=False, check_pcon=False)
+    ops = [quantum_LinearOperator(static, basis=spin_basis_general(size, Nup=7, pauli=0,
+                                                                   kblock=(chain_maps(size)["T"], k)), dtype=dtype,
+                                  **kw) for k in (0, 5)]
+    mf = [op._qsx_operator() for op in ops]
+    mats = [op.to_csr(dtype).to_scipy() for op in mf]
+    assert sum(A.nnz for A in mats) > 40 * sum(A.shape[0] for A in mats)
+    rng = np.random.default_rng(nv)
+    x = [_vectors(rng, op.Ns, nv, dtype) for op in ops]
+    batch = SectorBatch(mf, dtype, nv, form="csr", chunk_rows=16)
+    Y = batch.empty()
+    batch.apply(batch.stack(x), Y)
+    for y, A, xs in zip(batch.unstack(Y), mats, x):
+        exact = A.astype(np.complex128) @ xs.astype(np.complex128)
+        assert np.all(np.abs(L.to_host(y) - exact) <= _bound(A, xs, dtype))
+    from scipy.sparse.linalg import expm_multiply
+    E = expm_multiply_sectors(ops, a=-0.2j, dtype=dtype, nvec=nv, form="csr", chunk_rows=16)
+    at = 0
+    F = L.to_host(E.dot(x))
+    for A, xs in zip(mats, x):
+        exact = expm_multiply(-0.2j * A.astype(np.complex128), xs.astype(np.complex128))
+        assert np.abs(F[at:at + len(xs)] - exact).max() <= 100 * EPS[np.dtype(dtype)] * np.abs(xs).max() * 4
+        at += len(xs)
+
+
 @pytest.mark.parametrize("nv", [1, 2, 3, 8, 9, 16, 17, 31, 32, 33, 34, 63, 64, 70])
 @pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
 def test_sector_batch_csr_rows_side_by_side(nv, dtype):
