@@ -568,9 +568,10 @@ class _Ctx:
                 L.check(lib.qsx_hv_ctx_set_packed(self.h, ptr(off), ptr(ent), int(ent.numel()), ptr(lut),
                                                   int(lut.numel()), bits), "qsx_hv_ctx_set_packed")
         rc = lib.qsx_hv_ctx_set_schedule(self.h, code)
-        if rc == L.QSX_ERR_UNSUPPORTED and code == tuning.SCHEDULES["split"]:
+        if rc == L.QSX_ERR_UNSUPPORTED and code in (tuning.SCHEDULES["split"], tuning.SCHEDULES["split2"]):
             # the split-chain layout needs one hcb sector without symmetry
-            # maps and bit-parallel terms: other operators keep one lane per row
+            # maps and bit-parallel terms (its two-pass form at most 64 that
+            # cross the halves): other operators keep one lane per row
             self.cfg["schedule"] = "rows"
             rc = lib.qsx_hv_ctx_set_schedule(self.h, 0)
         L.check(rc, "qsx_hv_ctx_set_schedule")

@@ -103,3 +103,24 @@ def test_split_schedule_expm_and_lanczos(dt, sched, monkeypatch):
     E, _, _ = lanczos_full(Q, torch.from_numpy(v).cuda(), 80)
     E = np.asarray(E.cpu() if hasattr(E, "cpu") else E)
     assert abs(E[0] - np.linalg.eigvalsh(A)[0]) < tol_e
+
+
+def test_operators_without_the_two_pass_form_are_tuned(monkeypatch, tmp_path):
+    """More than 64 terms cross the halves: the tuner passes the form over and
+    the product is the operator's."""
+    from quspin_amd import _lib as L, tuning
+    from quspin_amd.basis import spin_basis_general
+    from quspin_amd.operators import quantum_LinearOperator
+    monkeypatch.setenv("QSX_TUNE_CACHE", str(tmp_path / "tune.json"))
+    monkeypatch.setattr(tuning, "_mem", {})
+    size = 18
+    bonds = [[0.5 / d, i, (i + d) % size] for d in range(1, 10) for i in range(size)]
+    basis = spin_basis_general(size, Nup=6, pauli=0)
+    Q = quantum_LinearOperator([["+-", bonds], ["-+", bonds], ["zz", bonds]], basis=basis, dtype=np.float64,
+                               check_symm=False, check_herm=False, check_pcon=False)
+    x = np.random.default_rng(0).normal(size=basis.Ns)
+    y = L.to_host(Q.dot(L.to_device(x)))
+    assert "split2" not in [t[1] for e in tuning._mem.values() for t in e["timings"]]
+    A = Q._qsx_operator().to_csr().to_scipy().real
+    # 2 x 160 products per row, the largest coefficient 1/2
+    assert np.abs(y - A @ x).max() <= 1024 * 2.0 ** -53 * (abs(A) @ np.abs(x)).max()
