@@ -144,6 +144,28 @@ def test_small_lanczos_packed_rows_per_thread(dtype, L_, Nup, monkeypatch):
     assert np.abs(E - Eh).max() <= 200 * EPS[np.dtype(dtype)] * np.abs(Eh).max() * m
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.complex64, np.complex128])
+def test_small_expm_packed_two_rows_per_thread(dtype):
+    """The Taylor loop in one workgroup on packed rows, 1,716 of them."""
+    from scipy.sparse.linalg import expm_multiply
+    from quspin_amd import _lib as L
+    from quspin_amd.basis import spin_basis_general
+    from quspin_amd.operators import quantum_LinearOperator
+    from quspin_amd.tools.evolution import expm_multiply_parallel
+    basis = spin_basis_general(13, Nup=6, pauli=0)
+    Q = quantum_LinearOperator(xxz_static(13, h=np.linspace(-1, 1, 13)), basis=basis, dtype=dtype, **KW)
+    A = Q._qsx_operator().to_csr(np.complex128).to_scipy()
+    x = _vec(np.random.default_rng(13), basis.Ns, dtype)
+    a = -0.4j if np.dtype(dtype).kind == "c" else -0.4
+    E = expm_multiply_parallel(Q, a=a, dtype=dtype)
+    got = L.to_host(E.dot(L.to_device(x)))
+    assert Q._qsx_operator().config[(np.dtype(dtype), 1)]["schedule"] == "packed"
+    exact = expm_multiply(a * A, x.astype(np.complex128))
+    # one rounding per term of partial sums of at most e^|a A|, |a A| <= 0.4 x 11
+    terms = E.partition[0] * E.partition[1]
+    assert np.linalg.norm(got - exact) <= (terms + 2) * EPS[np.dtype(dtype)] * np.exp(4.4)
+
+
 @pytest.mark.parametrize("dtype,small", [(np.float64, True), (np.float32, True), (np.complex128, False),
                                          (np.complex64, False)])
 def test_small_lanczos_limit_by_type(dtype, small, monkeypatch):
