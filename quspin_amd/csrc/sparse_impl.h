@@ -215,7 +215,10 @@ __device__ __forceinline__ void block_norm_partials(const CsrArgs& A, double mb,
   }
 }
 
-// Block max of the row norms of a matrix-free Taylor term into its slots.
+// Block max of the row norms of a matrix-free Taylor term into its slots, one
+// address per norm: the blocks' atomics queue up behind it (packed rows,
+// Heisenberg L = 28, complex128, 1,412 blocks: 29.4 us per term, 20.5 with plain
+// stores in their place; 126 blocks 7.6 and 7.2).
 __device__ __forceinline__ void epi_norms_out(const HvArgs& A, double mb, double mf) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
