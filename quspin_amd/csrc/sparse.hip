@@ -47,13 +47,14 @@ __global__ void __launch_bounds__(256) k_part_reduce(const double* __restrict__ 
 
 // Whether a CSR expm launch of nblocks blocks puts its norms straight into the
 // slots (one atomic per block and norm) instead of a partials buffer that a
-// second launch reduces.  Few blocks save the launch; from about 600 blocks on
+// second launch reduces.  Few blocks save the launch; from about 500 blocks on
 // the atomics that queue up behind one address cost more than it.  Per Taylor
-// term, partials and direct: XXZ, complex128 vectors, 402 blocks 18.6 / 16.6
-// us, 760 blocks 15.3 / 16.9 (4 vectors) and 19.4 / 20.3 (12), 2,887 blocks
-// 22.6 / 26.9, 11,023 blocks 54.9 / 111.3; eight driven Hubbard steps, complex64,
-// 497 blocks 1.26 / 1.15 ms, 1,668 blocks 1.87 / 2.29, 23,006 blocks 19.7 / 21.7.
-static bool norms_direct(int64_t nblocks) { return nblocks <= 512; }
+// term, partials and direct: XXZ, complex128 vectors, 380 blocks 12.6 / 11.1 us,
+// 402 blocks 18.6 / 16.6, 760 blocks 15.3 / 16.9 (4 vectors) and 19.4 / 20.3
+// (12), 2,887 blocks 22.6 / 26.9, 11,023 blocks 54.9 / 111.3; 16,000 rows of 32
+// entries, 500 blocks 12.2 / 12.9; eight driven Hubbard steps, complex64, 497
+// blocks 1.26 / 1.15 ms, 1,668 blocks 1.87 / 2.29, 23,006 blocks 19.7 / 21.7.
+static bool norms_direct(int64_t nblocks) { return nblocks <= 448; }
 
 // Fold the per-block norm partials of one expm launch (nblocks blocks) into
 // its norm slots (nothing to do without partials).
@@ -120,7 +121,7 @@ static int64_t mm_blocks(int64_t Ns, int G) {
 
 // Whether k_csr_mm is the faster form, by estimates in microseconds fitted to
 // both forms over 300 to 250,000 rows of 2 to 256 entries and 2 to 64 vectors
-// of every dtype (1,768 points: within 1 % of the faster one on average), with
+// of every dtype (1,768 points: within 1.5 % of the faster one on average), with
 // a floor per tile for float32, whose vectors k_csr_spmv reads cheapest (600,000
 // rows of 3, 5 vectors: 53 us against 34).
 // k_csr_mm walks a row with the few lanes that its vectors fill, and where the
@@ -135,7 +136,7 @@ static bool mm_wins(const CsrArgs& A, int64_t nnz, int G, int CW, size_t esz) {
   const double rounds = std::max(1.0, 256.0 / G * k / CSR_MM_CAP);
   double mm = 1.5 + 0.085 * k * rounds * passes;
   if (esz == 4) mm = std::max(mm, 2.9e-3 * (double)A.Ns * G / 256.0);
-  return mm <= 0.7 * nv + 3e-6 * (double)nnz * nv;
+  return mm <= 0.7 * nv + 2.6e-6 * (double)nnz * nv;
 }
 
 template <typename MT, typename VT, int CW, bool EPI>

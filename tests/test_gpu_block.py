@@ -224,7 +224,7 @@ def test_sector_batch_csr_rows_side_by_side(nv, dtype):
 
 
 @pytest.mark.parametrize("nv", [1, 2])
-@pytest.mark.parametrize("blocks", [512, 513, 8192])
+@pytest.mark.parametrize("blocks", [448, 449, 8192])
 def test_expm_norms_by_grid(blocks, nv):
     """Taylor loops either side of the number of blocks up to which the norms
     go straight into their slots, and on a large grid: the truncation that the
